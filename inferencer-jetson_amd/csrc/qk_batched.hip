@@ -28,17 +28,18 @@
 //   pack_activations  once per (block, 8 tokens): x -> the record of
 //                     MFMA A operands (fp16 hi / lo, sub-block sums, scales)
 //                     in the caller's workspace.
-//   batch_gemm        a workgroup (4 waves) owns 128 or 256 weight rows (one
-//                     or two 32-row tiles per wave, as many as its token
-//                     tiles) x one or two token tiles x a run of blocks.  Per block it copies the token tiles' records
-//                     into LDS with direct global->LDS loads (double-buffered:
-//                     the next block's records and weight bytes load while
-//                     this block computes); each wave decodes the raw bytes of
-//                     its rows into MFMA B operands in registers (lane l: row
-//                     l%32, block half l/32), and every decoded operand feeds
-//                     every token tile.  When one row group's blocks are split
-//                     over several workgroups (to put enough waves on the
-//                     chip), each writes its partial sums to the workspace;
+//   batch_gemm        (one token tile) and tile_gemm (two and more): a
+//                     workgroup (4 waves) owns 128 weight rows x one or two
+//                     token tiles x a run of blocks.  It copies the token
+//                     tiles' records into LDS with direct global->LDS loads
+//                     (double-buffered: the next ones and the next weight
+//                     bytes load while these compute); each wave decodes the
+//                     raw bytes of its rows into MFMA B operands in registers
+//                     (lane l: row l%32, block half l/32), and every decoded
+//                     operand feeds every token tile.  When one row group's
+//                     blocks are split over several workgroups (to put enough
+//                     waves on the chip), each writes its partial sums to the
+//                     workspace;
 //   reduce_splits     adds them in split order, so results are deterministic,
 //                     and applies the call's epilogue (one thread per output).
 #include "qk_internal.h"
@@ -53,16 +54,10 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 
 constexpr int kMfmaMinTokens = 8;
-// 32-row tiles per wave (RT): one for a single 32-token tile, two from two
-// token tiles on, so a workgroup (4 waves) owns 128 * RT weight rows and
-// writes 4 * RT * 1024 partial sums per token tile when blocks are split.
-// Measured: one row tile at 32 tokens (two workgroups per CU share each
-// SIMD's VALU and MFMA pipes) took the 32-sequence 1B step 2.15 -> 1.94 ms;
-// at 256 tokens two row tiles stay faster (4.60 against 4.74-4.78 ms).
-__host__ __device__ constexpr int group_rows(int rt) { return 128 * rt; }
-__host__ __device__ constexpr int partial_floats(int rt) { return 4 * rt * 16 * 64; }
+constexpr int kGroupRows = 128;         // weight rows of a workgroup (a 32-row tile per wave)
+constexpr int kPartialFloats = 4096;    // partial sums of one (row group, token tile): [wave][k][lane]
 constexpr int kMaxSplit = 16;           // workgroups splitting one row group's blocks
-static_assert(partial_floats(1) % 256 == 0, "reduce_splits covers whole partial slots with 256-thread workgroups");
+static_assert(kPartialFloats % 256 == 0, "reduce_splits covers whole partial slots with 256-thread workgroups");
 
 // K order of the A / B operands inside a block.  Step s (0..15) and half kh
 // (lane / 32) hold eight columns of the 64-column group G = 2*kh + s/8:
@@ -78,7 +73,7 @@ struct BatchMatrix {
     int type;
     int row_bytes;
     int ldy;
-    int group_begin;   // first row group (group_rows(RT) rows) of this matrix in the launch
+    int group_begin;   // first row group (kGroupRows rows) of this matrix in the launch
 };
 
 struct BatchParams {
@@ -91,7 +86,7 @@ struct BatchParams {
     int tiles;
     int splits;             // workgroups sharing one row group's blocks
     int blocks_per_split;
-    float *partials;        // [group][tile][split][partial_floats(RT)] when splits > 1
+    float *partials;        // [group][tile][split][kPartialFloats] when splits > 1
     const uint8_t *records; // packed activations, [tile][block][kTileBytes]
     // Decode-driver fusions (zero: plain x, overwrite y):
     const float *norm_w;    // stage RMSNorm(x) * norm_w
@@ -454,14 +449,16 @@ __device__ __forceinline__ void store_out(const BatchParams &p, float *y, float 
     *y = v;
 }
 
-// ---------------------------------------------------------------- GEMM --
+#include "qk_tile_gemm.h"
+
+// ------------------------------------------------ GEMM of one token tile --
 //
-// Workgroup = 4 waves x RT row tiles = 128 RT weight rows, x TT token
-// tiles of 32 tokens, x a run of blocks.  Per block the workgroup copies the
-// TT activation records into LDS with direct global->LDS loads (no register
-// round trip), double-buffered: block b+1's records and weight bytes are in
-// flight while block b computes.  Wave w owns rows (i*4 + w)*32 .. +31 of
-// the group for row tile i.
+// Workgroup = 4 waves = 128 weight rows x one 32-token tile x a run of
+// blocks.  Per block the workgroup copies the activation record into LDS with
+// direct global->LDS loads (no register round trip), double-buffered: block
+// b+1's record and weight bytes are in flight while block b computes.  Wave w
+// owns rows w*32 .. +31 of the group.  Two or more token tiles run
+// csrc/qk_tile_gemm.h.
 
 constexpr int kChunks = kTileBytes / 16;       // 16-byte chunks per record
 static_assert(kChunks > 8 * 256 && kChunks <= 9 * 256, "record copy layout");
@@ -483,17 +480,15 @@ __device__ __forceinline__ void record_dma(const uint8_t *rec, uint8_t *tile_lds
 
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-template <int TYPE, int TT>
+template <int TYPE>
 __global__ __launch_bounds__(256) void batch_gemm(BatchParams p) {
     extern __shared__ __align__(16) unsigned char lds[];
-    constexpr int RT = TT;
-    constexpr int kGroupRows = group_rows(RT);
-    constexpr int kPartialFloats = partial_floats(RT);
+    constexpr int RT = 1, TT = 1;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = lane >> 5, col = lane & 31;
     const int split = blockIdx.x % p.splits, group = blockIdx.x / p.splits;
-    const int tile0 = blockIdx.y * TT;
+    const int tile0 = 0;
 
     int m = 0;
     #pragma unroll
@@ -614,15 +609,12 @@ __device__ __forceinline__ float input_norm_scale(const BatchParams &p, int t) {
     return 1.0f / sqrtf(acc / static_cast<float>(p.nb * 256) + p.norm_eps);
 }
 
-template <int RT>
 __global__ __launch_bounds__(256) void reduce_splits(BatchParams p) {
-    constexpr int kGroupRows = group_rows(RT);
-    constexpr int kPartialFloats = partial_floats(RT);
     const int64_t u = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int64_t slot = u / kPartialFloats;
     const int rem = static_cast<int>(u - slot * kPartialFloats);
     const int group = static_cast<int>(slot / p.tiles), tile = static_cast<int>(slot - static_cast<int64_t>(group) * p.tiles);
-    const int wave = rem / (RT * 1024), i = (rem / 1024) % RT, k = (rem / 64) % 16, lane = rem % 64;
+    const int wave = rem / 1024, k = (rem / 64) % 16, lane = rem % 64;
     const int kh = lane >> 5, col = lane & 31;
     int m = 0;
     #pragma unroll
@@ -637,7 +629,7 @@ __global__ __launch_bounds__(256) void reduce_splits(BatchParams p) {
     for (int sp = 1; sp < kMaxSplit; ++sp)
         if (sp < p.splits) sum += v[sp];
     // Accumulator register k holds token 8*(k/4) + 4*kh + k%4 of its tile.
-    const int row = (group - M.group_begin) * kGroupRows + (i * 4 + wave) * 32 + col;
+    const int row = (group - M.group_begin) * kGroupRows + wave * 32 + col;
     const int t = tile * kTokTile + 8 * (k >> 2) + 4 * kh + (k & 3);
     if (row >= M.rows || t >= p.n_tokens) return;
     if (p.in_ss) sum *= input_norm_scale(p, t);
@@ -656,10 +648,7 @@ __global__ __launch_bounds__(256) void reduce_splits(BatchParams p) {
 // up pair).  Then every lane packs its four values of the next GEMM's input
 // block -- x * gain with the block's sum of squares of x, or SiLU(gate) * up
 // -- into the record (the pack kernel's layout, stage_store_wave).
-template <int RT>
 __global__ __launch_bounds__(64) void reduce_pack(BatchParams p) {
-    constexpr int kGroupRows = group_rows(RT);
-    constexpr int kPartialFloats = partial_floats(RT);
     const int ob = blockIdx.x;
     const int tile = blockIdx.y / kTokTile;
     const int lane = threadIdx.x;
@@ -675,7 +664,7 @@ __global__ __launch_bounds__(64) void reduce_pack(BatchParams p) {
         const int g = M.group_begin + row_q / kGroupRows, rr = (row_q % kGroupRows) / 32;
         const int64_t slot = static_cast<int64_t>(g) * p.tiles + tile;
         return reinterpret_cast<const float4 *>(p.partials + (slot * p.splits + sp) * kPartialFloats +
-                                                (rr & 3) * (RT * 1024) + (rr >> 2) * 1024 + k * 64 + kh * 32 +
+                                                rr * 1024 + k * 64 + kh * 32 +
                                                 part * 4);
     };
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -739,11 +728,13 @@ int check_batched(const char *where, const float *x, int ldx, int cols, int n_to
 
 int tile_count(int n_tokens) { return (n_tokens + kTokTile - 1) / kTokTile; }
 
-// Token tiles per workgroup: two once there are two tiles (each decoded
-// weight operand then feeds 64 tokens), else one.  The row tiles per wave
-// follow it.
-int token_tiles_per_group(int tiles) { return tiles >= 2 ? 2 : 1; }
-int row_tiles(int tiles) { return token_tiles_per_group(tiles); }
+// The workspace's size: what a GEMM of 128 * RT rows x 32 * RT tokens a
+// workgroup with split_plan's splits needs (RT 1 for one token tile, else 2).
+// The launches fit their own plans into it.
+int row_tiles(int tiles) { return tiles >= 2 ? 2 : 1; }
+constexpr int group_rows(int rt) { return 128 * rt; }
+constexpr int partial_floats(int rt) { return 4 * rt * 16 * 64; }
+static_assert(group_rows(1) == kGroupRows && partial_floats(1) == kPartialFloats, "one token tile's groups");
 
 // Workgroups sharing a row group's blocks: enough that about one workgroup
 // per CU is in flight (two with one row tile), at most kMaxSplit, at least
@@ -753,7 +744,7 @@ int row_tiles(int tiles) { return token_tiles_per_group(tiles); }
 // tokens: one per CU 2.14 ms per 1B step, two per CU 2.20 ms; with one row
 // tile, two per CU 1.94 ms against 1.98 at one).
 void split_plan(int64_t groups, int nb, int tiles, int &splits, int &per_split) {
-    const int tt = token_tiles_per_group(tiles);
+    const int tt = row_tiles(tiles);
     const int64_t target = static_cast<int64_t>(device_info().cus) * (row_tiles(tiles) == 1 ? 2 : 1);
     const int64_t have = std::max<int64_t>(1, groups * ((tiles + tt - 1) / tt));
     const int64_t want = (target + have - 1) / have;
@@ -814,16 +805,61 @@ size_t workspace_bound(int cols, int rows_total, int n_tokens, bool partials = f
     return bytes + best;
 }
 
-template <int TT>
-void launch_gemm(int type, const dim3 &grid, size_t lds, hipStream_t stream, const BatchParams &p) {
+void launch_gemm(int type, const dim3 &grid, hipStream_t stream, const BatchParams &p) {
+    constexpr size_t lds = 2 * kTileBytes;
     if (type == QK_TYPE_Q4_K)
-        hipLaunchKernelGGL((batch_gemm<QK_TYPE_Q4_K, TT>), grid, dim3(256), lds, stream, p);
+        hipLaunchKernelGGL(batch_gemm<QK_TYPE_Q4_K>, grid, dim3(256), lds, stream, p);
     else if (type == QK_TYPE_Q6_K)
-        hipLaunchKernelGGL((batch_gemm<QK_TYPE_Q6_K, TT>), grid, dim3(256), lds, stream, p);
+        hipLaunchKernelGGL(batch_gemm<QK_TYPE_Q6_K>, grid, dim3(256), lds, stream, p);
     else if (type == QK_TYPE_Q6_K_SPLIT)
-        hipLaunchKernelGGL((batch_gemm<QK_TYPE_Q6_K_SPLIT, TT>), grid, dim3(256), lds, stream, p);
+        hipLaunchKernelGGL(batch_gemm<QK_TYPE_Q6_K_SPLIT>, grid, dim3(256), lds, stream, p);
     else
-        hipLaunchKernelGGL((batch_gemm<0, TT>), grid, dim3(256), lds, stream, p);
+        hipLaunchKernelGGL(batch_gemm<0>, grid, dim3(256), lds, stream, p);
+}
+
+void launch_tile_gemm(int type, int64_t groups, hipStream_t stream, const BatchParams &p) {
+    const int tgroups = (p.tiles + 1) / 2, g = static_cast<int>(groups);
+    const dim3 grid(static_cast<unsigned>((groups * tgroups * p.splits + 7) / 8 * 8));
+    if (type == QK_TYPE_Q4_K)
+        hipLaunchKernelGGL(tile_gemm<QK_TYPE_Q4_K>, grid, dim3(256), kTileLds, stream, p, g, tgroups);
+    else if (type == QK_TYPE_Q6_K)
+        hipLaunchKernelGGL(tile_gemm<QK_TYPE_Q6_K>, grid, dim3(256), kTileLds, stream, p, g, tgroups);
+    else if (type == QK_TYPE_Q6_K_SPLIT)
+        hipLaunchKernelGGL(tile_gemm<QK_TYPE_Q6_K_SPLIT>, grid, dim3(256), kTileLds, stream, p, g, tgroups);
+    else
+        hipLaunchKernelGGL(tile_gemm<0>, grid, dim3(256), kTileLds, stream, p, g, tgroups);
+}
+
+// How many workgroups share one row group's blocks: the count with the least
+// estimated time.  A workgroup alone on its CU takes kBlockUs a Q4_K block
+// (kWideUs a Q6_K block, three chains), two on one CU twice that each
+// (csrc/qk_tile_gemm.h); a split's partial sums cost kPartialUsPerMb written
+// and read back, and the reduction kReduceUs once there are any.  Measured
+// against every count from 1 to 16 at 64 to 517 tokens on the 1B and 3B
+// shapes: within 2 us of the best.  max_splits bounds it by the workspace.
+void tile_split_plan(const BatchParams &p, int64_t groups, int max_splits, bool must_reduce, int &splits,
+                     int &per_split) {
+    constexpr double kBlockUs = 2.5, kWideUs = 3.4, kPartialUsPerMb = 0.4, kReduceUs = 4.;
+    const int64_t cus = device_info().cus, wide = (p.tiles + 1) / 2 * groups;
+    double block_us = 0., out_mb = 0.;
+    for (int i = 0; i < p.n_mats; ++i) {
+        block_us = std::max(block_us, p.mat[i].type == QK_TYPE_Q4_K ? kBlockUs : kWideUs);
+        out_mb += 4e-6 * p.mat[i].rows * p.n_tokens;
+    }
+    double best = 0.;
+    for (int s = 1; s <= std::min(std::min(max_splits, kMaxSplit), p.nb); ++s) {
+        const int per = (p.nb + s - 1) / s;
+        if ((p.nb + per - 1) / per != s) continue;
+        const int64_t wgs = wide * s, rest = wgs % (2 * cus);
+        const double rounds = 2. * static_cast<double>(wgs / (2 * cus)) + (rest > cus ? 2. : rest > 0 ? 1. : 0.);
+        const double us = rounds * per * block_us + (s > 1 || must_reduce ? s * out_mb * kPartialUsPerMb : 0.) +
+                          (s > 1 && !must_reduce ? kReduceUs : 0.);
+        if (best == 0. || us < best) {
+            best = us;
+            splits = s;
+            per_split = per;
+        }
+    }
 }
 
 int launch_mfma(const qk_matrix *mats, int n_mats, const int *ldy, const float *x, int ldx, int cols, int n_tokens,
@@ -831,8 +867,6 @@ int launch_mfma(const qk_matrix *mats, int n_mats, const int *ldy, const float *
                 const GemvFusion *fusion = nullptr) {
     const int nb = cols / 256;
     const int tiles = tile_count(n_tokens);
-    const int tt = token_tiles_per_group(tiles);
-    const int rt = row_tiles(tiles);
     if (tiles > 65535) return fail(QK_ERR_LIMIT, std::string(where) + ": too many tokens in one launch");
     BatchParams p{};
     p.n_mats = n_mats;
@@ -853,33 +887,40 @@ int launch_mfma(const qk_matrix *mats, int n_mats, const int *ldy, const float *
         M.row_bytes = static_cast<int>(row_bytes(M.type, nb));
         M.ldy = ldy[i];
         M.group_begin = static_cast<int>(groups);
-        groups += (M.rows + group_rows(rt) - 1) / group_rows(rt);
+        groups += (M.rows + kGroupRows - 1) / kGroupRows;
         rows[i] = M.rows;
         if (static_cast<int64_t>(M.rows) * M.row_bytes > (int64_t(1) << 40))
             return fail(QK_ERR_LIMIT, std::string(where) + ": matrix too large");
         if (M.type != type) type = 0;
     }
-    split_plan(groups, nb, tiles, p.splits, p.blocks_per_split);
-    if (groups * p.splits > (1 << 30)) return fail(QK_ERR_LIMIT, std::string(where) + ": too many rows");
+    if (groups * kMaxSplit * tiles > (1 << 30)) return fail(QK_ERR_LIMIT, std::string(where) + ": too many rows");
     // A decode chain's reduction stage (deferred input norm, or packing the
     // next call's records) runs even without a split.
     const bool chain_out = fusion && fusion->out_records;
-    const bool need_partials = p.splits > 1 || (fusion && fusion->in_ss) || chain_out;
+    const bool must_reduce = (fusion && fusion->in_ss) || chain_out;
     if (chain_out) {
         const bool pair = fusion->pair != 0;
         if ((pair && (n_mats != 2 || rows[0] != rows[1])) || (!pair && n_mats != 1) || rows[0] % 256 ||
             (!pair && !fusion->out_gain) || (fusion->out_gain && !fusion->out_ss))
             return fail(QK_ERR_INVALID_ARG, std::string(where) + ": unsupported chained reduction");
     }
-    const size_t need = workspace_bytes(cols, rows, n_mats, n_tokens, need_partials);
+    const size_t need = workspace_bytes(cols, rows, n_mats, n_tokens, must_reduce);
     if (!workspace || workspace_size < need)
         return fail(QK_ERR_INVALID_ARG, std::string(where) + ": workspace smaller than " + std::to_string(need) +
                                             " bytes (qk_gemv_batched_workspace_bytes)");
     if (!aligned(workspace, 256)) return fail(QK_ERR_ALIGN, std::string(where) + ": workspace not 256-byte aligned");
     uint8_t *ws = static_cast<uint8_t *>(workspace);
-    const int tgroups = (tiles + tt - 1) / tt;
+    const size_t rec_bytes = (records_bytes(cols, n_tokens) + 255) / 256 * 256;
+    if (tiles == 1) {
+        split_plan(groups, nb, tiles, p.splits, p.blocks_per_split);
+    } else {
+        const size_t slot = static_cast<size_t>(groups) * tiles * kPartialFloats * sizeof(float);
+        const int fit = static_cast<int>(std::min<size_t>(kMaxSplit, (workspace_size - rec_bytes) / slot));
+        tile_split_plan(p, groups, std::max(fit, 1), must_reduce, p.splits, p.blocks_per_split);
+    }
+    const bool need_partials = p.splits > 1 || must_reduce;
     p.records = ws;
-    if (need_partials) p.partials = reinterpret_cast<float *>(ws + (records_bytes(cols, n_tokens) + 255) / 256 * 256);
+    if (need_partials) p.partials = reinterpret_cast<float *>(ws + rec_bytes);
     if (fusion) {
         p.norm_w = fusion->norm_w;
         p.norm_eps = fusion->norm_eps;
@@ -895,25 +936,16 @@ int launch_mfma(const qk_matrix *mats, int n_mats, const int *ldy, const float *
     }
     if (!(fusion && fusion->in_records))
         hipLaunchKernelGGL(pack_activations, dim3(nb, tiles * (kTokTile / kPackTokens)), dim3(256), 0, stream, p, ws);
-    const dim3 grid(static_cast<unsigned>(groups * p.splits), tgroups);
-    const size_t lds = 2 * static_cast<size_t>(tt) * kTileBytes;
-    if (tt == 2)
-        launch_gemm<2>(type, grid, lds, stream, p);
+    if (tiles == 1)
+        launch_gemm(type, dim3(static_cast<unsigned>(groups * p.splits)), stream, p);
     else
-        launch_gemm<1>(type, grid, lds, stream, p);
-    if (chain_out) {
-        const dim3 rgrid(static_cast<unsigned>(p.out_nb), static_cast<unsigned>(tiles * kTokTile));
-        if (rt == 2)
-            hipLaunchKernelGGL(reduce_pack<2>, rgrid, dim3(64), 0, stream, p);
-        else
-            hipLaunchKernelGGL(reduce_pack<1>, rgrid, dim3(64), 0, stream, p);
-    } else if (need_partials) {
-        const dim3 rgrid(static_cast<unsigned>(groups * tiles * (partial_floats(rt) / 256)));
-        if (rt == 2)
-            hipLaunchKernelGGL(reduce_splits<2>, rgrid, dim3(256), 0, stream, p);
-        else
-            hipLaunchKernelGGL(reduce_splits<1>, rgrid, dim3(256), 0, stream, p);
-    }
+        launch_tile_gemm(type, groups, stream, p);
+    if (chain_out)
+        hipLaunchKernelGGL(reduce_pack, dim3(static_cast<unsigned>(p.out_nb), static_cast<unsigned>(tiles * kTokTile)),
+                           dim3(64), 0, stream, p);
+    else if (need_partials)
+        hipLaunchKernelGGL(reduce_splits, dim3(static_cast<unsigned>(groups * tiles * (kPartialFloats / 256))),
+                           dim3(256), 0, stream, p);
     return launch_status(where);
 }
 

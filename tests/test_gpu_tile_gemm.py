@@ -1,0 +1,77 @@
+"""The matrix-core GEMM of two token tiles and more (csrc/qk_tile_gemm.h) at
+the edges of its tiles: token counts around multiples of 32 and 64, row counts
+around multiples of 32 and 128, one block and odd block counts, every storage
+type alone and mixed in one launch, with and without split sums."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2, to_dev
+
+pytestmark = pytest.mark.gpu
+Q4_K, Q6_K, Q6_K_SPLIT = 12, 14, 114
+# Activations carry 22 bits (2^-22 of a value), the fp32 sums of a block's 256
+# products up to about sqrt(256) roundings of 2^-24: 1.2e-6 together.
+TOL = 2e-6
+
+
+def matrix(qk, t, workloads, synth, qtype, cols, rows, seed):
+    """(tensor, host bytes as the oracle reads them, oracle type)."""
+    if qtype == Q4_K:
+        w, _ = workloads.gemv_case(Q4_K, cols, rows, seed=seed)
+        return qk.Tensor((cols, rows), Q4_K, to_dev(t, w)), w, Q4_K
+    w = synth.quant_matrix(Q6_K, cols, rows, seed, 1).reshape(-1, 210).copy()
+    # Every third block's scales over the whole int8 range: the wave takes
+    # the third chain where one of its rows has such a block.
+    wide = synth.uniform_i32(w.shape[0] * 16, seed, 2, -128, 127).astype(np.int8).reshape(-1, 16)
+    w[::3, 192:208] = wide[::3].view(np.uint8)
+    w = w.reshape(-1)
+    g = qk.Tensor((cols, rows), Q6_K, to_dev(t, w))
+    if qtype == Q6_K:
+        return g, w, Q6_K
+    s = qk.split_q6k(g)
+    t.cuda.synchronize()
+    return s, w, Q6_K
+
+
+def check(qk, t, oracle, tensors, x, cols, extra=0):
+    ntok = x.shape[0]
+    rows = [ten.rows() for ten, _, _ in tensors]
+    nws = qk.batch_workspace_bytes(cols, sum(rows), ntok) + extra
+    ws = t.empty(max(nws, 256), dtype=t.uint8, device="cuda")
+    ys = [t.full((ntok, r), float("nan"), device="cuda") for r in rows]
+    xd = to_dev(t, x)
+    arr = qk._matrices([(ten, y) for (ten, _, _), y in zip(tensors, ys)])
+    qk.check(qk.lib().qk_gemv_multi_batched_f32(arr, len(tensors), xd.data_ptr(), cols, cols, ntok, ws.data_ptr(), nws,
+                                                None), "multi batched")
+    t.cuda.synchronize()
+    for (ten, w, qtype), y in zip(tensors, ys):
+        want = oracle.gemv_f64(qtype, w, x, cols, ten.rows())
+        # Over all tokens: one output of one row may cancel to far below its
+        # terms (its error is bounded by their size, not its own); the norm
+        # over the tokens does not.
+        assert rel_l2(y.cpu().numpy(), want) < TOL, qtype
+
+
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q6_K_SPLIT])
+@pytest.mark.parametrize("ntok,cols,rows", [(33, 256, 31), (64, 512, 129), (65, 768, 128), (97, 2048, 640),
+                                            (128, 1280, 33), (129, 3072, 257)])
+def test_edges(qk, torch_gpu, oracle, workloads, synth, qtype, ntok, cols, rows):
+    x = synth.normal_f32(ntok * cols, 31, ntok).reshape(ntok, cols)
+    check(qk, torch_gpu, oracle, [matrix(qk, torch_gpu, workloads, synth, qtype, cols, rows, 30 + ntok)], x, cols)
+
+
+@pytest.mark.parametrize("ntok", [34, 96, 161])
+def test_mixed_types(qk, torch_gpu, oracle, workloads, synth, ntok):
+    cols = 1024
+    x = synth.normal_f32(ntok * cols, 32, ntok).reshape(ntok, cols)
+    tensors = [matrix(qk, torch_gpu, workloads, synth, ty, cols, rows, 40 + i)
+               for i, (ty, rows) in enumerate([(Q4_K, 130), (Q6_K, 96), (Q6_K_SPLIT, 257), (Q4_K, 1)])]
+    check(qk, torch_gpu, oracle, tensors, x, cols)
+
+
+def test_large_workspace_splits(qk, torch_gpu, oracle, workloads, synth):
+    """Room for more splits than the queried size holds."""
+    ntok, cols, rows = 40, 4096, 200
+    x = synth.normal_f32(ntok * cols, 33, ntok).reshape(ntok, cols)
+    t = torch_gpu
+    check(qk, t, oracle, [matrix(qk, t, workloads, synth, Q4_K, cols, rows, 50)], x, cols, extra=8 << 20)
