@@ -476,6 +476,10 @@ struct SplitAttention {
     const float *qkv_parts;
     int qkv_splits, qkv_ttiles, qkv_tile0[3];
     int layer, pos, max_pos, n_tokens, heads, kv_heads, head_dim;
+    // 16-token tiles whose tokens share their rows take the tile kernel
+    // (csrc/qk_tile_attention.hip): 0 none, 1 those tiles (the other tokens
+    // one by one), 2 every tile is one (tile_attention_mode).
+    int tile_mode;
     // Cache layout: 0 the reference's [layers][cache_rows][kv_heads][head_dim],
     // 1 [layers][kv_heads][cache_rows][head_dim] (the decode drivers' own: a
     // (token, KV head) workgroup then reads one contiguous run of memory
@@ -490,6 +494,48 @@ __host__ __device__ __forceinline__ int64_t kv_offset(int head_major, int layer,
                       : (static_cast<int64_t>(layer) * cache_rows + row) * kv_heads * head_dim +
                             static_cast<int64_t>(h) * head_dim;
 }
+// Whether a token's descriptor lies in the cache: written without kv_row +
+// pos, which a huge kv_row would overflow.
+__host__ __device__ __forceinline__ bool token_ok(const qk_batch_token &d, int64_t cache_rows, int max_pos) {
+    return d.pos >= 0 && d.pos <= max_pos && d.kv_row >= 0 && d.kv_row < cache_rows - d.pos;
+}
+
+// Tokens t0 .. t0 + 15 of a batch as a tile of the tile attention: shared when
+// all of them are valid and form at most kMaxRuns runs of consecutive
+// positions of one sequence.  Taken by a whole wave, lane l for token t0 +
+// l % 16.
+constexpr int kAttnTile = 16;
+constexpr int kMaxRuns = 2;
+struct TokenTile {
+    bool shared;
+    unsigned starts;   // bit i: token t0 + i begins a run
+    int pos;           // of this lane's token (the last token's past the end)
+    int64_t kv_row;
+};
+__device__ __forceinline__ TokenTile token_tile(const qk_batch_token *desc, int t0, int n_tokens, int64_t cache_rows,
+                                                int max_pos, int lane) {
+    const int n = lane & 15, have = min(kAttnTile, n_tokens - t0);
+    const qk_batch_token d = desc[min(t0 + n, n_tokens - 1)];
+    const int prev = max(lane - 1, 0);
+    const int lo = static_cast<int>(d.kv_row), hi = static_cast<int>(d.kv_row >> 32);
+    const bool follows = __shfl(d.pos, prev) == d.pos - 1 && __shfl(lo, prev) == lo && __shfl(hi, prev) == hi;
+    const bool start = n < have && (n == 0 || !follows);
+    const unsigned starts = static_cast<unsigned>(__builtin_amdgcn_ballot_w64(start)) & 0xFFFFu;
+    const bool ok = __builtin_amdgcn_ballot_w64(n < have && !token_ok(d, cache_rows, max_pos)) == 0;
+    return {ok && __builtin_popcount(starts) <= kMaxRuns, starts, d.pos, d.kv_row};
+}
+
+// The tile kernel serves a's layout (head_dim 64 or 128, caches already
+// holding every row); takes less time than the per-token form for n_tokens
+// tokens of `rows` rows in all, the longest max_rows; runs.
+bool tile_attention_supported(const SplitAttention &a);
+bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int max_rows);
+int launch_tile_attention(const SplitAttention &a, hipStream_t stream);
+// SplitAttention::tile_mode of a batch whose descriptors the host holds
+// (valid ones): by the tiles' own test, when it pays.  Sets a.rows_hint to
+// the rows left to the per-token form.
+int tile_attention_mode(const qk_batch_token *desc, SplitAttention &a);
+
 // RoPE of q and k at each token's position, k and v written to row kv_row +
 // pos of the caches in either layout (qk_rope_kv_write_batched's kernel;
 // arguments validated by the caller).

@@ -1314,6 +1314,7 @@ int qk_llama_batch_forward_rows(qk_llama_batch *m, const int32_t *tokens, const 
     attn.heads = c.heads;
     attn.kv_heads = c.kv_heads;
     attn.head_dim = hd;
+    if (chained) attn.tile_mode = qk::tile_attention_mode(desc, attn);
     // From 8 tokens on (matrix cores) the projections chain: attention packs
     // its outputs as o's records, o's reduction adds the residual and packs
     // x * ffn_norm for gate/up (sums of squares for the deferred RMSNorm),

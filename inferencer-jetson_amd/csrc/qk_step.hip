@@ -175,11 +175,6 @@ __device__ __forceinline__ float dot4(const float4 &a, const float4 &b, float ac
 // a ragged batch.  A token whose descriptor falls outside the cache is not
 // written and its attention output is NaN.
 
-// Written without kv_row + pos, which a huge kv_row would overflow.
-__device__ __forceinline__ bool token_ok(const qk_batch_token &d, int64_t cache_rows, int max_pos) {
-    return d.pos >= 0 && d.pos <= max_pos && d.kv_row >= 0 && d.kv_row < cache_rows - d.pos;
-}
-
 __global__ void rope_kv_batched_kernel(float *q, const float *k, const float *v, const float *cosine,
                                        const float *sine, float *key_cache, float *value_cache, int layer,
                                        int64_t cache_rows, const qk_batch_token *desc, int context, int q_pairs,
@@ -241,7 +236,14 @@ struct SplitAttnKernelArgs {
     int split_rows;
     int splits;        // most splits of any token (the partials' stride)
     int head_split;    // workgroups sharing a KV head, each with heads / kv_heads / head_split query heads
+    int tiled;         // tokens of shared tiles are tile_attention's: leave them out
 };
+
+// Whether token b belongs to a tile that tile_attention serves.
+__device__ __forceinline__ bool tile_token(const SplitAttnKernelArgs &ka, int b) {
+    return ka.tiled && token_tile(ka.a.desc, b / kAttnTile * kAttnTile, ka.a.n_tokens, ka.a.cache_rows, ka.a.max_pos,
+                                  threadIdx.x & 63).shared;
+}
 
 // A split partial: max [G], sum of exp [G], padded to 16 bytes, then the
 // unnormalised output rows [G][head_dim].
@@ -438,6 +440,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(SplitAttnKerne
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = lane % L, rq = lane / L;
     const int hd = a.head_dim, hv = hd / 4, kv_dim = a.kv_heads * hd, half = hd / 2;
+    if (tile_token(ka, b)) return;
     const qk_batch_token d = a.desc ? a.desc[b] : qk_batch_token{a.pos, 0, 0};
     float *o = a.out + static_cast<int64_t>(b) * a.heads * hd + kvh * G * hd;
     if (!token_ok(d, a.cache_rows, a.max_pos)) {
@@ -667,6 +670,7 @@ __global__ __launch_bounds__(256) void split_merge_kernel(SplitAttnKernelArgs ka
     __shared__ float mo[G * 256];   // the merged outputs, for the records (head_dim <= 256)
     const SplitAttention &a = ka.a;
     const int kvh = blockIdx.x, b = blockIdx.y;
+    if (tile_token(ka, b)) return;
     const qk_batch_token d = a.desc ? a.desc[b] : qk_batch_token{a.pos, 0, 0};
     if (!token_ok(d, a.cache_rows, a.max_pos)) return;
     const int nsplit = (d.pos + ka.split_rows) / ka.split_rows;
@@ -855,6 +859,17 @@ const void *split_merge_instance(int G) {
 
 inline hipStream_t S(qk_stream s) { return static_cast<hipStream_t>(s); }
 
+// tile_mode of a call whose descriptors are on the device: n tokens of
+// sequences of their own hold at most cache_rows rows together, so when
+// n * (max_pos + 1) is far beyond that, tokens share rows (a prefill chunk) and
+// the tile kernel goes first; each tile's descriptors decide.  A decode batch
+// stays below it and launches no tile kernel.
+int call_tile_mode(const SplitAttention &a) {
+    const int64_t rows = static_cast<int64_t>(a.n_tokens) * (a.max_pos + 1);
+    return rows / 8 >= a.cache_rows && tile_attention_supported(a) &&
+           tile_attention_pays(a.n_tokens, a.kv_heads, a.heads, a.head_dim, rows / 4 * 3, a.max_pos + 1);
+}
+
 }  // namespace
 
 int split_attention_rows(int64_t head_rows, int max_rows) {
@@ -898,6 +913,14 @@ int launch_split_attention(const SplitAttention &a, int split_rows, void *worksp
         return fail(QK_ERR_LIMIT, "split attention: quantized outputs need head_dim % 32 == 0 and scales");
     if (a.qkv_splits > 1 && (!a.qkv_parts || !a.k || !a.v || a.qkv_ttiles < (a.n_tokens + 31) / 32))
         return fail(QK_ERR_INVALID_ARG, "split attention: split QKV sums need k, v and their partials");
+    // Tiles of tokens that share their rows (csrc/qk_tile_attention.hip), then
+    // the tokens outside such tiles, if there may be any.
+    int tile_mode = split_rows <= 0 && tile_attention_supported(a) ? a.tile_mode : 0;
+    if (splits_used) *splits_used = 1;
+    if (tile_mode) {
+        if (int st = launch_tile_attention(a, stream)) return st;
+        if (tile_mode == 2) return QK_OK;
+    }
     const int max_rows = a.max_pos + 1;
     // Few (token, KV head) pairs over short rows: one wide workgroup each
     // reads all of its rows, and no merge kernel runs.  A CU alone streams
@@ -946,6 +969,7 @@ int launch_split_attention(const SplitAttention &a, int split_rows, void *worksp
     ka.split_rows = split_rows;
     ka.splits = nsplit;
     ka.head_split = head_split;
+    ka.tiled = tile_mode;
     void *args[] = {&ka};
     if (hipLaunchKernel(fn, dim3(groups, a.n_tokens, nsplit), dim3(wide ? kWideWaves * 64 : kSplitThreads), args,
                         0, stream) != hipSuccess)
@@ -1063,6 +1087,7 @@ int qk_attention_f32(const float *q, const float *key_cache, const float *value_
     a.heads = heads;
     a.kv_heads = kv_heads;
     a.head_dim = head_dim;
+    a.tile_mode = qk::call_tile_mode(a);
     return qk::launch_split_attention(a, 0, nullptr, 0, qk::S(stream));
 }
 
@@ -1122,6 +1147,7 @@ int qk_attention_batched_f32(const float *q, const float *key_cache, const float
     a.heads = heads;
     a.kv_heads = kv_heads;
     a.head_dim = head_dim;
+    a.tile_mode = qk::call_tile_mode(a);
     return qk::launch_split_attention(a, 0, nullptr, 0, qk::S(stream));
 }
 
@@ -1164,6 +1190,7 @@ int qk_attention_split_f32(const float *q, const float *key_cache, const float *
     a.heads = heads;
     a.kv_heads = kv_heads;
     a.head_dim = head_dim;
+    a.tile_mode = qk::call_tile_mode(a);
     return qk::launch_split_attention(a, split_rows, workspace, workspace_size, qk::S(stream));
 }
 

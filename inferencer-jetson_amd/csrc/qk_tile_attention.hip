@@ -1,0 +1,411 @@
+// qk_tile_attention.hip - attention of prefill chunks: 16 consecutive tokens
+// of a batch that continue one sequence share its cache rows.
+//
+// split_attention_kernel (csrc/qk_step.hip) reads a token's rows once per
+// token: a 512-token chunk over 600 earlier rows read 3.6 GB through L2, 152
+// us at 24 TB/s.  Here a workgroup takes 16 tokens x one KV head with all its
+// query heads and reads every cache row once for them; both products run on
+// the FP32 matrix instructions (v_mfma_f32_16x16x4_f32), whose operands and
+// sums are fp32 as before, so the bound is their 157 TFLOP/s (34 us for that
+// chunk).  Measured: that chunk (24 heads over 8 KV heads of 128) 152 -> 80.7
+// us; 512 tokens from position 0, 84 -> 45 us (32 heads over 8 of 64: 51 -> 31
+// us); 1024 tokens over 3072 earlier rows, 1041 -> 469 us.
+//
+//   * Wave (g, s) of G x S waves (S at most 4): query head g, every S-th tile
+//     of 32 cache rows.  The products are taken transposed, scores S^T = K Q^T and outputs
+//     O^T = V^T P^T: a lane then holds one token's scores, the softmax needs
+//     two cross-lane steps, and the probabilities are the second product's
+//     operand as they stand.
+//   * Key and value tiles come into LDS by direct copies, each split group
+//     its own: the next key tile loads while the values are multiplied, the
+//     next value tile while the next scores are.  Keys are stored with their
+//     16-byte chunks rotated by row (chunk ^ row % 16), so the 16 rows of an
+//     operand read fall into different banks.
+//   * The S partial states of a head meet in LDS (merge as in
+//     split_merge_kernel) and the outputs leave through LDS, which also
+//     serves the o projection's records or codes.
+//
+// A tile runs here when its tokens are all valid and form at most kMaxRuns
+// runs of consecutive positions of one sequence (each run walks its own
+// rows); the other tiles' tokens go through split_attention_kernel, which
+// decides by the same test.
+#include "qk_internal.h"
+#include "qk_records.h"
+
+#include <algorithm>
+
+namespace qk {
+namespace {
+
+typedef float float4v __attribute__((ext_vector_type(4)));
+
+constexpr int kKeys = 32;            // cache rows of a tile
+// Waves of a workgroup at most: 128 registers a lane at head_dim 64, 168 at 128
+// (with 16 waves it spilled 33).
+constexpr int max_waves(int hd) { return hd == 64 ? 16 : 12; }
+
+struct TileAttnArgs {
+    SplitAttention a;
+    int groups;    // S: waves sharing a head's rows
+};
+
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void *)p));
+}
+
+// 16 bytes a lane to LDS at dst + 16 * lane (dst wave-uniform), untracked by
+// the compiler's wait insertion.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma16(const void *src, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+__device__ __forceinline__ void copies_barrier() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+constexpr int kv_bytes(int hd) { return kKeys * hd * 4; }
+
+// The outputs of one (token, head) taken plainly by one wave, for a token
+// whose tile result is not finite: an infinite or NaN value in a later
+// token's row reaches an earlier token of the tile as 0 * inf.
+template <int HD>
+__device__ void plain_token(const float *q, const float *kc, const float *vc, int64_t rs, int pos, float scale,
+                            int lane, float *out) {
+    float m = -INFINITY, l = 0.f;
+    auto score = [&](int key) {
+        const float *k = kc + key * rs;
+        float s = 0.f;
+        for (int d = 0; d < HD; ++d) s = fmaf(q[d], k[d], s);
+        return s * scale;
+    };
+    for (int key = lane; key <= pos; key += 64) {
+        const float s = score(key), mn = fmaxf(m, s);
+        const float ref = mn == -INFINITY ? 0.f : mn;
+        l = l * __builtin_amdgcn_exp2f(m - ref) + __builtin_amdgcn_exp2f(s - ref);
+        m = mn;
+    }
+    #pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const float mo = __shfl_xor(m, off), lo = __shfl_xor(l, off), mn = fmaxf(m, mo);
+        const float ref = mn == -INFINITY ? 0.f : mn;
+        l = l * __builtin_amdgcn_exp2f(m - ref) + lo * __builtin_amdgcn_exp2f(mo - ref);
+        m = mn;
+    }
+    const float ref = m == -INFINITY ? 0.f : m;
+    float acc[HD / 64];
+    #pragma unroll
+    for (int i = 0; i < HD / 64; ++i) acc[i] = 0.f;
+    for (int key = 0; key <= pos; ++key) {
+        const float p = __builtin_amdgcn_exp2f(score(key) - ref);
+        #pragma unroll
+        for (int i = 0; i < HD / 64; ++i) acc[i] = fmaf(p, vc[key * rs + i * 64 + lane], acc[i]);
+    }
+    #pragma unroll
+    for (int i = 0; i < HD / 64; ++i) out[i * 64 + lane] = acc[i] / l;
+}
+
+template <int HD>
+__global__ __launch_bounds__(max_waves(HD) * 64) void tile_attention(TileAttnArgs ta) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const SplitAttention &a = ta.a;
+    constexpr int NJ = HD / 16, NT = HD / 64;     // 16-dimension and 64-dimension steps
+    constexpr int kChunks = HD / 4;               // 16-byte chunks of a row
+    const int G = a.heads / a.kv_heads, S = ta.groups;
+    const int lane = threadIdx.x & 63, n = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = wave % G, sg = wave / G;
+    const int kvh = blockIdx.x, t0 = blockIdx.y * kAttnTile;
+
+    const TokenTile tile = token_tile(a.desc, t0, a.n_tokens, a.cache_rows, a.max_pos, lane);
+    if (!tile.shared) return;
+    const int t = min(t0 + n, a.n_tokens - 1);
+    const int64_t rs = a.head_major ? HD : static_cast<int64_t>(a.kv_heads) * HD;
+    const float scale = 1.4426950408889634f / sqrtf(static_cast<float>(HD));
+
+    float4 q[NJ];
+    const float *qrow = a.q + (static_cast<int64_t>(t) * a.heads + kvh * G + g) * HD + 4 * kq;
+    #pragma unroll
+    for (int j = 0; j < NJ; ++j) q[j] = *reinterpret_cast<const float4 *>(qrow + 16 * j);
+
+    float4v o[NT][4];
+    #pragma unroll
+    for (int x = 0; x < NT; ++x)
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) o[x][i] = float4v{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;   // this lane's token; l over this lane's rows only
+
+    unsigned char *const kbuf = lds + sg * 2 * kv_bytes(HD), *const vbuf = kbuf + kv_bytes(HD);
+    unsigned starts = tile.starts;
+    while (starts) {
+        // One run: tokens i0 .. i1 - 1, rows 0 .. last of its sequence.
+        const int i0 = __builtin_ctz(starts);
+        starts &= starts - 1;
+        const int i1 = starts ? __builtin_ctz(starts) : min(kAttnTile, a.n_tokens - t0);
+        const int last = __builtin_amdgcn_readfirstlane(__shfl(tile.pos, i1 - 1));
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(__shfl(static_cast<int>(tile.kv_row), i0));
+        const int hi = __builtin_amdgcn_readfirstlane(__shfl(static_cast<int>(tile.kv_row >> 32), i0));
+        const int64_t row = static_cast<int64_t>(hi) << 32 | lo;
+        const int mine = n >= i0 && n < i1 ? tile.pos : -1;   // rows this lane's token sees: 0 .. mine
+        const int64_t base = kv_offset(a.head_major, a.layer, a.cache_rows, a.kv_heads, HD, row, kvh);
+        const float *kc = a.key_cache + base, *vc = a.value_cache + base;
+        const int tiles = last / kKeys + 1, iters = (tiles + S - 1) / S;
+
+        // 1 KB of a tile is 256 / HD rows; the group's G waves share the
+        // pieces.  Rows past the last are the last again (in bounds; masked).
+        auto copy_tile = [&](const float *src, unsigned char *dst, int j, bool rotate) {
+            constexpr int kRowsPer = 256 / HD, kPieces = kKeys / kRowsPer;
+            for (int i = g; i < kPieces; i += G) {
+                const int r = i * kRowsPer + lane / kChunks, slot = lane % kChunks;
+                const int chunk = rotate ? slot ^ (r & 15) : slot;
+                dma16(src + static_cast<int64_t>(min(j * kKeys + r, last)) * rs + 4 * chunk, lds_address(dst + i * 1024));
+            }
+        };
+        copy_tile(kc, kbuf, sg, true);
+        copies_barrier();
+        copy_tile(vc, vbuf, sg, false);
+        for (int it = 0; it < iters; ++it) {
+            const int j = it * S + sg;
+            const bool live = j < tiles;
+            float4v st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            if (live) {
+                // Chains of 16 products (8 at head_dim 64), added as a tree: as
+                // exact as the per-token form's lane sums (2.1e-7 of float64
+                // at head_dim 128; 4.8e-7 as one chain over a head).
+                #pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    float4v part[2][4];
+                    #pragma unroll
+                    for (int e = 0; e < 4; ++e) part[0][e] = part[1][e] = float4v{0.f, 0.f, 0.f, 0.f};
+                    #pragma unroll
+                    for (int x = 0; x < NJ; ++x) {
+                        const float4 k =
+                            *reinterpret_cast<const float4 *>(kbuf + ((h * 16 + n) * kChunks + ((4 * x + kq) ^ n)) * 16);
+                        float4v(&c)[4] = part[x & 1];
+                        c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.x, q[x].x, c[0], 0, 0, 0);
+                        c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.y, q[x].y, c[1], 0, 0, 0);
+                        c[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.z, q[x].z, c[2], 0, 0, 0);
+                        c[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.w, q[x].w, c[3], 0, 0, 0);
+                    }
+                    #pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        st[h][r] = ((part[0][0][r] + part[0][1][r]) + (part[0][2][r] + part[0][3][r])) +
+                                   ((part[1][0][r] + part[1][1][r]) + (part[1][2][r] + part[1][3][r]));
+                }
+            }
+            copies_barrier();   // the values are in; every wave is done with the keys
+            if (it + 1 < iters) copy_tile(kc, kbuf, j + S, true);
+            if (live) {
+                // Register r of half h: row j * 32 + 16 h + 4 kq + r.
+                float mx = -INFINITY;
+                #pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    #pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        st[h][r] = j * kKeys + 16 * h + 4 * kq + r <= mine ? st[h][r] * scale : -INFINITY;
+                        mx = fmaxf(mx, st[h][r]);
+                    }
+                mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                const float mn = fmaxf(m, mx);
+                const float ref = mn == -INFINITY ? 0.f : mn;
+                const float f = __builtin_amdgcn_exp2f(m - ref);
+                m = mn;
+                #pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    #pragma unroll
+                    for (int r = 0; r < 4; ++r) st[h][r] = __builtin_amdgcn_exp2f(st[h][r] - ref);
+                l = fmaf(l, f, ((st[0][0] + st[0][1]) + (st[0][2] + st[0][3])) +
+                                   ((st[1][0] + st[1][1]) + (st[1][2] + st[1][3])));
+                // The tile's outputs on their own, then added: the chain over
+                // a head's rows is one step per tile.
+                #pragma unroll
+                for (int x = 0; x < NT; ++x) {
+                    float4v to[4];
+                    #pragma unroll
+                    for (int i = 0; i < 4; ++i) to[i] = float4v{0.f, 0.f, 0.f, 0.f};
+                    #pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        #pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float4 v = *reinterpret_cast<const float4 *>(
+                                vbuf + ((h * 16 + 4 * kq + r) * kChunks + 16 * x + n) * 16);
+                            to[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, st[h][r], to[0], 0, 0, 0);
+                            to[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, st[h][r], to[1], 0, 0, 0);
+                            to[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, st[h][r], to[2], 0, 0, 0);
+                            to[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, st[h][r], to[3], 0, 0, 0);
+                        }
+                    #pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        #pragma unroll
+                        for (int r = 0; r < 4; ++r) o[x][i][r] = fmaf(o[x][i][r], f, to[i][r]);
+                }
+            }
+            copies_barrier();   // the next keys are in; every wave is done with the values
+            if (it + 1 < iters) copy_tile(vc, vbuf, j + S, false);
+        }
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+
+    // The groups' states meet, in group order.
+    constexpr int kPart = 16 * HD + 32;   // floats of one wave's state: outputs, then (max, sum) per token
+    float *parts = reinterpret_cast<float *>(lds);
+    if (sg > 0) {
+        float *mine = parts + ((sg - 1) * G + g) * kPart;
+        #pragma unroll
+        for (int x = 0; x < NT; ++x)
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) *reinterpret_cast<float4v *>(mine + ((x * 4 + i) * 64 + lane) * 4) = o[x][i];
+        if (kq == 0) {
+            mine[16 * HD + 2 * n] = m;
+            mine[16 * HD + 2 * n + 1] = l;
+        }
+    }
+    __syncthreads();
+    if (sg == 0) {
+        for (int s = 1; s < S; ++s) {
+            const float *other = parts + ((s - 1) * G + g) * kPart;
+            const float mo = other[16 * HD + 2 * n], lo = other[16 * HD + 2 * n + 1];
+            const float mn = fmaxf(m, mo), ref = mn == -INFINITY ? 0.f : mn;
+            const float f = __builtin_amdgcn_exp2f(m - ref), fo = __builtin_amdgcn_exp2f(mo - ref);
+            m = mn;
+            l = l * f + lo * fo;
+            #pragma unroll
+            for (int x = 0; x < NT; ++x)
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float4v po = *reinterpret_cast<const float4v *>(other + ((x * 4 + i) * 64 + lane) * 4);
+                    #pragma unroll
+                    for (int r = 0; r < 4; ++r) o[x][i][r] = fmaf(po[r], fo, o[x][i][r] * f);
+                }
+        }
+    }
+    __syncthreads();   // the states are read: the output tile takes their place
+
+    // Outputs [16 tokens][G * HD]: register r of (x, i) is dimension 64 x +
+    // 16 kq + 4 r + i.
+    float *out = reinterpret_cast<float *>(lds);
+    const int width = G * HD;
+    if (sg == 0) {
+        bool finite = true;
+        #pragma unroll
+        for (int x = 0; x < NT; ++x)
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float4 v = make_float4(o[x][0][r] / l, o[x][1][r] / l, o[x][2][r] / l, o[x][3][r] / l);
+                finite = finite && isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
+                *reinterpret_cast<float4 *>(out + n * width + g * HD + 64 * x + 16 * kq + 4 * r) = v;
+            }
+        uint64_t bad = __builtin_amdgcn_ballot_w64(!finite && t0 + n < a.n_tokens);
+        bad = (bad | (bad >> 16) | (bad >> 32) | (bad >> 48)) & 0xFFFF;
+        while (bad) {
+            const int i = __builtin_ctzll(bad);
+            bad &= bad - 1;
+            const qk_batch_token d = a.desc[t0 + i];
+            const int64_t base = kv_offset(a.head_major, a.layer, a.cache_rows, a.kv_heads, HD, d.kv_row, kvh);
+            plain_token<HD>(a.q + (static_cast<int64_t>(t0 + i) * a.heads + kvh * G + g) * HD, a.key_cache + base,
+                            a.value_cache + base, rs, d.pos, scale, lane, out + i * width + g * HD);
+        }
+    }
+    __syncthreads();
+    const int have = min(kAttnTile, a.n_tokens - t0);
+    const int64_t ld = static_cast<int64_t>(a.heads) * HD;
+    for (int i = threadIdx.x; i < have * (width / 4); i += blockDim.x) {
+        const int tok = i / (width / 4), c = i - tok * (width / 4);
+        *reinterpret_cast<float4 *>(a.out + (t0 + tok) * ld + kvh * width + 4 * c) =
+            *reinterpret_cast<const float4 *>(out + tok * width + 4 * c);
+    }
+    // The o projection's input, 256 columns of one token a wave.
+    if (a.gemm_rec || a.q8_out) {
+        const int per = (width + 255) / 256, waves = blockDim.x / 64;
+        for (int i = wave; i < have * per; i += waves) {
+            const int tok = i / per, blk = i - tok * per, c = blk * 256 + 4 * lane, b = t0 + tok;
+            const bool in = c < width;
+            const float4 v = in ? *reinterpret_cast<const float4 *>(out + tok * width + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            if (a.gemm_rec) {
+                const float vr[4] = {v.x, v.y, v.z, v.w};
+                stage_store_wave(vr, lane, b % kTokTile,
+                                 a.gemm_rec + (static_cast<size_t>(b / kTokTile) * (a.heads * HD / 256) + kvh * per + blk) *
+                                                  kTileBytes);
+            }
+            if (a.q8_out && in) {
+                uint32_t codes;
+                const int64_t at = b * ld + kvh * width + c;
+                quantize_quad_store(v, (lane & 7) == 0, &codes, a.q8_scale + at / 32);
+                *reinterpret_cast<uint32_t *>(a.q8_out + at) = codes;
+            }
+        }
+    }
+}
+
+int tile_groups(int G, int hd) { return std::max(1, std::min(4, max_waves(hd) / G)); }
+
+}  // namespace
+
+bool tile_attention_supported(const SplitAttention &a) {
+    const int G = a.heads / a.kv_heads;
+    return (a.head_dim == 64 || a.head_dim == 128) && G <= 8 && a.desc && !a.k && !a.rec_out && aligned(a.q, 16) &&
+           (!a.gemm_rec || G * a.head_dim % 256 == 0) && (!a.q8_out || aligned(a.q8_out, 4));
+}
+
+// Whether 16-token tiles take less time than reading every token's rows: the
+// tile form walks ceil(rows / 32 / S) row tiles in 1.9 us per wave of a SIMD
+// at head_dim 128 (half that at 64), one workgroup per CU; the per-token form
+// reads all rows through L2 at about 20 TB/s.
+bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int max_rows) {
+    const int G = heads / kv_heads, S = tile_groups(G, head_dim);
+    const int64_t wgs = static_cast<int64_t>((n_tokens + kAttnTile - 1) / kAttnTile) * kv_heads;
+    const double rounds = static_cast<double>((wgs + device_info().cus - 1) / device_info().cus);
+    const double per_tile = 1.9 * head_dim / 128. * (G * S + 3) / 4;
+    const double tile_us = rounds * ((max_rows + kKeys - 1) / kKeys + S - 1) / S * per_tile;
+    const double split_us = static_cast<double>(rows) * kv_heads * head_dim * 8. / 20e6;
+    return n_tokens >= kAttnTile / 2 && 1.2 * tile_us < split_us;
+}
+
+int tile_attention_mode(const qk_batch_token *desc, SplitAttention &a) {
+    if (!tile_attention_supported(a)) return 0;
+    int64_t tiled_rows = 0, rows = 0;
+    int tiled = 0, max_rows = 0;
+    for (int t0 = 0; t0 < a.n_tokens; t0 += kAttnTile) {
+        const int t1 = std::min(t0 + kAttnTile, a.n_tokens);
+        int runs = 0, longest = 0;
+        int64_t tile_rows = 0;
+        for (int t = t0; t < t1; ++t) {
+            runs += t == t0 || desc[t].kv_row != desc[t - 1].kv_row || desc[t].pos != desc[t - 1].pos + 1;
+            tile_rows += desc[t].pos + 1;
+            longest = std::max(longest, desc[t].pos + 1);
+        }
+        if (runs <= kMaxRuns) {
+            tiled += t1 - t0;
+            tiled_rows += tile_rows;
+            max_rows = std::max(max_rows, longest);
+        } else {
+            rows += tile_rows;
+        }
+    }
+    if (!tiled || !tile_attention_pays(tiled, a.kv_heads, a.heads, a.head_dim, tiled_rows, max_rows)) return 0;
+    if (tiled == a.n_tokens) return 2;
+    a.rows_hint = rows;
+    return 1;
+}
+
+int launch_tile_attention(const SplitAttention &a, hipStream_t stream) {
+    TileAttnArgs ta{a, 1};
+    const int G = a.heads / a.kv_heads, hd = a.head_dim;
+    ta.groups = tile_groups(G, hd);
+    const size_t lds = std::max({static_cast<size_t>(ta.groups) * 2 * kv_bytes(hd),
+                                 static_cast<size_t>(ta.groups - 1) * G * (16 * hd + 32) * sizeof(float),
+                                 static_cast<size_t>(kAttnTile) * G * hd * sizeof(float)});
+    const dim3 grid(a.kv_heads, (a.n_tokens + kAttnTile - 1) / kAttnTile), block(64 * G * ta.groups);
+    if (hd == 64)
+        hipLaunchKernelGGL(tile_attention<64>, grid, block, lds, stream, ta);
+    else
+        hipLaunchKernelGGL(tile_attention<128>, grid, block, lds, stream, ta);
+    return launch_status("tile attention launch");
+}
+
+}  // namespace qk

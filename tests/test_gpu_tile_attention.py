@@ -1,0 +1,95 @@
+"""Attention of prefill chunks over shared rows (csrc/qk_tile_attention.hip)
+against float64: head layouts of every wave count, chunk lengths around the
+16-token tile and context lengths around the 32-row tile, chunks that begin or
+end inside a tile, tokens left to the per-token kernel, and values that are
+not finite in rows an earlier token must not see."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2, to_dev
+
+pytestmark = pytest.mark.gpu
+# fp32 products and sums over at most 700 rows and 128 dimensions: a score is
+# within about sqrt(128) * 2^-24 of its terms, a probability within that, the
+# output's sum within sqrt(700) * 2^-24: below 2e-6.
+TOL = 2e-6
+
+
+def reference(q, key, value, tokens, heads, kvh, hd):
+    """Float64 softmax attention of every (pos, first row) token."""
+    out = np.empty((len(tokens), heads * hd))
+    group = heads // kvh
+    k64, v64 = key.astype(np.float64), value.astype(np.float64)
+    for t, (pos, row) in enumerate(tokens):
+        for h in range(heads):
+            c = slice(h // group * hd, h // group * hd + hd)
+            s = k64[row:row + pos + 1, c] @ q[t, h * hd:(h + 1) * hd].astype(np.float64) / np.sqrt(hd)
+            p = np.exp(s - s.max())
+            out[t, h * hd:(h + 1) * hd] = p @ v64[row:row + pos + 1, c] / p.sum()
+    return out
+
+
+def run(qk, t, q, key, value, tokens, heads, kvh, hd, split_rows=0):
+    n, rows = len(tokens), key.shape[0]
+    top = max(p for p, _ in tokens)
+    desc = to_dev(t, np.array([[p | (i << 32), r] for i, (p, r) in enumerate(tokens)], dtype=np.int64))
+    nb = qk.lib().qk_attention_split_workspace_bytes(n, heads, kvh, hd, top, split_rows)
+    ws = t.empty(max(nb, 256), dtype=t.uint8, device="cuda")
+    out = t.full((n, heads * hd), float("nan"), device="cuda")
+    qd, kd, vd = to_dev(t, q), to_dev(t, key), to_dev(t, value)
+    qk.check(qk.lib().qk_attention_split_f32(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), 0, rows,
+                                             desc.data_ptr(), n, top, heads, kvh, hd, split_rows, ws.data_ptr(),
+                                             ws.numel(), None), "attention")
+    t.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def batch(rng, seqs, heads, kvh, hd):
+    """seqs: (rows after the chunk, chunk tokens) of each sequence."""
+    tokens, row = [], 0
+    for ctx, chunk in seqs:
+        tokens += [(ctx - chunk + i, row) for i in range(chunk)]
+        row += ctx
+    draw = lambda n, w: rng.standard_normal((n, w)).astype(np.float32)
+    return draw(len(tokens), heads * hd), draw(row, kvh * hd), draw(row, kvh * hd), tokens
+
+
+# Sizes at which the tile form is the shorter one (tile_attention_pays).
+@pytest.mark.parametrize("heads,kvh,hd", [(8, 8, 64), (16, 8, 64), (24, 8, 128), (32, 8, 64), (48, 8, 128), (64, 8, 64)])
+@pytest.mark.parametrize("seqs", [[(512, 512)], [(385, 337)], [(640, 300), (33, 17)], [(200, 200), (451, 243)]])
+def test_chunks(qk, torch_gpu, heads, kvh, hd, seqs):
+    rng = np.random.default_rng(heads * 1000 + len(seqs))
+    q, key, value, tokens = batch(rng, seqs, heads, kvh, hd)
+    got = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
+    pick = sorted(set(rng.integers(0, len(tokens), 24).tolist() + [0, 1, 15, 16, len(tokens) - 1]))
+    want = reference(q[pick], key, value, [tokens[i] for i in pick], heads, kvh, hd)
+    assert rel_l2(got[pick], want) < TOL
+    # Every token, against the per-token form (a split size given asks for it).
+    assert rel_l2(got, run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd, split_rows=256)) < TOL
+
+
+def test_decodes_beside_a_chunk(qk, torch_gpu):
+    """16-token tiles with more than two sequences go one token at a time."""
+    heads, kvh, hd = 32, 8, 64
+    rng = np.random.default_rng(7)
+    q, key, value, tokens = batch(rng, [(500, 460)] + [(40 + i, 1) for i in range(20)], heads, kvh, hd)
+    got = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
+    pick = [0, 200, 459] + list(range(460, 480))
+    want = reference(q[pick], key, value, [tokens[i] for i in pick], heads, kvh, hd)
+    assert rel_l2(got[pick], want) < TOL
+
+
+def test_later_rows_not_finite(qk, torch_gpu):
+    """Infinite or NaN values in a later token's row reach that token only."""
+    heads, kvh, hd = 24, 8, 128
+    rng = np.random.default_rng(8)
+    q, key, value, tokens = batch(rng, [(500, 500)], heads, kvh, hd)
+    clean = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
+    value[300, 5], value[421, hd + 7] = np.inf, np.nan
+    key[421, 3 * hd] = np.nan
+    got = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
+    assert rel_l2(got[:300], clean[:300]) < TOL
+    assert np.isfinite(got[:300]).all() and not np.isfinite(got[300:, 5]).any()
+    per_token = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd, split_rows=512)
+    assert np.array_equal(np.isfinite(got), np.isfinite(per_token))
+    assert rel_l2(got[np.isfinite(got)], per_token[np.isfinite(got)]) < TOL
