@@ -411,7 +411,9 @@ __device__ void merge_splits(const SplitAttnKernelArgs &ka, int b, int kvh, int 
     }
 }
 
-template <int G, int NF, int L, int NW>
+// TILED: tokens of shared tiles are left to tile_attention.  (An instance of
+// its own: the test alone cost the plain one 3 % at head_dim 128.)
+template <int G, int NF, int L, int NW, bool TILED>
 __global__ __launch_bounds__(NW * 64) void split_attention_kernel(SplitAttnKernelArgs ka) {
     constexpr int kSplitWaves = NW;
     constexpr int kSplitThreads = NW * 64;
@@ -440,7 +442,8 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(SplitAttnKerne
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = lane % L, rq = lane / L;
     const int hd = a.head_dim, hv = hd / 4, kv_dim = a.kv_heads * hd, half = hd / 2;
-    if (tile_token(ka, b)) return;
+    if constexpr (TILED)
+        if (tile_token(ka, b)) return;
     const qk_batch_token d = a.desc ? a.desc[b] : qk_batch_token{a.pos, 0, 0};
     float *o = a.out + static_cast<int64_t>(b) * a.heads * hd + kvh * G * hd;
     if (!token_ok(d, a.cache_rows, a.max_pos)) {
@@ -799,39 +802,40 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const float *pv, cons
 // G * head_dim <= 512, else 16; NF float4 per lane.  NULL when unsupported.
 // NW: waves per workgroup -- 4 for splits and for the one-split form that
 // needs no merge (section below).
-template <int G, int NF, int L, int NW>
+template <int G, int NF, int L, int NW, bool TILED>
 const void *split_fn() {
-    return reinterpret_cast<const void *>(split_attention_kernel<G, NF, L, NW>);
+    return reinterpret_cast<const void *>(split_attention_kernel<G, NF, L, NW, TILED>);
 }
 
-template <int G, int NW>
+template <int G, int NW, bool TILED>
 const void *split_for(int head_dim) {
     if (G * head_dim <= 512) {
-        if (head_dim <= 32) return split_fn<G, 1, 8, NW>();
-        if (head_dim == 64) return split_fn<G, 2, 8, NW>();
+        if constexpr (!TILED)
+            if (head_dim <= 32) return split_fn<G, 1, 8, NW, TILED>();
+        if (head_dim == 64) return split_fn<G, 2, 8, NW, TILED>();
         if constexpr (G <= 4)
-            if (head_dim == 128) return split_fn<G, 4, 8, NW>();
-        if constexpr (G <= 2)
-            if (head_dim == 256) return split_fn<G, 8, 8, NW>();
+            if (head_dim == 128) return split_fn<G, 4, 8, NW, TILED>();
+        if constexpr (G <= 2 && !TILED)
+            if (head_dim == 256) return split_fn<G, 8, 8, NW, TILED>();
         return nullptr;
     }
     if constexpr (G >= 6)
-        if (head_dim == 128) return split_fn<G, 2, 16, NW>();
-    if constexpr (G >= 3)
-        if (head_dim == 256) return split_fn<G, 4, 16, NW>();
+        if (head_dim == 128) return split_fn<G, 2, 16, NW, TILED>();
+    if constexpr (G >= 3 && !TILED)
+        if (head_dim == 256) return split_fn<G, 4, 16, NW, TILED>();
     return nullptr;
 }
 
-template <int NW>
+template <int NW, bool TILED>
 const void *split_instance_w(int G, int head_dim) {
     if (head_dim < 4 || head_dim % 4 || 256 % head_dim) return nullptr;
     switch (G) {
-        case 1: return split_for<1, NW>(head_dim);
-        case 2: return split_for<2, NW>(head_dim);
-        case 3: return split_for<3, NW>(head_dim);
-        case 4: return split_for<4, NW>(head_dim);
-        case 6: return split_for<6, NW>(head_dim);
-        case 8: return split_for<8, NW>(head_dim);
+        case 1: return split_for<1, NW, TILED>(head_dim);
+        case 2: return split_for<2, NW, TILED>(head_dim);
+        case 3: return split_for<3, NW, TILED>(head_dim);
+        case 4: return split_for<4, NW, TILED>(head_dim);
+        case 6: return split_for<6, NW, TILED>(head_dim);
+        case 8: return split_for<8, NW, TILED>(head_dim);
         default: return nullptr;
     }
 }
@@ -842,8 +846,11 @@ const void *split_instance_w(int G, int head_dim) {
 constexpr int kWideWaves = 4;
 
 const void *split_instance(int G, int head_dim, bool wide = false) {
-    return wide ? split_instance_w<kWideWaves>(G, head_dim) : split_instance_w<4>(G, head_dim);
+    return wide ? split_instance_w<kWideWaves, false>(G, head_dim) : split_instance_w<4, false>(G, head_dim);
 }
+
+// The instance that leaves shared tiles out (head_dim 64 and 128).
+const void *split_instance_tiled(int G, int head_dim) { return split_instance_w<4, true>(G, head_dim); }
 
 const void *split_merge_instance(int G) {
     switch (G) {
@@ -920,6 +927,7 @@ int launch_split_attention(const SplitAttention &a, int split_rows, void *worksp
     if (tile_mode) {
         if (int st = launch_tile_attention(a, stream)) return st;
         if (tile_mode == 2) return QK_OK;
+        fn = split_instance_tiled(G, a.head_dim);
     }
     const int max_rows = a.max_pos + 1;
     // Few (token, KV head) pairs over short rows: one wide workgroup each
@@ -929,7 +937,7 @@ int launch_split_attention(const SplitAttention &a, int split_rows, void *worksp
     // Each wide workgroup serves one query head (its KV head's rows are read
     // by G workgroups, mostly from cache), so the softmax arithmetic spreads
     // over heads CUs instead of kv_heads.
-    const bool wide = split_rows <= 0 && wide_attention(a);
+    const bool wide = split_rows <= 0 && !tile_mode && wide_attention(a);
     int head_split = 1, Gk = G;
     if (wide) {
         head_split = G;

@@ -352,18 +352,21 @@ bool tile_attention_supported(const SplitAttention &a) {
            (!a.gemm_rec || G * a.head_dim % 256 == 0) && (!a.q8_out || aligned(a.q8_out, 4));
 }
 
-// Whether 16-token tiles take less time than reading every token's rows: the
-// tile form walks ceil(rows / 32 / S) row tiles in 1.9 us per wave of a SIMD
-// at head_dim 128 (half that at 64), one workgroup per CU; the per-token form
-// reads all rows through L2 at about 20 TB/s.
+// Whether 16-token tiles take less time than reading every token's rows, both
+// estimated.  Tiles: rounds of one workgroup per CU, each walking ceil(rows /
+// 32 / S) row tiles in 2.4 us per wave of a SIMD at head_dim 128 (half that at
+// 64), and 12 us of launch, ramp and merge.  Per token: 6 ns a (token, KV
+// head) and the rows through L2 at 20 TB/s.  Both within a fifth of what 100
+// to 1024 tokens over 128 to 4096 rows measured on either layout, so the
+// tiles have to be a tenth shorter.
 bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int max_rows) {
     const int G = heads / kv_heads, S = tile_groups(G, head_dim);
     const int64_t wgs = static_cast<int64_t>((n_tokens + kAttnTile - 1) / kAttnTile) * kv_heads;
-    const double rounds = static_cast<double>((wgs + device_info().cus - 1) / device_info().cus);
-    const double per_tile = 1.9 * head_dim / 128. * (G * S + 3) / 4;
-    const double tile_us = rounds * ((max_rows + kKeys - 1) / kKeys + S - 1) / S * per_tile;
-    const double split_us = static_cast<double>(rows) * kv_heads * head_dim * 8. / 20e6;
-    return n_tokens >= kAttnTile / 2 && 1.2 * tile_us < split_us;
+    const int64_t rounds = (wgs + device_info().cus - 1) / device_info().cus;
+    const int64_t steps = ((max_rows + kKeys - 1) / kKeys + S - 1) / S;
+    const double tile_us = 12. + static_cast<double>(rounds * steps) * 2.4 * head_dim / 128. * ((G * S + 3) / 4);
+    const double split_us = 6e-3 * n_tokens * kv_heads + static_cast<double>(rows) * kv_heads * head_dim * 8. / 20e6;
+    return 1.1 * tile_us < split_us;
 }
 
 int tile_attention_mode(const qk_batch_token *desc, SplitAttention &a) {
