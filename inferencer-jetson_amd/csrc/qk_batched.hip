@@ -43,6 +43,7 @@
 //   reduce_splits     adds them in split order, so results are deterministic,
 //                     and applies the call's epilogue (one thread per output).
 #include "qk_internal.h"
+#include "qk_operands.h"
 #include "qk_records.h"
 
 #include <algorithm>
@@ -50,7 +51,6 @@
 namespace qk {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 
 constexpr int kMfmaMinTokens = 8;
@@ -222,8 +222,6 @@ __device__ __forceinline__ uint32_t word(const uint4 *v, int i) {
     return (i & 3) == 0 ? u.x : (i & 3) == 1 ? u.y : (i & 3) == 2 ? u.z : u.w;
 }
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
 // Bytes 0 and 2 (sel 0x04020400) or 1 and 3 (sel 0x04030401) of v as the
 // fp16 halves 0x64nn = 1024 + n, then fma(1024 + n, s, bias) with bias =
 // -(1024 + offset) * s: the exact product (n - offset) * s, rounded once.
@@ -297,11 +295,6 @@ __device__ __forceinline__ bool q6_scales_wide(const RawBlock &r) {
         w |= s > 62 || s < -62;
     }
     return w;
-}
-
-__device__ __forceinline__ _Float16 u8_to_h(uint32_t v) { return static_cast<_Float16>(static_cast<float>(v & 0xFFu)); }
-__device__ __forceinline__ _Float16 s8_to_h(uint32_t v) {
-    return static_cast<_Float16>(static_cast<float>(static_cast<int8_t>(v & 0xFFu)));
 }
 
 // Scale / bias operands of step j of block half hf for one row tile: the
@@ -987,6 +980,8 @@ int launch_batched_fused(const qk_matrix *mats, int n_mats, const float *x, int 
     if (n_tokens >= kMfmaMinTokens)
         return launch_mfma(mats, n_mats, ldy, x, ldx, cols, n_tokens, workspace, workspace_size, stream,
                            "fused batched GEMM", &f);
+    if (few_pays(mats, n_mats, cols, n_tokens, f.pair != 0))
+        return launch_few(mats, n_mats, x, ldx, cols, n_tokens, ldy, f, stream, "fused batched GEMM");
     return launch_gemv_fused(mats, n_mats, x, ldx, cols, n_tokens, ldy, f, stream);
 }
 
@@ -1010,6 +1005,9 @@ int qk_gemv_batched_f32(int type, const void *w, const float *x, int ldx, float 
     if (n_tokens >= qk::kMfmaMinTokens)
         return qk::launch_mfma(&m, 1, &ldy, x, ldx, cols, n_tokens, workspace, workspace_bytes,
                                static_cast<hipStream_t>(stream), "qk_gemv_batched_f32");
+    if (qk::few_pays(&m, 1, cols, n_tokens, false))
+        return qk::launch_few(&m, 1, x, ldx, cols, n_tokens, &ldy, qk::GemvFusion{}, static_cast<hipStream_t>(stream),
+                              "qk_gemv_batched_f32");
     return qk::launch_gemv_f32(&m, 1, x, ldx, cols, n_tokens, &ldy, static_cast<hipStream_t>(stream));
 }
 
@@ -1052,6 +1050,15 @@ int qk_ffn_batched_f32(int gate_type, const void *gate, int up_type, const void 
         float *u = reinterpret_cast<float *>(ws + qk::ffn_gemv_slot(hidden, n_tokens));
         const qk_matrix gu[2] = {{gate_type, hidden, gate, g}, {up_type, hidden, up, u}};
         const int ldg[2] = {hidden, hidden};
+        if (qk::few_pays(gu, 2, dim, n_tokens, true)) {
+            // SiLU(gate) * up from the pair's own epilogue; down over it.
+            qk::GemvFusion gf;
+            gf.pair = 1;
+            if ((st = qk::launch_few(gu, 2, x, ldx, dim, n_tokens, ldg, gf, s, where))) return st;
+            if (qk::few_pays(&dm, 1, hidden, n_tokens, false))
+                return qk::launch_few(&dm, 1, g, hidden, hidden, n_tokens, &ldy, df, s, where);
+            return qk::launch_gemv_fused(&dm, 1, g, hidden, hidden, n_tokens, &ldy, df, s);
+        }
         if ((st = qk::launch_gemv_f32(gu, 2, x, ldx, dim, n_tokens, ldg, s))) return st;
         df.up = u;
         return qk::launch_gemv_fused(&dm, 1, g, hidden, hidden, n_tokens, &ldy, df, s);
@@ -1089,6 +1096,9 @@ int qk_gemv_multi_batched_f32(const qk_matrix *mats, int n_mats, const float *x,
     if (n_tokens >= qk::kMfmaMinTokens)
         return qk::launch_mfma(mats, n_mats, ldy, x, ldx, cols, n_tokens, workspace, workspace_bytes,
                                static_cast<hipStream_t>(stream), "qk_gemv_multi_batched_f32");
+    if (qk::few_pays(mats, n_mats, cols, n_tokens, false))
+        return qk::launch_few(mats, n_mats, x, ldx, cols, n_tokens, ldy, qk::GemvFusion{},
+                              static_cast<hipStream_t>(stream), "qk_gemv_multi_batched_f32");
     return qk::launch_gemv_f32(mats, n_mats, x, ldx, cols, n_tokens, ldy, static_cast<hipStream_t>(stream));
 }
 

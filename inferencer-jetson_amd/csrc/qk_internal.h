@@ -271,6 +271,14 @@ size_t batched_chain_workspace_bytes(int cols, int rows_total, int n_tokens);
 size_t batched_records_bytes(int cols, int n_tokens);
 int launch_batched_fused(const qk_matrix *mats, int n_mats, const float *x, int ldx, int cols, int n_tokens,
                          const GemvFusion &f, void *workspace, size_t workspace_size, hipStream_t stream);
+// 2 to 7 tokens over matrices read and decoded once (csrc/qk_few.hip).
+// Arguments as launch_gemv_fused's, already validated; of the fusion norm_w,
+// up, accumulate, and pair (gate and up: y0 = SiLU(W0 x) * (W1 x), y1 unused).
+// Only for calls that few_pays accepts: it serves them in less time than the
+// GEMV kernels.
+bool few_pays(const qk_matrix *mats, int n_mats, int cols, int n_tokens, bool pair);
+int launch_few(const qk_matrix *mats, int n_mats, const float *x, int ldx, int cols, int n_tokens, const int *ldy,
+               const GemvFusion &f, hipStream_t stream, const char *where);
 // ------------------------------------------------ activation records --
 //
 // The FP32 GEMVs read activations as 64-byte records, one per 16 columns:

@@ -1353,9 +1353,14 @@ int qk_llama_batch_forward_rows(qk_llama_batch *m, const int32_t *tokens, const 
         const qk_matrix gu[2] = {{L.gate_type, c.hidden, L.gate, m->gate}, {L.up_type, c.hidden, L.up, m->up}};
         const qk_matrix down{L.down_type, dim, L.down, m->x};
         if (!chain) {
+            // From two tokens on the pair kernel forms SiLU(gate) * up itself
+            // where it is the shorter one.
+            qk::GemvFusion gu_in = ffn_in;
+            gu_in.pair = qk::few_pays(gu, 2, dim, T, true);
             if ((st = qk::launch_batched_fused(&o, 1, m->attn, dim, dim, T, residual, ws, wsb, s)) ||
-                (st = qk::launch_batched_fused(gu, 2, m->x, dim, dim, T, ffn_in, ws, wsb, s)) ||
-                (st = qk::launch_batched_fused(&down, 1, m->gate, c.hidden, c.hidden, T, down_in, ws, wsb, s)) ||
+                (st = qk::launch_batched_fused(gu, 2, m->x, dim, dim, T, gu_in, ws, wsb, s)) ||
+                (st = qk::launch_batched_fused(&down, 1, m->gate, c.hidden, c.hidden, T, gu_in.pair ? residual : down_in,
+                                               ws, wsb, s)) ||
                 (st = batch_trace_x(m, l, T, s)))
                 return st;
             continue;

@@ -25,6 +25,7 @@
 // (192 / 119 us: a barrier per 32 columns).
 #pragma once
 
+#include "qk_operands.h"
 #include "qk_records.h"
 
 #include <type_traits>
@@ -95,56 +96,6 @@ __device__ __forceinline__ uint4 load_header(const uint8_t *row, int b, int nb, 
         const uint2 sc = load8(f.sc + kh * 8);
         return make_uint4(sc.x, sc.y, load2(f.d), 0);
     }
-}
-
-__device__ __forceinline__ uint32_t quad_word(const uint4 &q, int i) {
-    return i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w;
-}
-
-__device__ __forceinline__ half2v h2(_Float16 v) { return half2v{v, v}; }
-
-// (v >> S) & mask as two 16-bit lanes OR'd onto 0x6400: the fp16 values 1024 +
-// bits (S negative shifts left).
-template <int S>
-__device__ __forceinline__ uint32_t shift_by(uint32_t v) {
-    if constexpr (S >= 0) return v >> S;
-    else return v << -S;
-}
-__device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
-__device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast(uint32_t, v); }
-
-// Eight Q4_K weights sc * q of one word: bytes (0, 2), (1, 3) low nibbles with
-// scale sa, then the high nibbles with sb, each fma(1024 + n, sa, -1024 sa) or
-// fma(1024 + 16 n, sb / 16, -64 sb), exact.
-__device__ __forceinline__ uint4 decode_q4(uint32_t w, half2v sa, half2v ba, half2v sb, half2v bb) {
-    const uint32_t w8 = w >> 8;
-    uint4 o;
-    o.x = as_u32(__builtin_elementwise_fma(as_h2((w & 0x000F000Fu) | 0x64006400u), sa, ba));
-    o.y = as_u32(__builtin_elementwise_fma(as_h2((w8 & 0x000F000Fu) | 0x64006400u), sa, ba));
-    o.z = as_u32(__builtin_elementwise_fma(as_h2((w & 0x00F000F0u) | 0x64006400u), sb, bb));
-    o.w = as_u32(__builtin_elementwise_fma(as_h2((w8 & 0x00F000F0u) | 0x64006400u), sb, bb));
-    return o;
-}
-
-// One pair of Q6_K weights: 6-bit code = low 4 bits of lo >> SL, 2 bits of
-// hq >> SH; a = fp16(s * (code - 32)), b the exact residual.
-template <int SL, int SH>
-__device__ __forceinline__ void decode_q6_pair(uint32_t lo, uint32_t hq, half2v s, uint32_t &a, uint32_t &b) {
-    const uint32_t n = (shift_by<SL>(lo) & 0x000F000Fu) | 0x64006400u;
-    const uint32_t v = (shift_by<SH - 4>(hq) & 0x00300030u) | n;
-    const half2v c = as_h2(v) + h2(static_cast<_Float16>(-1056.f));   // 1024 + code - 1056
-    const half2v w = c * s;
-    a = as_u32(w);
-    b = as_u32(__builtin_elementwise_fma(c, s, -w));
-}
-
-template <int HF>
-__device__ __forceinline__ void decode_q6(uint32_t la, uint32_t lb, uint32_t hq, half2v sa, half2v sb, uint4 &a,
-                                          uint4 &b) {
-    decode_q6_pair<4 * HF, 4 * HF>(la, hq, sa, a.x, b.x);
-    decode_q6_pair<4 * HF + 8, 4 * HF + 8>(la, hq, sa, a.y, b.y);
-    decode_q6_pair<4 * HF, 4 * HF + 2>(lb, hq, sb, a.z, b.z);
-    decode_q6_pair<4 * HF + 8, 4 * HF + 10>(lb, hq, sb, a.w, b.w);
 }
 
 // Scale operands of one half: Q4_K sub-blocks 2 kh + h's low and high nibbles
