@@ -188,6 +188,16 @@ int launch_skinny_i8(const qk_matrix *mats, int n_mats, const int *ldy, const in
                      float *out_xs, int out_ldxq, int out_ldxs, void *workspace, size_t workspace_size,
                      hipStream_t stream, const char *where, const SkNorm *norm = nullptr,
                      SkDeferred *defer = nullptr);
+// The same product of many tokens on the fp16 matrix cores
+// (csrc/qk_tile_i8.hip).  tile_i8_splits: the splits of the rows (their sums
+// within workspace_size bytes), or 0 where launch_skinny_i8's own kernels are
+// the better choice.  Matrices of one type; out_xq 4-byte aligned, out_ldxq a
+// multiple of 4.
+int tile_i8_splits(const qk_matrix *mats, int n_mats, int cols, int n_tokens, int ldxq, int ldscale, bool pair,
+                   size_t workspace_size);
+int launch_tile_i8(int splits, const qk_matrix *mats, int n_mats, const int *ldy, const int8_t *xq, int ldxq,
+                   const float *xscale, int ldscale, int cols, int n_tokens, int accumulate, int8_t *out_xq,
+                   float *out_xs, int out_ldxq, int out_ldxs, void *workspace, hipStream_t stream, const char *where);
 // SiLU(gate) * up quantized per 32 values straight into xq / xscale (n a
 // multiple of 32): bit-identical to qk_silu_mul_f32 then qk_quantize_x32,
 // without the fp32 product written.  Arguments already validated.

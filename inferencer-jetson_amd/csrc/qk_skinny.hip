@@ -928,6 +928,19 @@ int launch_skinny_i8(const qk_matrix *mats, int n_mats, const int *ldy, const in
         if (!aligned(workspace, 16)) return fail(QK_ERR_ALIGN, std::string(where) + ": workspace not 16-byte aligned");
         p.partials = static_cast<float *>(workspace);
     }
+    // What would walk row tiles with skinny_i8_loop goes to the fp16 matrix
+    // cores where that fills the chip (qk_tile_i8.hip: a 3B feed-forward block
+    // of 517 tokens 402 -> 233 us, of 96 89 -> 77 us).  Launches of one round,
+    // and rows short enough for skinny_i8_rows, are as fast or faster here
+    // (Q4_K 16384 x 2048 on 256 tokens 47 against 42 us, on 64 26 against 26;
+    // 2048 x 2048 on 256 tokens 12 against 20).
+    if (plan.loop_groups && !plan.rows && (!pair || (aligned(out_xq, 4) && out_ldxq % 4 == 0))) {
+        const int splits = tile_i8_splits(mats, n_mats, cols, n_tokens, ldxq, ldscale, pair,
+                                          workspace && aligned(workspace, 16) ? workspace_size : 0);
+        if (splits)
+            return launch_tile_i8(splits, mats, n_mats, ldy, xq, ldxq, xscale, ldscale, cols, n_tokens, accumulate,
+                                  out_xq, out_xs, out_ldxq, out_ldxs, workspace, stream, where);
+    }
     const size_t lds = plan.rows ? rows_lds(nb) : skinny_lds(p.waves, rt);
     const int groups = plan.loop_groups ? plan.loop_groups : tiles;   // workgroups per (split, token tile)
     void *args[] = {&p};

@@ -1,0 +1,89 @@
+"""INT8 products of more (row tile, token tile) units than the chip holds at
+once (csrc/qk_tile_i8.hip): ragged token and row tiles, split rows, the gate /
+up pair, accumulation, strided inputs and outputs, and a workspace too small
+for the planned splits.
+
+Integer blocks (d = dmin = 1) with unit scales make every partial sum an exact
+integer below 2^24, so the outputs equal an int64 product bit for bit; random
+blocks are compared with the fp64 combine.  Its bar: an output adds K / 32
+products of fp32 operands, each rounded a few times, so the relative error of
+the whole is below about sqrt(K / 32) * 2^-24 * a small factor: 1e-5 as for the
+integer matrix cores."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2, to_dev
+from test_gpu_int8_matrix_core import Q4_K, Q6_K, _integer_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def _dense(t, qk, qtype, w, cols, rows):
+    out = t.empty((rows, cols), device="cuda")
+    wd = to_dev(t, w)
+    qk.check(qk.lib().qk_dequant_rows(qtype, wd.data_ptr(), out.data_ptr(), cols, 0, rows, None), "dequant")
+    t.cuda.synchronize()
+    return out.cpu().double()
+
+
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K])
+@pytest.mark.parametrize("cols,rows,ntok", [(5632, 2050, 300), (8192, 1055, 545), (4096, 4096, 161)])
+def test_exact_ragged(qk, torch_gpu, synth, qtype, cols, rows, ntok):
+    t = torch_gpu
+    w = _integer_blocks(qtype, synth.quant_matrix(qtype, cols, rows, 5, 1), cols, rows)
+    dense = _dense(t, qk, qtype, w, cols, rows)
+    g = t.Generator().manual_seed(3)
+    ldxq, ldsc, ldy = cols + 32, cols // 32 + 3, rows + 5
+    # Small codes keep whole sums below 2^24 (scale * code <= 4096).
+    xq = t.randint(-1, 2, (ntok, ldxq), generator=g, dtype=t.int8)
+    xq *= (t.rand(ntok, ldxq, generator=g) < 0.1).to(t.int8)
+    want = xq[:, :cols].double() @ dense.T
+    assert want.abs().max() < 2 ** 24
+    L = qk.lib()
+    n = L.qk_gemv_batched_i8_workspace_bytes(cols, rows, ntok)
+    ws = t.empty(n, dtype=t.uint8, device="cuda")
+    wd, xd, xs = to_dev(t, w), xq.cuda(), t.ones(ntok, ldsc, device="cuda")
+    y = t.full((ntok, ldy), 7.0, device="cuda")
+    qk.check(L.qk_gemv_batched_i8(qtype, wd.data_ptr(), xd.data_ptr(), ldxq, xs.data_ptr(), ldsc, y.data_ptr(), ldy,
+                                  cols, rows, ntok, ws.data_ptr(), n, None), "batched INT8")
+    t.cuda.synchronize()
+    got = y.cpu().double()
+    assert (got[:, :rows] == want).all()
+    assert (got[:, rows:] == 7.0).all()
+
+
+@pytest.mark.parametrize("down", [Q4_K, Q6_K])
+@pytest.mark.parametrize("dim,hidden,ntok", [(2048, 5632, 97), (3072, 8192, 200), (1024, 2816, 517)])
+def test_ffn(qk, torch_gpu, synth, down, dim, hidden, ntok):
+    t = torch_gpu
+    ws = [synth.quant_matrix(Q4_K, dim, hidden, 9, i) for i in (1, 2)]
+    ws.append(synth.quant_matrix(down, hidden, dim, 9, 3))
+    g, u = (_dense(t, qk, Q4_K, ws[i], dim, hidden) for i in (0, 1))
+    d = _dense(t, qk, down, ws[2], hidden, dim)
+    gen = t.Generator().manual_seed(11)
+    xq = t.randint(-128, 128, (ntok, dim), generator=gen, dtype=t.int8)
+    xs = t.rand(ntok, dim // 32, generator=gen) * 2e-4 + 1e-5
+    x = xq.double() * xs.double().repeat_interleave(32, 1)
+    a = x @ g.T
+    h = (a / (1 + t.exp(-a)) * (x @ u.T)).view(ntok, hidden // 32, 32)
+    scale = (h.abs().amax(2, keepdim=True) / 127).float().double()
+    scale = t.where(scale > 0, scale, t.ones_like(scale))
+    hq = (t.round(h / scale).clamp(-127, 127) * scale).view(ntok, hidden)
+    y0 = t.randn(ntok, dim, generator=gen)
+    want = hq @ d.T
+    L = qk.lib()
+    n = L.qk_ffn_batched_i8_workspace_bytes(dim, hidden, ntok)
+    dev = [to_dev(t, w) for w in ws]
+    xd, sd, work = xq.cuda(), xs.cuda(), t.empty(n, dtype=t.uint8, device="cuda")
+    for accumulate in (0, 1):
+        y = y0.cuda()
+        qk.check(L.qk_ffn_batched_i8(Q4_K, dev[0].data_ptr(), Q4_K, dev[1].data_ptr(), down, dev[2].data_ptr(),
+                                     xd.data_ptr(), dim, sd.data_ptr(), dim // 32, y.data_ptr(), dim, dim, hidden, ntok,
+                                     accumulate, work.data_ptr(), n, None), "INT8 FFN")
+        t.cuda.synchronize()
+        ref = want + y0.double() if accumulate else want
+        # h in fp32 is off by some 2^-20 of itself, so a share of about
+        # 127 * 2^-20 of the codes rounds the other way, by 1 / 127 of the
+        # group's peak (some three times its RMS): sqrt(127 * 2^-20) * 3 / 127
+        # = 2.6e-4 of the whole.
+        assert rel_l2(y.cpu().numpy(), ref.numpy()) < 5e-4
