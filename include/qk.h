@@ -148,8 +148,10 @@ int qk_gemv_multi_batched_f32(const qk_matrix *mats, int n_mats, const float *x,
    1362-1380) with FP32 semantics.  From 8 tokens on it runs as five
    launches on the matrix cores: the gate / up reduction packs SiLU(gate) *
    up straight into the down projection's input records, so neither gate,
-   up nor their product is stored as fp32; below 8 tokens, the fused GEMV
-   pair of qk_gemv_multi_f32 and a down GEMV staging SiLU * up.  workspace:
+   up nor their product is stored as fp32; below 8 tokens, a gate / up
+   launch that writes SiLU * up (2 to 7 tokens of like gate and up: one read
+   of the weights on the matrix cores; otherwise the fused GEMV pair) and a
+   down launch.  workspace:
    qk_ffn_batched_workspace_bytes(dim, hidden, n_tokens) bytes (256-byte
    aligned; also enough for fewer tokens), not shared by calls in flight at
    the same time.  dim and hidden multiples of 256.  No reference
@@ -249,7 +251,10 @@ int qk_gemv_i8(int type, const void *w, const int8_t *xq, int ldxq, const float 
    wave.  Each launch's plan, chosen from the kernels' occupancy on the
    device, may split rows over workgroups, whose sums a second launch adds
    in split order (deterministic), and a launch larger than the chip holds
-   at once lets resident workgroups walk the row tiles.  The workspace
+   at once lets resident workgroups walk the row tiles or, with enough
+   tokens, takes 128 rows x 64 tokens a workgroup with the integer scales
+   folded into fp16 operands (the same exact sub-block sums, scaled per 32
+   columns and then by d).  The workspace
    holds the split sums of any plan:
    qk_gemv_batched_i8_workspace_bytes(cols, rows, n_tokens) bytes, 16-byte
    aligned (0, and NULL allowed, below 8 tokens or at 256 columns; a plan

@@ -5,9 +5,10 @@
 // 678-699; qkv_batch_cuda / gate_up_batch_cuda, inferencer.cu:701-751).
 // Token t reads x + t*ldx and writes y + t*ldy.
 //
-// Few tokens (< kMfmaMinTokens) run the batch-1 GEMV kernels with one grid
-// column per token.  From kMfmaMinTokens on, the product is a dense
-// contraction and runs on the matrix cores:
+// Few tokens (< kMfmaMinTokens) run qk_few.hip's kernel where few_pays says so,
+// else the batch-1 GEMV kernels with one grid column per token.  From
+// kMfmaMinTokens on, the product is a dense contraction and runs on the matrix
+// cores:
 //
 //   Y[t][r] = sum_b d_rb * sum_{c in b} W_int[r][c] * x[t][c]
 //             - dmin_rb * sum_j m_rbj * X[t][b][j]          (Q4_K only)

@@ -547,7 +547,8 @@ __device__ __forceinline__ TokenTile token_tile(const qk_batch_token *desc, int 
 // holding every row); takes less time than the per-token form for n_tokens
 // tokens of `rows` rows in all, the longest max_rows; runs.
 bool tile_attention_supported(const SplitAttention &a);
-bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int max_rows);
+bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int64_t max_rows,
+                         bool two_runs);
 int launch_tile_attention(const SplitAttention &a, hipStream_t stream);
 // SplitAttention::tile_mode of a batch whose descriptors the host holds
 // (valid ones): by the tiles' own test, when it pays.  Sets a.rows_hint to

@@ -26,7 +26,8 @@
 // workgroup applies the epilogue itself -- store, residual add, or SiLU(gate)
 // * up quantized per 32 values for the next product (silu_cuda then
 // quantize_batch_cuda, inferencer.cu:1053-1057, 891-904) -- so the call
-// needs no workspace and no reduction launch.
+// needs no workspace and no reduction launch.  Launches of more tiles than the
+// chip holds at once go to qk_tile_i8.hip where that is the faster form.
 #include "qk_internal.h"
 
 #include <algorithm>
@@ -930,10 +931,11 @@ int launch_skinny_i8(const qk_matrix *mats, int n_mats, const int *ldy, const in
     }
     // What would walk row tiles with skinny_i8_loop goes to the fp16 matrix
     // cores where that fills the chip (qk_tile_i8.hip: a 3B feed-forward block
-    // of 517 tokens 402 -> 233 us, of 96 89 -> 77 us).  Launches of one round,
-    // and rows short enough for skinny_i8_rows, are as fast or faster here
-    // (Q4_K 16384 x 2048 on 256 tokens 47 against 42 us, on 64 26 against 26;
-    // 2048 x 2048 on 256 tokens 12 against 20).
+    // of 517 tokens 402 -> 233 us, of 96 89 -> 77 us).  Launches of one round
+    // are faster here (Q4_K 2048 x 2048 on 256 tokens 12 against 20 us); of
+    // those skinny_i8_rows serves some are slower here (Q4_K 16384 x 2048 on
+    // 256 tokens 47 against 42) and some faster (5120 x 3072, 36 against 39;
+    // split or short Q6_K 512 x 2048 on 517, 17 against 18), so they stay.
     if (plan.loop_groups && !plan.rows && (!pair || (aligned(out_xq, 4) && out_ldxq % 4 == 0))) {
         const int splits = tile_i8_splits(mats, n_mats, cols, n_tokens, ldxq, ldscale, pair,
                                           workspace && aligned(workspace, 16) ? workspace_size : 0);

@@ -358,39 +358,49 @@ bool tile_attention_supported(const SplitAttention &a) {
 // 64), and 12 us of launch, ramp and merge.  Per token: 6 ns a (token, KV
 // head) and the rows through L2 at 20 TB/s.  Both within a fifth of what 100
 // to 1024 tokens over 128 to 4096 rows measured on either layout, so the
-// tiles have to be a tenth shorter.
-bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int max_rows) {
+// tiles have to be a tenth shorter.  One query head a KV head leaves a SIMD one
+// wave, 3.7 us a step.  Where tiles may hold two runs, the second one's start
+// adds 12 us and the margin is three tenths (8 heads of 128, 4 x 58 tokens over
+// 450 rows: 34.5 us per token, 53 in tiles).
+bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int64_t max_rows,
+                         bool two_runs) {
     const int G = heads / kv_heads, S = tile_groups(G, head_dim);
     const int64_t wgs = static_cast<int64_t>((n_tokens + kAttnTile - 1) / kAttnTile) * kv_heads;
     const int64_t rounds = (wgs + device_info().cus - 1) / device_info().cus;
     const int64_t steps = ((max_rows + kKeys - 1) / kKeys + S - 1) / S;
-    const double tile_us = 12. + static_cast<double>(rounds * steps) * 2.4 * head_dim / 128. * ((G * S + 3) / 4);
+    const double step_us = std::max(3.7, 2.4 * ((G * S + 3) / 4)) * head_dim / 128.;
+    const double tile_us = (two_runs ? 24. : 12.) + static_cast<double>(rounds * steps) * step_us;
     const double split_us = 6e-3 * n_tokens * kv_heads + static_cast<double>(rows) * kv_heads * head_dim * 8. / 20e6;
-    return 1.1 * tile_us < split_us;
+    return (two_runs ? 1.3 : 1.1) * tile_us < split_us;
 }
 
 int tile_attention_mode(const qk_batch_token *desc, SplitAttention &a) {
     if (!tile_attention_supported(a)) return 0;
-    int64_t tiled_rows = 0, rows = 0;
-    int tiled = 0, max_rows = 0;
+    int64_t tiled_rows = 0, rows = 0, max_rows = 0;
+    int tiled = 0;
+    bool two_runs = false;
     for (int t0 = 0; t0 < a.n_tokens; t0 += kAttnTile) {
         const int t1 = std::min(t0 + kAttnTile, a.n_tokens);
-        int runs = 0, longest = 0;
+        int runs = 0;
+        int64_t walked = 0;   // rows the tile's workgroup walks: each run's last position
         int64_t tile_rows = 0;
         for (int t = t0; t < t1; ++t) {
             runs += t == t0 || desc[t].kv_row != desc[t - 1].kv_row || desc[t].pos != desc[t - 1].pos + 1;
             tile_rows += desc[t].pos + 1;
-            longest = std::max(longest, desc[t].pos + 1);
+            if (t + 1 == t1 || desc[t + 1].kv_row != desc[t].kv_row || desc[t + 1].pos != desc[t].pos + 1)
+                walked += desc[t].pos + 1;
         }
         if (runs <= kMaxRuns) {
             tiled += t1 - t0;
             tiled_rows += tile_rows;
-            max_rows = std::max(max_rows, longest);
+            max_rows = std::max(max_rows, walked);
+            two_runs |= runs > 1;
         } else {
             rows += tile_rows;
         }
     }
-    if (!tiled || !tile_attention_pays(tiled, a.kv_heads, a.heads, a.head_dim, tiled_rows, max_rows)) return 0;
+    if (!tiled || !tile_attention_pays(tiled, a.kv_heads, a.heads, a.head_dim, tiled_rows, max_rows, two_runs))
+        return 0;
     if (tiled == a.n_tokens) return 2;
     a.rows_hint = rows;
     return 1;
