@@ -931,7 +931,7 @@ int launch_skinny_i8(const qk_matrix *mats, int n_mats, const int *ldy, const in
     }
     // What would walk row tiles with skinny_i8_loop goes to the fp16 matrix
     // cores where that fills the chip (qk_tile_i8.hip: a 3B feed-forward block
-    // of 517 tokens 402 -> 233 us, of 96 89 -> 77 us).  Launches of one round
+    // of 517 tokens 402 -> 226 us, of 96 89 -> 77 us).  Launches of one round
     // are faster here (Q4_K 2048 x 2048 on 256 tokens 12 against 20 us); of
     // those skinny_i8_rows serves some are slower here (Q4_K 16384 x 2048 on
     // 256 tokens 47 against 42) and some faster (5120 x 3072, 36 against 39;

@@ -26,11 +26,19 @@
 // against 3.0 us of VALU work: what is left is the wait for weights and the
 // barrier of each half.
 //
+// Sums: a Q4_K block's dots and mins are added to each other before they
+// enter the running sum (1.55e-7 of float64 over 16 blocks, 1.6e-7 over 32;
+// the int32 kernels 1.62 and 1.65e-7; with every min product entering the
+// running sum on its own 2.0 and 2.2 to 3.3e-7), and sums of many blocks have
+// two levels (kShortBlocks).
+//
 // Measured against the looping int32 kernel: a 3B feed-forward block (gate /
-// up 8192 x 3072 Q4_K, down 3072 x 8192 Q6_K split) on 517 tokens 400 -> 234
-// us, its down product alone 163 -> 99 us.  Tried: two row tiles a wave (two
-// waves a SIMD, spills: 298 us) and no step of dots ahead of the combine (256
-// us).
+// up 8192 x 3072 Q4_K, down 3072 x 8192 Q6_K split) on 517 tokens 402 -> 226
+// us, its down product alone 165 -> 97 us; Q4_K 8192 x 8192 on 1000 tokens 452
+// -> 278 us.  Tried: two row tiles a wave (two waves a SIMD, spills: 298 us),
+// no step of dots ahead of the combine (256 us), the mins on the bf16 matrix
+// instructions in three exact parts (4 to 19 % more: the splitting), and two
+// levels of sums at every length (2 to 5 % more).
 #include "qk_operands.h"
 
 #include <algorithm>
@@ -70,9 +78,22 @@ struct TiParams {
     int out_ldxq, out_ldxs;
 };
 
-// LDS: two halves' operands, their activation scales and scale * sum products
-// ([half][tile][sub-block][token] each), then d of the waves' rows.
-__host__ __device__ constexpr int ti_lds(int tt) { return 2 * tt * kHalfTile + 2 * 2 * tt * 4 * kTok * 4 + 4 * kRowTile * 4; }
+// LDS: two halves' operands, their activation scales ([half][tile][sub-block]
+// [token]), three halves' scale * sum products (the same; a block's two are read
+// when it ends, while the next one's first are written: those of first halves
+// alternate, slots 0 and 1, second halves take slot 2), then d of the waves' rows.
+__host__ __device__ constexpr int ti_lds(int tt) {
+    return 2 * tt * kHalfTile + (2 + 3) * tt * 4 * kTok * 4 + 4 * kRowTile * 4;
+}
+
+// A lane's 32-bit offset from a wave-uniform base, kept in that form: the
+// compiler otherwise carries 64-bit lane pointers through the loop, spills
+// some and waits for the weights in flight when it reloads them.
+__device__ __forceinline__ uint32_t lane_offset(uint32_t lane, uint32_t uniform) {
+    uint32_t o = lane + uniform;
+    asm("" : "+v"(o));
+    return o;
+}
 
 // Half h (sub-blocks 4h .. 4h + 3) of the lane's row, column half kh of each
 // sub-block (columns 16 kh .. + 15).  Q4_K: qs of groups 2h, 2h + 1 (low and
@@ -86,9 +107,9 @@ __device__ __forceinline__ RawI8<TYPE == QK_TYPE_Q4_K> load_half(const uint8_t *
                                                                     int kh, int h) {
     RawI8<TYPE == QK_TYPE_Q4_K> r;
     if constexpr (TYPE == QK_TYPE_Q4_K) {
-        const uint8_t *p = base + static_cast<size_t>(b) * 144 + 16 + 64 * h;
-        r.q[0] = load16(p + (ofs + 16 * kh));
-        r.q[1] = load16(p + 32 + (ofs + 16 * kh));
+        const uint32_t o = lane_offset(ofs + 16 * kh, b * 144);
+        r.q[0] = load16(base + o + (16 + 64 * h));
+        r.q[1] = load16(base + o + (48 + 64 * h));
     } else {
         const Q6Fields f = q6_fields(base, nb, b, TYPE == QK_TYPE_Q6_K_SPLIT);
         r.q[0] = load16(f.ql + 64 * h + (ofs + 16 * kh));
@@ -106,7 +127,7 @@ struct Header {
 template <int TYPE>
 __device__ __forceinline__ Header load_header(const uint8_t *base, uint32_t ofs, int b, int nb) {
     if constexpr (TYPE == QK_TYPE_Q4_K) {
-        return {load16(base + static_cast<size_t>(b) * 144 + ofs), 0};
+        return {load16(base + lane_offset(ofs, b * 144)), 0};
     } else {
         const Q6Fields f = q6_fields(base, nb, b, TYPE == QK_TYPE_Q6_K_SPLIT);
         return {load16(f.sc + ofs), load2(f.d + ofs)};
@@ -160,17 +181,27 @@ __device__ __forceinline__ uint2 codes_to_h(uint32_t v) {
                       as_u32(as_h2(((x >> 8) & 0x00FF00FFu) | 0x64006400u) + o));
 }
 
+// Blocks that one running sum takes in the short form: up to these, its error
+// against 64 bits is not above the int32 kernels' (1.65e-7 at 32 Q4_K blocks in
+// two sums of 16; 9.2e-8 for Q6_K, whose 16-block sums reach 9.7e-8).  The long
+// form keeps a second level, every kRun blocks added to a total: 1.6e-7 and
+// 9.4e-8 up to 96 blocks, at two workgroups a CU (registers).
+template <int TYPE>
+constexpr int kShortBlocks = TYPE == QK_TYPE_Q4_K ? 16 : 12;
+constexpr int kRun = 8;
+
 // One workgroup: TT token tiles from tile0 (all exist) x its rows x the
 // blocks of a split.
-template <int TYPE, int TT, bool PAIR>
+template <int TYPE, int TT, bool PAIR, bool LONG>
 __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, int row0, int tile0, int split,
                                           unsigned char *lds) {
     constexpr bool Q4 = TYPE == QK_TYPE_Q4_K;
     const int lane = threadIdx.x & 63, kh = lane >> 5, col = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float *const scales = reinterpret_cast<float *>(lds + 2 * TT * kHalfTile);   // [half][tile][4][32]
-    float *const sums = scales + 2 * TT * 4 * kTok;                              // the same, scale * sum of codes
-    float *const drow = sums + 2 * TT * 4 * kTok + wave * kRowTile;              // d of the wave's rows
+    constexpr int kPlane = TT * 4 * kTok;                                        // one half's
+    float *const sums = scales + 2 * kPlane;                                     // [slot][tile][4][32], scale * sum of codes
+    float *const drow = sums + 3 * kPlane + wave * kRowTile;                     // d of the wave's rows
     // Rows past the matrix read its last row (and store nothing).
     // A pair's waves 0, 1 take the gate rows, 2, 3 the same rows of up.  Lane
     // addresses: a wave-uniform base and a 32-bit offset.
@@ -198,7 +229,7 @@ __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, 
             cs[u] = (xs + b * 8 + h * 4)[tofs[u] * static_cast<uint32_t>(p.ldxs)];
         }
     };
-    auto commit = [&](int h) {
+    auto commit = [&](int block, int h) {
         #pragma unroll
         for (int u = 0; u < TT; ++u) {
             unsigned char *dst = lds + (h * TT + u) * kHalfTile + wave * 2048 + lane * 16;
@@ -206,17 +237,16 @@ __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, 
             const uint2 c = codes_to_h(codes[u].z), d = codes_to_h(codes[u].w);
             *reinterpret_cast<uint4 *>(dst) = make_uint4(a.x, a.y, b.x, b.y);
             *reinterpret_cast<uint4 *>(dst + 1024) = make_uint4(c.x, c.y, d.x, d.y);
-            float *to = scales + ((h * TT + u) * 4 + wave) * kTok + col;
+            // (Both column halves write the same values.)
+            float *const at = scales + wave * kTok + col + u * 4 * kTok;
+            at[h * kPlane] = cs[u];
             if constexpr (Q4) {
                 int sum = __builtin_amdgcn_sdot4(static_cast<int>(codes[u].x), 0x01010101, 0, false);
                 sum = __builtin_amdgcn_sdot4(static_cast<int>(codes[u].y), 0x01010101, sum, false);
                 sum = __builtin_amdgcn_sdot4(static_cast<int>(codes[u].z), 0x01010101, sum, false);
                 sum = __builtin_amdgcn_sdot4(static_cast<int>(codes[u].w), 0x01010101, sum, false);
                 sum += __shfl_xor(sum, 32);
-                // Column half 0 stores the scale, half 1 the product.
-                to[kh * 2 * TT * 4 * kTok] = kh ? static_cast<float>(sum) * cs[u] : cs[u];
-            } else {
-                *to = cs[u];
+                at[(2 + (h ? 2 : block & 1)) * kPlane] = static_cast<float>(sum) * cs[u];
             }
         }
     };
@@ -227,41 +257,35 @@ __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, 
     float16v acc[TT], blk[TT];
     #pragma unroll
     for (int u = 0; u < TT; ++u) acc[u] = blk[u] = zero;
+    float16v total[LONG ? TT : 1];
+    if constexpr (LONG)
+        #pragma unroll
+        for (int u = 0; u < TT; ++u) total[u] = zero;
 
     request(b0, 0);
     Header hdr = load_header<TYPE>(wbase, wofs, b0, p.nb);
     RawI8<Q4> cur = load_half<TYPE>(wbase, wofs, b0, p.nb, kh, 0);
-    commit(0);
+    commit(b0, 0);
     __syncthreads();
     for (int b = b0; b < b1; ++b) {
         const int bn = min(b + 1, b1 - 1);   // the last block requests itself again (in bounds)
         Header hdr_next = hdr;
+        uint32_t mn4[2];   // Q4_K: the halves' mins
         #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const RawI8<Q4> next = load_half<TYPE>(wbase, wofs, h ? bn : b, p.nb, kh, h ^ 1);
             if (h) hdr_next = load_header<TYPE>(wbase, wofs, bn, p.nb);
             __builtin_amdgcn_sched_barrier(0);
-            uint32_t sc4, mn4 = 0;   // Q4_K: the half's scales and mins; Q6_K: column half kh's scales
+            uint32_t sc4;   // Q4_K: the half's scales; Q6_K: column half kh's
             if constexpr (Q4) {
-                q4k_scale_min4(hdr.v, h, sc4, mn4);
+                q4k_scale_min4(hdr.v, h, sc4, mn4[h]);
             } else {
                 const uint32_t lo = h ? hdr.v.z : hdr.v.x, hi = h ? hdr.v.w : hdr.v.y;
                 sc4 = __builtin_amdgcn_perm(hi, lo, kh ? 0x07050301u : 0x06040200u);
             }
             if (h == 0) drow[col] = f16_bits_to_f32(Q4 ? hdr.v.x & 0xFFFFu : hdr.d);
             const unsigned char *op = lds + h * TT * kHalfTile + lane * 16;
-            const float *sx = scales + h * TT * 4 * kTok + col, *sp = sums + h * TT * 4 * kTok + col;
-            if constexpr (Q4) {
-                // acc -= dmin m (scale * sum) over the half's sub-blocks, fp32.
-                #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const float m = static_cast<float>((mn4 >> (16 * j + 8 * kh)) & 0xFFu);
-                    const float am = -f16_bits_to_f32(hdr.v.x >> 16) * m;
-                    #pragma unroll
-                    for (int u = 0; u < TT; ++u)
-                        acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(am, sp[(u * 4 + 2 * j + kh) * kTok], acc[u], 0, 0, 0);
-                }
-            }
+            const float *sx = scales + h * kPlane + col;
             // Each Q4_K step issues one tile's dots, then combines the step
             // before's; Q6_K has the registers for one tile's only.
             half8 w[2], wb[2];
@@ -297,6 +321,16 @@ __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, 
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (h == 1) {
+                // Both halves' sums are still in LDS; dmin m of the lane's row,
+                // sub-blocks 2 j + kh.
+                float am[4];
+                const float *const sl = sums + (b & 1) * kPlane + lane, *const sh = sums + 2 * kPlane + lane;
+                if constexpr (Q4) {
+                    const float dmin = -f16_bits_to_f32(hdr.v.x >> 16);
+                    #pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        am[j] = dmin * static_cast<float>((mn4[j >> 1] >> (16 * (j & 1) + 8 * kh)) & 0xFFu);
+                }
                 float d[16];
                 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
@@ -306,16 +340,40 @@ __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, 
                     d[4 * q + 2] = v.z;
                     d[4 * q + 3] = v.w;
                 }
+                // The block's mins -- the fp32 product of dmin m and scale *
+                // sum over its eight sub-blocks -- and its dots meet first:
+                // each is about twice their sum, so the running sum takes
+                // one rounding a block, of the block's own size.
+                float16v tm[TT];
+                if constexpr (Q4) {
+                    #pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        #pragma unroll
+                        for (int u = 0; u < TT; ++u)
+                            tm[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                am[j], (j >> 1 ? sh : sl)[(u * 4 + 2 * (j & 1)) * kTok], j ? tm[u] : zero, 0, 0, 0);
+                }
                 #pragma unroll
                 for (int u = 0; u < TT; ++u)
                     #pragma unroll
-                    for (int k = 0; k < 16; ++k) acc[u][k] = fmaf(d[k], blk[u][k], acc[u][k]);
+                    for (int k = 0; k < 16; ++k)
+                        acc[u][k] = Q4 ? acc[u][k] + fmaf(d[k], blk[u][k], tm[u][k]) : fmaf(d[k], blk[u][k], acc[u][k]);
             }
-            commit(h ^ 1);
+            commit(h ? b + 1 : b, h ^ 1);
             __syncthreads();
             cur = next;
         }
         hdr = hdr_next;
+        if constexpr (LONG) {
+            const bool ends = b + 1 == b1;
+            if ((b - b0) % kRun == kRun - 1 || ends) {
+                #pragma unroll
+                for (int u = 0; u < TT; ++u) {
+                    total[u] += acc[u];
+                    acc[u] = ends ? total[u] : zero;
+                }
+            }
+        }
     }
 
     if constexpr (PAIR) {
@@ -401,8 +459,8 @@ __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, 
 // Consecutive workgroups go to the eight XCDs in turn: item (w % 8) *
 // ceil(n / 8) + w / 8 of a list in which the token groups of one row group are
 // neighbours, so they share its weight bytes in one XCD's L2.
-template <int TYPE, bool PAIR>
-__global__ __launch_bounds__(256, 3) void tile_i8(TiParams p) {
+template <int TYPE, bool PAIR, bool LONG>
+__global__ __launch_bounds__(256, LONG ? 2 : 3) void tile_i8(TiParams p) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int total = p.groups * p.tgroups * p.splits;
     const int per = (total + 7) / 8, place = static_cast<int>(blockIdx.x) >> 3;
@@ -420,9 +478,9 @@ __global__ __launch_bounds__(256, 3) void tile_i8(TiParams p) {
     const int row0 = (group - M.group_begin) * (PAIR ? kPairRows : kStoreRows), tile0 = tgroup * 2;
     // A ragged last group of one tile does the work of one.
     if (tile0 + 1 < p.tiles)
-        tile_body<TYPE, 2, PAIR>(p, M, row0, tile0, split, lds);
+        tile_body<TYPE, 2, PAIR, LONG>(p, M, row0, tile0, split, lds);
     else
-        tile_body<TYPE, 1, PAIR>(p, M, row0, tile0, split, lds);
+        tile_body<TYPE, 1, PAIR, LONG>(p, M, row0, tile0, split, lds);
 }
 
 // Adds the splits' sums in split order and stores: four rows of one token a
@@ -454,16 +512,24 @@ __global__ __launch_bounds__(256) void tile_i8_reduce(TiParams p) {
         if (r + k < M.rows) y[k] = p.accumulate ? e[k] + y[k] : e[k];
 }
 
-template <bool PAIR>
-void launch(int type, const TiParams &p, hipStream_t stream) {
+template <int TYPE, bool PAIR>
+void launch_type(const TiParams &p, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>((p.groups * p.tgroups * p.splits + 7) / 8 * 8));
     const size_t lds = ti_lds(std::min(p.tiles, 2));
-    if (type == QK_TYPE_Q4_K)
-        hipLaunchKernelGGL((tile_i8<QK_TYPE_Q4_K, PAIR>), grid, dim3(256), lds, stream, p);
-    else if (type == QK_TYPE_Q6_K)
-        hipLaunchKernelGGL((tile_i8<QK_TYPE_Q6_K, PAIR>), grid, dim3(256), lds, stream, p);
+    if (p.blocks_per_split > kShortBlocks<TYPE>)
+        hipLaunchKernelGGL((tile_i8<TYPE, PAIR, true>), grid, dim3(256), lds, stream, p);
     else
-        hipLaunchKernelGGL((tile_i8<QK_TYPE_Q6_K_SPLIT, PAIR>), grid, dim3(256), lds, stream, p);
+        hipLaunchKernelGGL((tile_i8<TYPE, PAIR, false>), grid, dim3(256), lds, stream, p);
+}
+
+template <bool PAIR>
+void launch(int type, const TiParams &p, hipStream_t stream) {
+    if (type == QK_TYPE_Q4_K)
+        launch_type<QK_TYPE_Q4_K, PAIR>(p, stream);
+    else if (type == QK_TYPE_Q6_K)
+        launch_type<QK_TYPE_Q6_K, PAIR>(p, stream);
+    else
+        launch_type<QK_TYPE_Q6_K_SPLIT, PAIR>(p, stream);
 }
 
 }  // namespace
@@ -497,8 +563,11 @@ int tile_i8_splits(const qk_matrix *mats, int n_mats, int cols, int n_tokens, in
     for (int s = 1; s <= (pair ? 1 : std::min(nb, kMaxSplits)); ++s) {
         if (s > 1 && mb * s > 1e-6 * static_cast<double>(workspace_size)) break;
         if (items * s < cus) continue;
-        const int64_t wgs = items * s, full = wgs / (3 * cus), rest = wgs % (3 * cus);
-        const double us = (nb + s - 1) / s * (full * kBlockUs[2] + (rest ? kBlockUs[(rest - 1) / cus] : 0.)) +
+        const int per = (nb + s - 1) / s;
+        const int resident = per > (mats[0].type == QK_TYPE_Q4_K ? kShortBlocks<QK_TYPE_Q4_K> : kShortBlocks<QK_TYPE_Q6_K>)
+                                 ? 2 : 3;
+        const int64_t wgs = items * s, full = wgs / (resident * cus), rest = wgs % (resident * cus);
+        const double us = per * (full * kBlockUs[resident - 1] + (rest ? kBlockUs[(rest - 1) / cus] : 0.)) +
                           (s > 1 ? kReduceUs + kSumUsPerMb * mb * s : 0.);
         if (!best || us < least) {
             best = s;

@@ -52,8 +52,51 @@ def test_exact_ragged(qk, torch_gpu, synth, qtype, cols, rows, ntok):
     assert (got[:, rows:] == 7.0).all()
 
 
+def _centred_blocks(synth, cols, rows, seed):
+    """Q4_K blocks as a quantizer leaves them: min = scale, dmin = 7.5 d, so
+    that a sub-block's mins centre its codes on zero."""
+    w = synth.quant_matrix(Q4_K, cols, rows, seed, 1).reshape(-1, 144).copy()
+    sc = synth.uniform_i32(w.shape[0] * 8, seed, 2, 16, 63).astype(np.uint8).reshape(-1, 8)
+    a, b = sc[:, :4], sc[:, 4:]
+    w[:, 4:16] = np.concatenate([a | (b >> 4) << 6, a | (b >> 4) << 6, b & 15 | (b & 15) << 4], 1)
+    d = w[:, :2].copy().view(np.float16).astype(np.float32)
+    d = np.float16(1e-4) * (1 + np.abs(d) / (1 + np.abs(d)))
+    w[:, :2] = d.astype(np.float16).view(np.uint8)
+    w[:, 2:4] = (7.5 * d.astype(np.float16)).astype(np.float16).view(np.uint8)
+    return w.reshape(-1)
+
+
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K])
+@pytest.mark.parametrize("cols,rows,ntok", [(8192, 3072, 256), (8192, 2050, 517), (14336, 4096, 256), (8192, 8192, 1000)])
+def test_rounding(qk, torch_gpu, synth, qtype, cols, rows, ntok):
+    """The fp32 sums' own error.  A rounding is 0.42 * 2^-24 of its result
+    (RMS).  The eight dots of a block are summed one after the other: 4.5
+    roundings of the block's size (RMS of the running sums).  A Q4_K block of
+    centred weights has dots of 1.9 times its own size and mins of 1.6 times,
+    the latter rounded once more before they are summed: 1.9^2 * 4.5 + 1.6^2 *
+    5.5 = 30, and two where they meet.  The nb blocks' running sum: nb / 2."""
+    t = torch_gpu
+    nb = cols // 256
+    w = _centred_blocks(synth, cols, rows, 13) if qtype == Q4_K else synth.quant_matrix(Q6_K, cols, rows, 13, 1)
+    dense = _dense(t, qk, qtype, w, cols, rows)
+    g = t.Generator().manual_seed(17)
+    xq = t.randn(ntok, cols, generator=g).mul(40).round().clamp(-127, 127).to(t.int8)
+    xs = t.rand(ntok, cols // 32, generator=g) * 1e-2 + 1e-2
+    want = (xq.double() * xs.double().repeat_interleave(32, 1)) @ dense.T
+    L = qk.lib()
+    n = L.qk_gemv_batched_i8_workspace_bytes(cols, rows, ntok)
+    ws = t.empty(n, dtype=t.uint8, device="cuda")
+    wd, xd, sd = to_dev(t, w), xq.cuda(), xs.cuda()
+    y = t.empty(ntok, rows, device="cuda")
+    qk.check(L.qk_gemv_batched_i8(qtype, wd.data_ptr(), xd.data_ptr(), cols, sd.data_ptr(), cols // 32, y.data_ptr(),
+                                  rows, cols, rows, ntok, ws.data_ptr(), n, None), "batched INT8")
+    t.cuda.synchronize()
+    roundings = (32 if qtype == Q4_K else 4.5) + nb / 2
+    assert rel_l2(y.cpu().numpy(), want.numpy()) < 0.42 * 2 ** -24 * roundings ** 0.5
+
+
 @pytest.mark.parametrize("down", [Q4_K, Q6_K])
-@pytest.mark.parametrize("dim,hidden,ntok", [(2048, 5632, 97), (3072, 8192, 200), (1024, 2816, 517)])
+@pytest.mark.parametrize("dim,hidden,ntok", [(2048, 5632, 97), (3072, 8192, 200), (1024, 2816, 517), (5120, 5632, 200)])
 def test_ffn(qk, torch_gpu, synth, down, dim, hidden, ntok):
     t = torch_gpu
     ws = [synth.quant_matrix(Q4_K, dim, hidden, 9, i) for i in (1, 2)]
