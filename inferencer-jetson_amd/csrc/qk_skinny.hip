@@ -639,7 +639,7 @@ __global__ __launch_bounds__(64 * kLoopWaves) void skinny_i8_loop(SkParams p) {
     skinny_body<TYPE, RT, true>(p, lds);
 }
 
-constexpr int kSplitsMax = 8;
+constexpr int kSplitsMax = 8;   // of a one-pass launch
 
 // The splits' sums of one (row tile, token tile), added in split order
 // (deterministic) with every split's load issued first, then the epilogue.
@@ -657,6 +657,8 @@ __global__ __launch_bounds__(256) void skinny_reduce(SkParams p) {
         #pragma unroll
         for (int s = 1; s < kSplitsMax; ++s)
             if (s < p.splits) sum += v[s];
+        // The looping kernel alone splits further: rows of 65 to 96 blocks.
+        for (int s = kSplitsMax; s < p.splits; ++s) sum += src[static_cast<size_t>(s) * RT * 1024 + e];
         return sum;
     });
 }
@@ -702,6 +704,10 @@ __global__ __launch_bounds__(256) void skinny_reduce_norm(SkParams p, int token_
                 sum.z += t.z;
                 sum.w += t.w;
             }
+        }
+        for (int sp = kSplitsMax; sp < p.splits; ++sp) {
+            const float4 t = src[static_cast<size_t>(sp) * 256];
+            sum = make_float4(sum.x + t.x, sum.y + t.y, sum.z + t.z, sum.w + t.w);
         }
         const float4 old = reinterpret_cast<const float4 *>(y)[i];
         v[k] = make_float4(sum.x + old.x, sum.y + old.y, sum.z + old.z, sum.w + old.w);

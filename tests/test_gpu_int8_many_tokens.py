@@ -27,7 +27,8 @@ def _dense(t, qk, qtype, w, cols, rows):
 
 
 @pytest.mark.parametrize("qtype", [Q4_K, Q6_K])
-@pytest.mark.parametrize("cols,rows,ntok", [(5632, 2050, 300), (8192, 1055, 545), (4096, 4096, 161)])
+@pytest.mark.parametrize("cols,rows,ntok", [(5632, 2050, 300), (8192, 1055, 545), (4096, 4096, 161),
+                                            (20480, 2050, 130)])
 def test_exact_ragged(qk, torch_gpu, synth, qtype, cols, rows, ntok):
     t = torch_gpu
     w = _integer_blocks(qtype, synth.quant_matrix(qtype, cols, rows, 5, 1), cols, rows)
