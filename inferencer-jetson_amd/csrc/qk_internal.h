@@ -498,6 +498,7 @@ struct SplitAttention {
     // (csrc/qk_tile_attention.hip): 0 none, 1 those tiles (the other tokens
     // one by one), 2 every tile is one (tile_attention_mode).
     int tile_mode;
+    int tile_runs;   // 1: no such tile has two runs; 0: it may
     // Cache layout: 0 the reference's [layers][cache_rows][kv_heads][head_dim],
     // 1 [layers][kv_heads][cache_rows][head_dim] (the decode drivers' own: a
     // (token, KV head) workgroup then reads one contiguous run of memory

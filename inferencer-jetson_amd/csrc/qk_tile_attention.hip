@@ -26,9 +26,16 @@
 //     serves the o projection's records or codes.
 //
 // A tile runs here when its tokens are all valid and form at most kMaxRuns
-// runs of consecutive positions of one sequence (each run walks its own
-// rows); the other tiles' tokens go through split_attention_kernel, which
-// decides by the same test.
+// runs of consecutive positions of one sequence, a workgroup (blockIdx.z) each;
+// the other tiles' tokens go through split_attention_kernel, which decides by
+// the same test.
+//
+// Values that are not finite: the matrix product gives every token of the tile
+// probability * value of every row, 0 * value for the rows of later tokens.
+// The few rows at the run's end that some token does not see are therefore
+// looked at first, and if one holds such a value, it takes part as zero and
+// reaches the tokens that see it after the loop.  Elsewhere the products are
+// what the per-token form's are.
 #include "qk_internal.h"
 #include "qk_records.h"
 
@@ -69,43 +76,20 @@ __device__ __forceinline__ void copies_barrier() {
 
 constexpr int kv_bytes(int hd) { return kKeys * hd * 4; }
 
-// The outputs of one (token, head) taken plainly by one wave, for a token
-// whose tile result is not finite: an infinite or NaN value in a later
-// token's row reaches an earlier token of the tile as 0 * inf.
+__device__ __forceinline__ bool finite4(const float4 &v) {
+    return isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
+}
+
+// Zeroes what is not finite in a tile of value rows: every wave that reads the
+// tile does, before it reads.
 template <int HD>
-__device__ void plain_token(const float *q, const float *kc, const float *vc, int64_t rs, int pos, float scale,
-                            int lane, float *out) {
-    float m = -INFINITY, l = 0.f;
-    auto score = [&](int key) {
-        const float *k = kc + key * rs;
-        float s = 0.f;
-        for (int d = 0; d < HD; ++d) s = fmaf(q[d], k[d], s);
-        return s * scale;
-    };
-    for (int key = lane; key <= pos; key += 64) {
-        const float s = score(key), mn = fmaxf(m, s);
-        const float ref = mn == -INFINITY ? 0.f : mn;
-        l = l * __builtin_amdgcn_exp2f(m - ref) + __builtin_amdgcn_exp2f(s - ref);
-        m = mn;
+__device__ __forceinline__ void clear_not_finite(unsigned char *vbuf, int lane) {
+    for (int i = 0; i < kv_bytes(HD) / 1024; ++i) {
+        float4 *at = reinterpret_cast<float4 *>(vbuf + i * 1024 + lane * 16);
+        const float4 v = *at;
+        *at = make_float4(isfinite(v.x) ? v.x : 0.f, isfinite(v.y) ? v.y : 0.f, isfinite(v.z) ? v.z : 0.f,
+                          isfinite(v.w) ? v.w : 0.f);
     }
-    #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const float mo = __shfl_xor(m, off), lo = __shfl_xor(l, off), mn = fmaxf(m, mo);
-        const float ref = mn == -INFINITY ? 0.f : mn;
-        l = l * __builtin_amdgcn_exp2f(m - ref) + lo * __builtin_amdgcn_exp2f(mo - ref);
-        m = mn;
-    }
-    const float ref = m == -INFINITY ? 0.f : m;
-    float acc[HD / 64];
-    #pragma unroll
-    for (int i = 0; i < HD / 64; ++i) acc[i] = 0.f;
-    for (int key = 0; key <= pos; ++key) {
-        const float p = __builtin_amdgcn_exp2f(score(key) - ref);
-        #pragma unroll
-        for (int i = 0; i < HD / 64; ++i) acc[i] = fmaf(p, vc[key * rs + i * 64 + lane], acc[i]);
-    }
-    #pragma unroll
-    for (int i = 0; i < HD / 64; ++i) out[i * 64 + lane] = acc[i] / l;
 }
 
 template <int HD>
@@ -121,7 +105,19 @@ __global__ __launch_bounds__(max_waves(HD) * 64) void tile_attention(TileAttnArg
     const int kvh = blockIdx.x, t0 = blockIdx.y * kAttnTile;
 
     const TokenTile tile = token_tile(a.desc, t0, a.n_tokens, a.cache_rows, a.max_pos, lane);
-    if (!tile.shared) return;
+    // This workgroup's run: tokens i0 .. i1 - 1 of the tile, rows 0 .. last of
+    // their sequence, of which `seen` and the ones before are all the tokens'.
+    unsigned starts = tile.starts;
+    for (unsigned r = blockIdx.z; r > 0; --r) starts &= starts - 1;
+    if (!tile.shared || !starts) return;
+    const int i0 = __builtin_ctz(starts);
+    starts &= starts - 1;
+    const int i1 = starts ? __builtin_ctz(starts) : min(kAttnTile, a.n_tokens - t0);
+    const int last = __builtin_amdgcn_readfirstlane(__shfl(tile.pos, i1 - 1)), seen = last - (i1 - i0 - 1);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(__shfl(static_cast<int>(tile.kv_row), i0));
+    const int hi = __builtin_amdgcn_readfirstlane(__shfl(static_cast<int>(tile.kv_row >> 32), i0));
+    const int64_t row = static_cast<int64_t>(hi) << 32 | lo;
+    const int mine = n >= i0 && n < i1 ? tile.pos : -1;   // rows this lane's token sees: 0 .. mine
     const int t = min(t0 + n, a.n_tokens - 1);
     const int64_t rs = a.head_major ? HD : static_cast<int64_t>(a.kv_heads) * HD;
     const float scale = 1.4426950408889634f / sqrtf(static_cast<float>(HD));
@@ -139,114 +135,114 @@ __global__ __launch_bounds__(max_waves(HD) * 64) void tile_attention(TileAttnArg
     float m = -INFINITY, l = 0.f;   // this lane's token; l over this lane's rows only
 
     unsigned char *const kbuf = lds + sg * 2 * kv_bytes(HD), *const vbuf = kbuf + kv_bytes(HD);
-    unsigned starts = tile.starts;
-    while (starts) {
-        // One run: tokens i0 .. i1 - 1, rows 0 .. last of its sequence.
-        const int i0 = __builtin_ctz(starts);
-        starts &= starts - 1;
-        const int i1 = starts ? __builtin_ctz(starts) : min(kAttnTile, a.n_tokens - t0);
-        const int last = __builtin_amdgcn_readfirstlane(__shfl(tile.pos, i1 - 1));
-        const uint32_t lo = __builtin_amdgcn_readfirstlane(__shfl(static_cast<int>(tile.kv_row), i0));
-        const int hi = __builtin_amdgcn_readfirstlane(__shfl(static_cast<int>(tile.kv_row >> 32), i0));
-        const int64_t row = static_cast<int64_t>(hi) << 32 | lo;
-        const int mine = n >= i0 && n < i1 ? tile.pos : -1;   // rows this lane's token sees: 0 .. mine
-        const int64_t base = kv_offset(a.head_major, a.layer, a.cache_rows, a.kv_heads, HD, row, kvh);
-        const float *kc = a.key_cache + base, *vc = a.value_cache + base;
-        const int tiles = last / kKeys + 1, iters = (tiles + S - 1) / S;
+    const int64_t base = kv_offset(a.head_major, a.layer, a.cache_rows, a.kv_heads, HD, row, kvh);
+    const float *kc = a.key_cache + base, *vc = a.value_cache + base;
+    const int tiles = last / kKeys + 1, iters = (tiles + S - 1) / S;
+    // Tiles from `edge` on hold rows that some token does not see: such a row
+    // meets that token as 0 * value, so what is not finite in them (bad: there
+    // is any) is zeroed there and joins after the loop.
+    const int edge = (seen + 1) / kKeys;
 
-        // 1 KB of a tile is 256 / HD rows; the group's G waves share the
-        // pieces.  Rows past the last are the last again (in bounds; masked).
-        auto copy_tile = [&](const float *src, unsigned char *dst, int j, bool rotate) {
-            constexpr int kRowsPer = 256 / HD, kPieces = kKeys / kRowsPer;
-            for (int i = g; i < kPieces; i += G) {
-                const int r = i * kRowsPer + lane / kChunks, slot = lane % kChunks;
-                const int chunk = rotate ? slot ^ (r & 15) : slot;
-                dma16(src + static_cast<int64_t>(min(j * kKeys + r, last)) * rs + 4 * chunk, lds_address(dst + i * 1024));
-            }
-        };
-        copy_tile(kc, kbuf, sg, true);
-        copies_barrier();
-        copy_tile(vc, vbuf, sg, false);
-        for (int it = 0; it < iters; ++it) {
-            const int j = it * S + sg;
-            const bool live = j < tiles;
-            float4v st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-            if (live) {
-                // Chains of 16 products (8 at head_dim 64), added as a tree: as
-                // exact as the per-token form's lane sums (2.1e-7 of float64
-                // at head_dim 128; 4.8e-7 as one chain over a head).
+    // 1 KB of a tile is 256 / HD rows; the group's G waves share the
+    // pieces.  Rows past the last are the last again (in bounds; masked).
+    auto copy_tile = [&](const float *src, unsigned char *dst, int j, bool rotate) {
+        constexpr int kRowsPer = 256 / HD, kPieces = kKeys / kRowsPer;
+        for (int i = g; i < kPieces; i += G) {
+            const int r = i * kRowsPer + lane / kChunks, slot = lane % kChunks;
+            const int chunk = rotate ? slot ^ (r & 15) : slot;
+            dma16(src + static_cast<int64_t>(min(j * kKeys + r, last)) * rs + 4 * chunk, lds_address(dst + i * 1024));
+        }
+    };
+    copy_tile(kc, kbuf, sg, true);
+    bool bad = false;
+    for (int i = threadIdx.x; i < (last + 1 - edge * kKeys) * kChunks; i += blockDim.x)
+        bad |= !finite4(*reinterpret_cast<const float4 *>(vc + (edge * kKeys + i / kChunks) * rs + i % kChunks * 4));
+    bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    int *const flags = reinterpret_cast<int *>(lds + S * 2 * kv_bytes(HD));   // one a wave
+    if (lane == 0) flags[wave] = bad;
+    copies_barrier();
+    copy_tile(vc, vbuf, sg, false);
+    bad = __builtin_amdgcn_ballot_w64(flags[lane < G * S ? lane : 0]) != 0;
+    for (int it = 0; it < iters; ++it) {
+        const int j = it * S + sg;
+        const bool live = j < tiles;
+        float4v st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        if (live) {
+            // Chains of 16 products (8 at head_dim 64), added as a tree: as
+            // exact as the per-token form's lane sums (2.1e-7 of float64
+            // at head_dim 128; 4.8e-7 as one chain over a head).
+            #pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float4v part[2][4];
                 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    float4v part[2][4];
-                    #pragma unroll
-                    for (int e = 0; e < 4; ++e) part[0][e] = part[1][e] = float4v{0.f, 0.f, 0.f, 0.f};
-                    #pragma unroll
-                    for (int x = 0; x < NJ; ++x) {
-                        const float4 k =
-                            *reinterpret_cast<const float4 *>(kbuf + ((h * 16 + n) * kChunks + ((4 * x + kq) ^ n)) * 16);
-                        float4v(&c)[4] = part[x & 1];
-                        c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.x, q[x].x, c[0], 0, 0, 0);
-                        c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.y, q[x].y, c[1], 0, 0, 0);
-                        c[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.z, q[x].z, c[2], 0, 0, 0);
-                        c[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.w, q[x].w, c[3], 0, 0, 0);
-                    }
-                    #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        st[h][r] = ((part[0][0][r] + part[0][1][r]) + (part[0][2][r] + part[0][3][r])) +
-                                   ((part[1][0][r] + part[1][1][r]) + (part[1][2][r] + part[1][3][r]));
+                for (int e = 0; e < 4; ++e) part[0][e] = part[1][e] = float4v{0.f, 0.f, 0.f, 0.f};
+                #pragma unroll
+                for (int x = 0; x < NJ; ++x) {
+                    const float4 k =
+                        *reinterpret_cast<const float4 *>(kbuf + ((h * 16 + n) * kChunks + ((4 * x + kq) ^ n)) * 16);
+                    float4v(&c)[4] = part[x & 1];
+                    c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.x, q[x].x, c[0], 0, 0, 0);
+                    c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.y, q[x].y, c[1], 0, 0, 0);
+                    c[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.z, q[x].z, c[2], 0, 0, 0);
+                    c[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.w, q[x].w, c[3], 0, 0, 0);
                 }
+                #pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    st[h][r] = ((part[0][0][r] + part[0][1][r]) + (part[0][2][r] + part[0][3][r])) +
+                               ((part[1][0][r] + part[1][1][r]) + (part[1][2][r] + part[1][3][r]));
             }
-            copies_barrier();   // the values are in; every wave is done with the keys
-            if (it + 1 < iters) copy_tile(kc, kbuf, j + S, true);
-            if (live) {
-                // Register r of half h: row j * 32 + 16 h + 4 kq + r.
-                float mx = -INFINITY;
+        }
+        copies_barrier();   // the values are in; every wave is done with the keys
+        if (it + 1 < iters) copy_tile(kc, kbuf, j + S, true);
+        if (live) {
+            // Register r of half h: row j * 32 + 16 h + 4 kq + r.
+            float mx = -INFINITY;
+            #pragma unroll
+            for (int h = 0; h < 2; ++h)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    st[h][r] = j * kKeys + 16 * h + 4 * kq + r <= mine ? st[h][r] * scale : -INFINITY;
+                    mx = fmaxf(mx, st[h][r]);
+                }
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float mn = fmaxf(m, mx);
+            const float ref = mn == -INFINITY ? 0.f : mn;
+            const float f = __builtin_amdgcn_exp2f(m - ref);
+            m = mn;
+            #pragma unroll
+            for (int h = 0; h < 2; ++h)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) st[h][r] = __builtin_amdgcn_exp2f(st[h][r] - ref);
+            l = fmaf(l, f, ((st[0][0] + st[0][1]) + (st[0][2] + st[0][3])) +
+                               ((st[1][0] + st[1][1]) + (st[1][2] + st[1][3])));
+            if (bad && j >= edge) clear_not_finite<HD>(vbuf, lane);
+            // The tile's outputs on their own, then added: the chain over
+            // a head's rows is one step per tile.
+            #pragma unroll
+            for (int x = 0; x < NT; ++x) {
+                float4v to[4];
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) to[i] = float4v{0.f, 0.f, 0.f, 0.f};
                 #pragma unroll
                 for (int h = 0; h < 2; ++h)
                     #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        st[h][r] = j * kKeys + 16 * h + 4 * kq + r <= mine ? st[h][r] * scale : -INFINITY;
-                        mx = fmaxf(mx, st[h][r]);
+                        const float4 v = *reinterpret_cast<const float4 *>(
+                            vbuf + ((h * 16 + 4 * kq + r) * kChunks + 16 * x + n) * 16);
+                        to[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, st[h][r], to[0], 0, 0, 0);
+                        to[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, st[h][r], to[1], 0, 0, 0);
+                        to[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, st[h][r], to[2], 0, 0, 0);
+                        to[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, st[h][r], to[3], 0, 0, 0);
                     }
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
-                const float mn = fmaxf(m, mx);
-                const float ref = mn == -INFINITY ? 0.f : mn;
-                const float f = __builtin_amdgcn_exp2f(m - ref);
-                m = mn;
                 #pragma unroll
-                for (int h = 0; h < 2; ++h)
+                for (int i = 0; i < 4; ++i)
                     #pragma unroll
-                    for (int r = 0; r < 4; ++r) st[h][r] = __builtin_amdgcn_exp2f(st[h][r] - ref);
-                l = fmaf(l, f, ((st[0][0] + st[0][1]) + (st[0][2] + st[0][3])) +
-                                   ((st[1][0] + st[1][1]) + (st[1][2] + st[1][3])));
-                // The tile's outputs on their own, then added: the chain over
-                // a head's rows is one step per tile.
-                #pragma unroll
-                for (int x = 0; x < NT; ++x) {
-                    float4v to[4];
-                    #pragma unroll
-                    for (int i = 0; i < 4; ++i) to[i] = float4v{0.f, 0.f, 0.f, 0.f};
-                    #pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const float4 v = *reinterpret_cast<const float4 *>(
-                                vbuf + ((h * 16 + 4 * kq + r) * kChunks + 16 * x + n) * 16);
-                            to[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, st[h][r], to[0], 0, 0, 0);
-                            to[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, st[h][r], to[1], 0, 0, 0);
-                            to[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, st[h][r], to[2], 0, 0, 0);
-                            to[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, st[h][r], to[3], 0, 0, 0);
-                        }
-                    #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        #pragma unroll
-                        for (int r = 0; r < 4; ++r) o[x][i][r] = fmaf(o[x][i][r], f, to[i][r]);
-                }
+                    for (int r = 0; r < 4; ++r) o[x][i][r] = fmaf(o[x][i][r], f, to[i][r]);
             }
-            copies_barrier();   // the next keys are in; every wave is done with the values
-            if (it + 1 < iters) copy_tile(vc, vbuf, j + S, false);
         }
+        copies_barrier();   // the next keys are in; every wave is done with the values
+        if (it + 1 < iters) copy_tile(vc, vbuf, j + S, false);
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
@@ -283,6 +279,29 @@ __global__ __launch_bounds__(max_waves(HD) * 64) void tile_attention(TileAttnArg
                     for (int r = 0; r < 4; ++r) o[x][i][r] = fmaf(po[r], fo, o[x][i][r] * f);
                 }
         }
+        // The values that were zeroed, for the tokens that see them: of the
+        // few rows at the run's end, p * value as the sums would have taken it.
+        for (int key = edge * kKeys; bad && key <= last; ++key) {
+            float sc = 0.f;
+            #pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float4 k = *reinterpret_cast<const float4 *>(kc + key * rs + 16 * j + 4 * kq);
+                sc = fmaf(q[j].x, k.x, fmaf(q[j].y, k.y, fmaf(q[j].z, k.z, fmaf(q[j].w, k.w, sc))));
+            }
+            sc += __shfl_xor(sc, 16);
+            sc += __shfl_xor(sc, 32);
+            const float pr = __builtin_amdgcn_exp2f(sc * scale - m);
+            #pragma unroll
+            for (int x = 0; x < NT; ++x)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float4 v = *reinterpret_cast<const float4 *>(vc + key * rs + 64 * x + 16 * kq + 4 * r);
+                    const float v4[4] = {v.x, v.y, v.z, v.w};
+                    #pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        o[x][i][r] = key <= mine && !isfinite(v4[i]) ? fmaf(pr, v4[i], o[x][i][r]) : o[x][i][r];
+                }
+        }
     }
     __syncthreads();   // the states are read: the output tile takes their place
 
@@ -291,31 +310,18 @@ __global__ __launch_bounds__(max_waves(HD) * 64) void tile_attention(TileAttnArg
     float *out = reinterpret_cast<float *>(lds);
     const int width = G * HD;
     if (sg == 0) {
-        bool finite = true;
         #pragma unroll
         for (int x = 0; x < NT; ++x)
             #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float4 v = make_float4(o[x][0][r] / l, o[x][1][r] / l, o[x][2][r] / l, o[x][3][r] / l);
-                finite = finite && isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
-                *reinterpret_cast<float4 *>(out + n * width + g * HD + 64 * x + 16 * kq + 4 * r) = v;
-            }
-        uint64_t bad = __builtin_amdgcn_ballot_w64(!finite && t0 + n < a.n_tokens);
-        bad = (bad | (bad >> 16) | (bad >> 32) | (bad >> 48)) & 0xFFFF;
-        while (bad) {
-            const int i = __builtin_ctzll(bad);
-            bad &= bad - 1;
-            const qk_batch_token d = a.desc[t0 + i];
-            const int64_t base = kv_offset(a.head_major, a.layer, a.cache_rows, a.kv_heads, HD, d.kv_row, kvh);
-            plain_token<HD>(a.q + (static_cast<int64_t>(t0 + i) * a.heads + kvh * G + g) * HD, a.key_cache + base,
-                            a.value_cache + base, rs, d.pos, scale, lane, out + i * width + g * HD);
-        }
+            for (int r = 0; r < 4; ++r)
+                *reinterpret_cast<float4 *>(out + n * width + g * HD + 64 * x + 16 * kq + 4 * r) =
+                    make_float4(o[x][0][r] / l, o[x][1][r] / l, o[x][2][r] / l, o[x][3][r] / l);
     }
     __syncthreads();
-    const int have = min(kAttnTile, a.n_tokens - t0);
+    const int have = i1 - i0;
     const int64_t ld = static_cast<int64_t>(a.heads) * HD;
     for (int i = threadIdx.x; i < have * (width / 4); i += blockDim.x) {
-        const int tok = i / (width / 4), c = i - tok * (width / 4);
+        const int at = i / (width / 4), c = i - at * (width / 4), tok = i0 + at;
         *reinterpret_cast<float4 *>(a.out + (t0 + tok) * ld + kvh * width + 4 * c) =
             *reinterpret_cast<const float4 *>(out + tok * width + 4 * c);
     }
@@ -323,7 +329,7 @@ __global__ __launch_bounds__(max_waves(HD) * 64) void tile_attention(TileAttnArg
     if (a.gemm_rec || a.q8_out) {
         const int per = (width + 255) / 256, waves = blockDim.x / 64;
         for (int i = wave; i < have * per; i += waves) {
-            const int tok = i / per, blk = i - tok * per, c = blk * 256 + 4 * lane, b = t0 + tok;
+            const int at = i / per, blk = i - at * per, c = blk * 256 + 4 * lane, tok = i0 + at, b = t0 + tok;
             const bool in = c < width;
             const float4 v = in ? *reinterpret_cast<const float4 *>(out + tok * width + c) : make_float4(0.f, 0.f, 0.f, 0.f);
             if (a.gemm_rec) {
@@ -401,6 +407,7 @@ int tile_attention_mode(const qk_batch_token *desc, SplitAttention &a) {
     }
     if (!tiled || !tile_attention_pays(tiled, a.kv_heads, a.heads, a.head_dim, tiled_rows, max_rows, two_runs))
         return 0;
+    a.tile_runs = two_runs ? kMaxRuns : 1;
     if (tiled == a.n_tokens) return 2;
     a.rows_hint = rows;
     return 1;
@@ -410,10 +417,11 @@ int launch_tile_attention(const SplitAttention &a, hipStream_t stream) {
     TileAttnArgs ta{a, 1};
     const int G = a.heads / a.kv_heads, hd = a.head_dim;
     ta.groups = tile_groups(G, hd);
-    const size_t lds = std::max({static_cast<size_t>(ta.groups) * 2 * kv_bytes(hd),
+    const size_t lds = std::max({static_cast<size_t>(ta.groups) * 2 * kv_bytes(hd) + sizeof(int) * max_waves(hd),
                                  static_cast<size_t>(ta.groups - 1) * G * (16 * hd + 32) * sizeof(float),
                                  static_cast<size_t>(kAttnTile) * G * hd * sizeof(float)});
-    const dim3 grid(a.kv_heads, (a.n_tokens + kAttnTile - 1) / kAttnTile), block(64 * G * ta.groups);
+    const dim3 grid(a.kv_heads, (a.n_tokens + kAttnTile - 1) / kAttnTile, a.tile_runs == 1 ? 1 : kMaxRuns),
+        block(64 * G * ta.groups);
     if (hd == 64)
         hipLaunchKernelGGL(tile_attention<64>, grid, block, lds, stream, ta);
     else

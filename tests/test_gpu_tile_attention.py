@@ -93,3 +93,57 @@ def test_later_rows_not_finite(qk, torch_gpu):
     per_token = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd, split_rows=512)
     assert np.array_equal(np.isfinite(got), np.isfinite(per_token))
     assert rel_l2(got[np.isfinite(got)], per_token[np.isfinite(got)]) < TOL
+
+
+def test_poisoned_sequence_time(qk, torch_gpu):
+    """A non-finite early row makes every result of its sequence non-finite, at
+    the cost of a clean one: every tile is taken once, whatever it holds."""
+    t = torch_gpu
+    heads, kvh, hd = 24, 8, 128
+    rng = np.random.default_rng(9)
+    q, key, value, tokens = batch(rng, [(1000, 500)], heads, kvh, hd)
+    n, top = len(tokens), tokens[-1][0]
+    desc = to_dev(t, np.array([[p | (i << 32), r] for i, (p, r) in enumerate(tokens)], dtype=np.int64))
+    ws = t.empty(qk.lib().qk_attention_split_workspace_bytes(n, heads, kvh, hd, top, 0), dtype=t.uint8, device="cuda")
+    out, qd, kd = t.empty((n, heads * hd), device="cuda"), to_dev(t, q), to_dev(t, key)
+
+    def best(vd):
+        times = []
+        for _ in range(5):
+            a, b = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
+            a.record()
+            qk.check(qk.lib().qk_attention_split_f32(
+                qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), 0, len(key), desc.data_ptr(), n, top, heads,
+                kvh, hd, 0, ws.data_ptr(), ws.numel(), t.cuda.current_stream().cuda_stream), "attention")
+            b.record()
+            t.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    clean = best(to_dev(t, value))
+    value[3] = np.nan
+    assert best(to_dev(t, value)) < 3 * clean
+    assert t.isnan(out).all()
+
+
+def test_rows_at_a_run_end_not_finite(qk, torch_gpu):
+    """Infinities in the rows of the chunk's own tokens, among them the first
+    and last of a 16-token tile and of a 32-row tile: a token that sees one has
+    it in its result (two of opposite sign: NaN), one that does not is untouched."""
+    heads, kvh, hd = 32, 8, 64
+    rng = np.random.default_rng(10)
+    q, key, value, tokens = batch(rng, [(700, 500)], heads, kvh, hd)
+    clean = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd, split_rows=704)
+    want = clean.copy()
+    group = heads // kvh
+    for tok, h, d, v in [(0, 0, 3, np.inf), (15, 1, 60, -np.inf), (16, 2, 0, np.nan), (56, 3, 63, np.inf),
+                         (87, 4, 33, -np.inf), (88, 4, 33, np.inf), (499, 7, 17, np.inf)]:
+        value[200 + tok, h * hd + d] = v
+        for g in range(group):
+            with np.errstate(invalid="ignore"):
+                want[tok:, (h * group + g) * hd + d] += v
+    got = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isfinite(got), finite)
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert rel_l2(got[finite], want[finite]) < TOL
