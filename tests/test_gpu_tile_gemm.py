@@ -75,3 +75,39 @@ def test_large_workspace_splits(qk, torch_gpu, oracle, workloads, synth):
     x = synth.normal_f32(ntok * cols, 33, ntok).reshape(ntok, cols)
     t = torch_gpu
     check(qk, t, oracle, [matrix(qk, t, workloads, synth, Q4_K, cols, rows, 50)], x, cols, extra=8 << 20)
+
+
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K_SPLIT])
+def test_error_of_long_rows(qk, torch_gpu, workloads, synth, qtype):
+    """32-block rows of 517 tokens are as exact as the same tokens 32 at a time
+    (the kernel of one token tile, whose sums are at most four blocks long):
+    both errors are RMS over a million outputs, so 2 % covers the draw."""
+    t = torch_gpu
+    ntok, cols, rows = 517, 8192, 3072
+    g = t.Generator(device="cuda").manual_seed(5)
+    x = t.randn((ntok, cols), device="cuda", generator=g) * t.exp(0.5 * t.randn(cols, device="cuda", generator=g))
+    if qtype == Q4_K:   # mins that centre the weights, as a quantizer leaves them
+        w, _ = workloads.gemv_case(Q4_K, cols, rows, seed=55)
+        w = w.reshape(-1, 144).copy()
+        sc = synth.uniform_i32(w.shape[0] * 8, 56, 2, 16, 63).astype(np.uint8).reshape(-1, 8)
+        a, b = sc[:, :4], sc[:, 4:]
+        w[:, 4:16] = np.concatenate([a | (b >> 4) << 6, a | (b >> 4) << 6, b & 15 | (b & 15) << 4], 1)
+        w[:, 0:2], w[:, 2:4] = np.array([1e-4], np.float16).view(np.uint8), np.array([7.5e-4], np.float16).view(np.uint8)
+        ten = qk.Tensor((cols, rows), Q4_K, to_dev(t, w.reshape(-1)))
+    else:
+        ten, _, _ = matrix(qk, t, workloads, synth, qtype, cols, rows, 57)
+    dense = t.empty((rows, cols), device="cuda")
+    qk.dequant_rows(ten, dense, 0, rows)
+    want = x.double() @ dense.double().T
+    ws = t.empty(qk.batch_workspace_bytes(cols, rows, ntok), dtype=t.uint8, device="cuda")
+
+    def error(step):
+        y = t.empty((ntok, rows), device="cuda")
+        for i in range(0, ntok, step):
+            n = min(step, ntok - i)
+            qk.check(qk.lib().qk_gemv_batched_f32(ten.type, ten.gpu, x[i:].data_ptr(), cols, y[i:].data_ptr(), rows, cols,
+                                                  rows, n, ws.data_ptr(), ws.numel(), None), "batched")
+        t.cuda.synchronize()
+        return float((y.double() - want).norm() / want.norm())
+
+    assert error(ntok) < 1.02 * error(32)
