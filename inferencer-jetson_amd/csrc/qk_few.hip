@@ -131,7 +131,7 @@ __device__ __forceinline__ void load_block_input(const float *x, int ldx, int n_
 // [2^14, 2^15), fp16 high and low halves, sums of 32 values, a non-finite value
 // making the token's scale NaN).  Rows of absent tokens hold anything.
 template <bool Q4>
-__device__ __forceinline__ void build_operand(const float4 (&v)[kSlots - 1], int n_tokens, bool real, int lane,
+__device__ __forceinline__ void build_operand(const float4 (&v)[kSlots - 1], int n_tokens, int lane,
                                               unsigned char *scratch, Operand<Q4> &op) {
     const int kq = lane >> 4;
     // Lane l's columns 4 l .. +3: operand step, quarter and half.
@@ -156,10 +156,8 @@ __device__ __forceinline__ void build_operand(const float4 (&v)[kSlots - 1], int
             f = ldexpf(1.f, -shift);
         }
         if (bad) f = __builtin_nanf("");
-        if (!real) f = 0.f;
-        const bool zero = bad || !real;
-        const float x4[4] = {zero ? 0.f : ldexpf(x.x, shift), zero ? 0.f : ldexpf(x.y, shift),
-                             zero ? 0.f : ldexpf(x.z, shift), zero ? 0.f : ldexpf(x.w, shift)};
+        const float x4[4] = {bad ? 0.f : ldexpf(x.x, shift), bad ? 0.f : ldexpf(x.y, shift),
+                             bad ? 0.f : ldexpf(x.z, shift), bad ? 0.f : ldexpf(x.w, shift)};
         half4 h, l;
         #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -273,7 +271,7 @@ __device__ __forceinline__ void few_body(const FewParams &p, const FewMatrix &M,
         return m.w + static_cast<size_t>(min(tile * kTileRows + n, M.rows - 1)) * m.row_bytes;
     };
     // Wave w's blocks: w and, with two, w + waves (past the row's end the last
-    // block again, over zero activations).
+    // block is read again and left out).
     const bool second = wave + waves < p.nb;
     const int blk0 = wave, blk1 = min(wave + waves, p.nb - 1);
     Raw<Q4> cur[NTL], more;
@@ -329,8 +327,8 @@ __device__ __forceinline__ void few_body(const FewParams &p, const FewMatrix &M,
         }
     }
     Operand<Q4> op, op2;
-    build_operand<Q4>(v[0], p.n_tokens, true, lane, scratch, op);
-    if constexpr (BPW == 2) build_operand<Q4>(v[1], p.n_tokens, second, lane, scratch, op2);
+    build_operand<Q4>(v[0], p.n_tokens, lane, scratch, op);
+    if constexpr (BPW == 2) build_operand<Q4>(v[1], p.n_tokens, lane, scratch, op2);
     __syncthreads();   // the scratch becomes the sums
 
     // Store the step's outputs from its sums: the waves' in wave order, the
@@ -368,7 +366,7 @@ __device__ __forceinline__ void few_body(const FewParams &p, const FewMatrix &M,
         // One step a workgroup (launch_few).
         float4v acc = {0.f, 0.f, 0.f, 0.f};
         multiply_block<TYPE>(cur[0], op, kq, acc);
-        multiply_block<TYPE>(more, op2, kq, acc);
+        if (second) multiply_block<TYPE>(more, op2, kq, acc);
         publish(acc, red + wave * 128);
         meet();
         store(item0, red);

@@ -64,3 +64,24 @@ def test_not_finite(qk, torch_gpu, workloads, synth):
     t.cuda.synchronize()
     got = y.cpu().numpy()
     assert np.isnan(got[2]).all() and np.isfinite(got[[0, 1, 3]]).all()
+
+
+def test_infinite_scale_in_the_last_block(qk, torch_gpu, oracle, workloads, synth):
+    """31 blocks a row, two a wave: the wave without a second block adds nothing.
+    Where the row's last block has an infinite scale, its high and low products
+    are infinite, of one sign in about half of the outputs; the last block again
+    over zeros would make every one NaN."""
+    t = torch_gpu
+    ntok, cols, rows = 7, 31 * 256, 4096
+    x = synth.normal_f32(ntok * cols, 65, ntok).reshape(ntok, cols)
+    w, _ = workloads.gemv_case(Q4_K, cols, rows, seed=91)
+    w = w.reshape(rows, 31, 144).copy()
+    w[::5, 30, 0:2] = np.array([np.inf], np.float16).view(np.uint8)
+    ten, y = qk.Tensor((cols, rows), Q4_K, to_dev(t, w.reshape(-1))), t.empty((ntok, rows), device="cuda")
+    qk.batch_matvec(ten, to_dev(t, x), y, cols, rows, ntok)
+    t.cuda.synchronize()
+    y = y.cpu().numpy()
+    assert not np.isfinite(y[:, ::5]).any() and 0.3 < np.isinf(y[:, ::5]).mean() < 0.7
+    keep = np.arange(rows) % 5 != 0
+    w[::5, 30, 0:2] = 0
+    assert rel_l2(y[:, keep], oracle.gemv_f64(Q4_K, w.reshape(-1), x, cols, rows)[:, keep]) < TOL
