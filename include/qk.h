@@ -118,7 +118,11 @@ int qk_gemv_multi_f32(const qk_matrix *mats, int n_mats, const float *x, int col
    partial sums; below 8 tokens it is 0 and the pointer may be NULL.  It
    plays the part of the reference's preallocated batch buffers
    (inferencer.cu:1237-1238) and never needs clearing.  Base alignment 256
-   bytes. */
+   bytes.  With this many bytes or more, what a call adds in which order
+   depends on the call alone; from 33 tokens on, a smaller buffer that holds
+   what the call cannot do without is accepted too and may get fewer splits
+   (the same sums, rounded in another order).  The same holds for the queries
+   of the feed-forward block and of the INT8 products below. */
 size_t qk_gemv_batched_workspace_bytes(int cols, int rows, int n_tokens);
 
 /* Multi-token variant: y[t*ldy + r] = sum_c W[r][c] * x[t*ldx + c] for
@@ -148,10 +152,11 @@ int qk_gemv_multi_batched_f32(const qk_matrix *mats, int n_mats, const float *x,
    1362-1380) with FP32 semantics.  From 8 tokens on it runs as five
    launches on the matrix cores: the gate / up reduction packs SiLU(gate) *
    up straight into the down projection's input records, so neither gate,
-   up nor their product is stored as fp32; below 8 tokens, a gate / up
-   launch that writes SiLU * up (2 to 7 tokens of like gate and up: one read
-   of the weights on the matrix cores; otherwise the fused GEMV pair) and a
-   down launch.  workspace:
+   up nor their product is stored as fp32; below 8 tokens, the fused GEMV pair
+   of qk_gemv_multi_f32 and a down GEMV staging SiLU * up, or, where that is
+   estimated to take less time (3 to 7 tokens of large like gate and up), one
+   read of their weights on the matrix cores that writes SiLU * up, and a down
+   launch over it.  workspace:
    qk_ffn_batched_workspace_bytes(dim, hidden, n_tokens) bytes (256-byte
    aligned; also enough for fewer tokens), not shared by calls in flight at
    the same time.  dim and hidden multiples of 256.  No reference

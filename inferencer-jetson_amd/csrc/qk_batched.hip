@@ -722,9 +722,8 @@ int check_batched(const char *where, const float *x, int ldx, int cols, int n_to
 
 int tile_count(int n_tokens) { return (n_tokens + kTokTile - 1) / kTokTile; }
 
-// The workspace's size: what a GEMM of 128 * RT rows x 32 * RT tokens a
-// workgroup with split_plan's splits needs (RT 1 for one token tile, else 2).
-// The launches fit their own plans into it.
+// The least workspace: split_plan's for 128 * RT rows x 32 * RT tokens a
+// workgroup (RT 1 for one token tile, else 2).
 int row_tiles(int tiles) { return tiles >= 2 ? 2 : 1; }
 constexpr int group_rows(int rt) { return 128 * rt; }
 constexpr int partial_floats(int rt) { return 4 * rt * 16 * 64; }
@@ -757,9 +756,43 @@ int64_t group_count(const int *rows, int n, int rt) {
     return g;
 }
 
-// Workspace: packed activation records, then (when blocks are split, or
-// always with `partials`: a reduction stage that must run) the partial sums
-// of every (row group, token tile, split).
+// How many workgroups share one row group's blocks from two token tiles on:
+// the count with the least estimated time.  A workgroup alone on its CU takes
+// kBlockUs a Q4_K block (kWideUs a Q6_K block, three chains), two on one CU
+// twice that each (csrc/qk_tile_gemm.h); a split's partial sums cost
+// kPartialUsPerMb written and read back, and the reduction kReduceUs once there
+// are any.  Measured against every count from 1 to 16 at 64 to 517 tokens on
+// the 1B and 3B shapes: within 2 us of the best.  Splits make at most
+// kMaxSplitGroups workgroups, which bounds their sums to 32 MB.
+constexpr int kMaxSplitGroups = 1024;
+void tile_split_plan(int64_t groups, int64_t rows, int nb, int n_tokens, bool wide, bool must_reduce, int max_splits,
+                     int &splits, int &per_split) {
+    constexpr double kBlockUs = 2.5, kWideUs = 3.4, kPartialUsPerMb = 0.4, kReduceUs = 4.;
+    const int64_t cus = device_info().cus, wgs1 = (tile_count(n_tokens) + 1) / 2 * groups;
+    const double block_us = wide ? kWideUs : kBlockUs, out_mb = 4e-6 * static_cast<double>(rows) * n_tokens;
+    double best = 0.;
+    for (int s = 1; s <= std::min(std::min(max_splits, kMaxSplit), nb); ++s) {
+        const int per = (nb + s - 1) / s;
+        if ((nb + per - 1) / per != s || (s > 1 && wgs1 * s > kMaxSplitGroups)) continue;
+        const int64_t wgs = wgs1 * s, rest = wgs % (2 * cus);
+        const double rounds = 2. * static_cast<double>(wgs / (2 * cus)) + (rest > cus ? 2. : rest > 0 ? 1. : 0.);
+        const double us = rounds * per * block_us + (s > 1 || must_reduce ? s * out_mb * kPartialUsPerMb : 0.) +
+                          (s > 1 && !must_reduce ? kReduceUs : 0.);
+        if (best == 0. || us < best) {
+            best = us;
+            splits = s;
+            per_split = per;
+        }
+    }
+}
+
+size_t tile_partial_bytes(int64_t groups, int tiles, int splits) {
+    return static_cast<size_t>(groups) * tiles * splits * kPartialFloats * sizeof(float);
+}
+
+// The least workspace a call takes: packed activation records, then (when
+// blocks are split, or always with `partials`: a reduction stage that must run)
+// the partial sums of every (row group, token tile, split).
 size_t workspace_bytes(int cols, const int *rows, int n_mats, int n_tokens, bool partials = false) {
     if (cols <= 0 || cols % 256 || n_mats < 1 || n_tokens < kMfmaMinTokens) return 0;
     const int tiles = tile_count(n_tokens);
@@ -776,7 +809,7 @@ size_t workspace_bytes(int cols, const int *rows, int n_mats, int n_tokens, bool
 // Workspace bound for the public query, which knows only the total row
 // count: the group count of any split of `rows_total` rows over at most
 // QK_MAX_FUSED matrices is at most rows_total/group_rows + QK_MAX_FUSED.
-size_t workspace_bound(int cols, int rows_total, int n_tokens, bool partials = false) {
+size_t least_bound(int cols, int rows_total, int n_tokens, bool partials = false) {
     if (rows_total <= 0) return 0;
     const int tiles = tile_count(n_tokens);
     if (cols <= 0 || cols % 256 || n_tokens < kMfmaMinTokens) return 0;
@@ -797,6 +830,33 @@ size_t workspace_bound(int cols, int rows_total, int n_tokens, bool partials = f
     split_plan(gmin, cols / 256, tiles, s_min, ps);
     if (s_min > 1 || partials) best = std::max(best, static_cast<size_t>(gmax) * tiles * s_min * slot);
     return bytes + best;
+}
+
+// What the queries answer: also what tile_split_plan's choice takes, for any
+// types and row groups, so that a launch with this much need not look at the
+// size.
+size_t workspace_bound(int cols, int rows_total, int n_tokens, bool partials = false) {
+    const size_t least = least_bound(cols, rows_total, n_tokens, partials);
+    const int tiles = tile_count(n_tokens);
+    if (!least || tiles < 2) return least;
+    size_t best = 0;
+    for (int64_t g = (rows_total + kGroupRows - 1) / kGroupRows; g <= rows_total / kGroupRows + QK_MAX_FUSED; ++g)
+        for (bool wide : {false, true}) {
+            int splits, per_split;
+            tile_split_plan(g, rows_total, cols / 256, n_tokens, wide, partials, kMaxSplit, splits, per_split);
+            if (splits > 1 || partials) best = std::max(best, tile_partial_bytes(g, tiles, splits));
+        }
+    return std::max(least, (records_bytes(cols, n_tokens) + 255) / 256 * 256 + best);
+}
+
+// The same bound without the enumeration, also for fewer tokens: splits of a
+// workgroup write two tiles' sums each, all of them at most kMaxSplitGroups'.
+size_t plan_bytes(int cols, int rows_total, int n_tokens, bool partials) {
+    const int tiles = tile_count(n_tokens);
+    if (tiles < 2) return 0;
+    const size_t once = tile_partial_bytes(rows_total / kGroupRows + QK_MAX_FUSED, tiles, 1);
+    return (records_bytes(cols, n_tokens) + 255) / 256 * 256 +
+           std::max(partials ? once : 0, std::min(kMaxSplit * once, tile_partial_bytes(kMaxSplitGroups, 2, 1)));
 }
 
 void launch_gemm(int type, const dim3 &grid, hipStream_t stream, const BatchParams &p) {
@@ -822,38 +882,6 @@ void launch_tile_gemm(int type, int64_t groups, hipStream_t stream, const BatchP
         hipLaunchKernelGGL(tile_gemm<QK_TYPE_Q6_K_SPLIT>, grid, dim3(256), kTileLds, stream, p, g, tgroups);
     else
         hipLaunchKernelGGL(tile_gemm<0>, grid, dim3(256), kTileLds, stream, p, g, tgroups);
-}
-
-// How many workgroups share one row group's blocks: the count with the least
-// estimated time.  A workgroup alone on its CU takes kBlockUs a Q4_K block
-// (kWideUs a Q6_K block, three chains), two on one CU twice that each
-// (csrc/qk_tile_gemm.h); a split's partial sums cost kPartialUsPerMb written
-// and read back, and the reduction kReduceUs once there are any.  Measured
-// against every count from 1 to 16 at 64 to 517 tokens on the 1B and 3B
-// shapes: within 2 us of the best.  max_splits bounds it by the workspace.
-void tile_split_plan(const BatchParams &p, int64_t groups, int max_splits, bool must_reduce, int &splits,
-                     int &per_split) {
-    constexpr double kBlockUs = 2.5, kWideUs = 3.4, kPartialUsPerMb = 0.4, kReduceUs = 4.;
-    const int64_t cus = device_info().cus, wide = (p.tiles + 1) / 2 * groups;
-    double block_us = 0., out_mb = 0.;
-    for (int i = 0; i < p.n_mats; ++i) {
-        block_us = std::max(block_us, p.mat[i].type == QK_TYPE_Q4_K ? kBlockUs : kWideUs);
-        out_mb += 4e-6 * p.mat[i].rows * p.n_tokens;
-    }
-    double best = 0.;
-    for (int s = 1; s <= std::min(std::min(max_splits, kMaxSplit), p.nb); ++s) {
-        const int per = (p.nb + s - 1) / s;
-        if ((p.nb + per - 1) / per != s) continue;
-        const int64_t wgs = wide * s, rest = wgs % (2 * cus);
-        const double rounds = 2. * static_cast<double>(wgs / (2 * cus)) + (rest > cus ? 2. : rest > 0 ? 1. : 0.);
-        const double us = rounds * per * block_us + (s > 1 || must_reduce ? s * out_mb * kPartialUsPerMb : 0.) +
-                          (s > 1 && !must_reduce ? kReduceUs : 0.);
-        if (best == 0. || us < best) {
-            best = us;
-            splits = s;
-            per_split = per;
-        }
-    }
 }
 
 int launch_mfma(const qk_matrix *mats, int n_mats, const int *ldy, const float *x, int ldx, int cols, int n_tokens,
@@ -908,9 +936,21 @@ int launch_mfma(const qk_matrix *mats, int n_mats, const int *ldy, const float *
     if (tiles == 1) {
         split_plan(groups, nb, tiles, p.splits, p.blocks_per_split);
     } else {
-        const size_t slot = static_cast<size_t>(groups) * tiles * kPartialFloats * sizeof(float);
-        const int fit = static_cast<int>(std::min<size_t>(kMaxSplit, (workspace_size - rec_bytes) / slot));
-        tile_split_plan(p, groups, std::max(fit, 1), must_reduce, p.splits, p.blocks_per_split);
+        int64_t rows_total = 0;
+        bool wide = false;
+        for (int i = 0; i < n_mats; ++i) {
+            rows_total += mats[i].rows;
+            wide |= mats[i].type != QK_TYPE_Q4_K;
+        }
+        tile_split_plan(groups, rows_total, nb, n_tokens, wide, must_reduce, kMaxSplit, p.splits, p.blocks_per_split);
+        // Less than the queried size that still holds what it has to: the
+        // splits that fit.
+        const size_t room = workspace_size - rec_bytes;
+        if (p.splits > 1 && tile_partial_bytes(groups, tiles, p.splits) > room) {
+            const int fit = static_cast<int>(room / tile_partial_bytes(groups, tiles, 1));
+            tile_split_plan(groups, rows_total, nb, n_tokens, wide, must_reduce, std::max(fit, 1), p.splits,
+                            p.blocks_per_split);
+        }
     }
     const bool need_partials = p.splits > 1 || must_reduce;
     p.records = ws;
@@ -964,7 +1004,7 @@ size_t ffn_shared_bytes(int dim, int hidden, int n_tokens) {
     size_t ws = 0;
     for (int tq = 1; tq <= tile_count(n_tokens); ++tq) {
         const int n = std::min(n_tokens, std::max(kMfmaMinTokens, tq * kTokTile));
-        ws = std::max({ws, workspace_bound(dim, 2 * hidden, n, true), workspace_bound(hidden, dim, n)});
+        ws = std::max({ws, least_bound(dim, 2 * hidden, n, true), least_bound(hidden, dim, n)});
     }
     return (ws + 255) / 256 * 256;
 }
@@ -972,6 +1012,18 @@ size_t ffn_shared_bytes(int dim, int hidden, int n_tokens) {
 // Below kMfmaMinTokens: the gate and up outputs, each 256-byte aligned.
 size_t ffn_gemv_slot(int hidden, int n_tokens) {
     return (static_cast<size_t>(n_tokens) * hidden * sizeof(float) + 255) / 256 * 256;
+}
+
+// The same with room for both products' plans (monotonic in the tokens).
+size_t ffn_planned_bytes(int dim, int hidden, int n_tokens, size_t shared) {
+    return std::max({shared, (plan_bytes(dim, 2 * hidden, n_tokens, true) + 255) / 256 * 256,
+                     (plan_bytes(hidden, dim, n_tokens, false) + 255) / 256 * 256});
+}
+
+// A call's workspace around the shared part.  Also enough for any smaller call:
+// the GEMV form's gate and up outputs.
+size_t ffn_bytes(int hidden, int n_tokens, size_t shared) {
+    return std::max(shared + (records_bytes(hidden, n_tokens) + 255) / 256 * 256, 2 * ffn_gemv_slot(hidden, kMfmaMinTokens - 1));
 }
 
 int launch_batched_fused(const qk_matrix *mats, int n_mats, const float *x, int ldx, int cols, int n_tokens,
@@ -1015,9 +1067,8 @@ int qk_gemv_batched_f32(int type, const void *w, const float *x, int ldx, float 
 size_t qk_ffn_batched_workspace_bytes(int dim, int hidden, int n_tokens) {
     if (dim <= 0 || hidden <= 0 || n_tokens <= 0 || dim % 256 || hidden % 256) return 0;
     if (n_tokens < qk::kMfmaMinTokens) return 2 * qk::ffn_gemv_slot(hidden, n_tokens);
-    // Also enough for any smaller call: the GEMV form's gate and up outputs.
-    return std::max(qk::ffn_shared_bytes(dim, hidden, n_tokens) + (qk::records_bytes(hidden, n_tokens) + 255) / 256 * 256,
-                    2 * qk::ffn_gemv_slot(hidden, qk::kMfmaMinTokens - 1));
+    return qk::ffn_bytes(hidden, n_tokens,
+                         qk::ffn_planned_bytes(dim, hidden, n_tokens, qk::ffn_shared_bytes(dim, hidden, n_tokens)));
 }
 
 int qk_ffn_batched_f32(int gate_type, const void *gate, int up_type, const void *up, int down_type, const void *down,
@@ -1033,7 +1084,9 @@ int qk_ffn_batched_f32(int gate_type, const void *gate, int up_type, const void 
     if (!y || ldy < dim) return qk::fail(QK_ERR_INVALID_ARG, "qk_ffn_batched_f32: null y or ldy smaller than dim");
     if (!qk::aligned(y, 4)) return qk::fail(QK_ERR_ALIGN, "qk_ffn_batched_f32: y must be 4-byte aligned");
     if (n_tokens == 0) return qk::ok();
-    const size_t need = qk_ffn_batched_workspace_bytes(dim, hidden, n_tokens);
+    const bool mfma = n_tokens >= qk::kMfmaMinTokens;
+    size_t shared = mfma ? qk::ffn_shared_bytes(dim, hidden, n_tokens) : 0;
+    const size_t need = mfma ? qk::ffn_bytes(hidden, n_tokens, shared) : 2 * qk::ffn_gemv_slot(hidden, n_tokens);
     if (!workspace || workspace_bytes < need)
         return qk::fail(QK_ERR_INVALID_ARG, "qk_ffn_batched_f32: workspace smaller than " + std::to_string(need) +
                                                 " bytes (qk_ffn_batched_workspace_bytes)");
@@ -1066,7 +1119,8 @@ int qk_ffn_batched_f32(int gate_type, const void *gate, int up_type, const void 
     }
     // Matrix cores: gate / up's reduction writes the records of SiLU(gate) *
     // up (gate and up themselves are never stored), which down reads.
-    const size_t shared = qk::ffn_shared_bytes(dim, hidden, n_tokens);
+    const size_t planned = qk::ffn_planned_bytes(dim, hidden, n_tokens, shared);
+    if (workspace_bytes >= qk::ffn_bytes(hidden, n_tokens, planned)) shared = planned;
     uint8_t *rec = ws + shared;
     const qk_matrix gu[2] = {{gate_type, hidden, gate, y}, {up_type, hidden, up, y}};
     const int ldg[2] = {hidden, hidden};

@@ -155,7 +155,7 @@ int launch_gemv_i8_pair_quant(const qk_matrix *gu, const float *x, int ldx, cons
 // longer than 2048 columns are split over workgroups whose sums a second
 // launch adds: the workspace holds them (skinny_i8_workspace_bytes of the
 // launch's row tiles: sum of ceil(rows / 32), or rows / 32 for a pair).
-size_t skinny_i8_workspace_bytes(int cols, int tiles, int n_tokens, bool pair);
+size_t skinny_i8_workspace_bytes(int cols, int tiles, int n_tokens, bool pair, bool plans = true);
 // The next RMSNorm + quantization of an accumulating one-matrix launch's
 // output rows, folded into its split reduction: x (the launch's y) as
 // rmsnorm_quantize_kernel would normalise it with w, into xq [token][ldxq]
@@ -189,12 +189,13 @@ int launch_skinny_i8(const qk_matrix *mats, int n_mats, const int *ldy, const in
                      hipStream_t stream, const char *where, const SkNorm *norm = nullptr,
                      SkDeferred *defer = nullptr);
 // The same product of many tokens on the fp16 matrix cores
-// (csrc/qk_tile_i8.hip).  tile_i8_splits: the splits of the rows (their sums
-// within workspace_size bytes), or 0 where launch_skinny_i8's own kernels are
+// (csrc/qk_tile_i8.hip).  tile_i8_splits: the splits of the rows (by the call
+// alone from tile_i8_workspace_bytes on, else those that fit), or 0 where launch_skinny_i8's own kernels are
 // the better choice.  Matrices of one type; out_xq 4-byte aligned, out_ldxq a
 // multiple of 4.
 int tile_i8_splits(const qk_matrix *mats, int n_mats, int cols, int n_tokens, int ldxq, int ldscale, bool pair,
                    size_t workspace_size);
+size_t tile_i8_workspace_bytes(int cols, int tiles, int n_tokens);
 int launch_tile_i8(int splits, const qk_matrix *mats, int n_mats, const int *ldy, const int8_t *xq, int ldxq,
                    const float *xscale, int ldscale, int cols, int n_tokens, int accumulate, int8_t *out_xq,
                    float *out_xs, int out_ldxq, int out_ldxs, void *workspace, hipStream_t stream, const char *where);

@@ -854,14 +854,17 @@ int row_tiles(const qk_matrix *mats, int n_mats, bool pair) {
 // Workspace bound of a launch, for any storage type: the split sums of
 // the fewest splits of the narrowest workgroups (the looping kernel's), or
 // of the planner's extra splits (at most kPartialUnitsMax units).
-size_t skinny_i8_workspace_bytes(int cols, int tiles, int n_tokens, bool pair) {
+// With `plans` also what tile_i8_splits' choice takes, so that a launch with
+// this much need not look at the size.
+size_t skinny_i8_workspace_bytes(int cols, int tiles, int n_tokens, bool pair, bool plans) {
     const int nb = cols / 256;
     if (nb <= 1 || n_tokens <= 0 || tiles <= 0) return 0;
     const int64_t units = static_cast<int64_t>(tiles) * ((n_tokens + kToks - 1) / kToks);
     const int s0 = fewest_splits(nb, kLoopWaves);
     const int64_t sums = std::max<int64_t>(s0 > 1 ? units * s0 : 0,
                                            std::min<int64_t>(units * std::min(nb, kSplitsMax), kPartialUnitsMax));
-    return static_cast<size_t>(sums) * (pair ? 2 : 1) * 1024 * sizeof(float);
+    const size_t bytes = static_cast<size_t>(sums) * (pair ? 2 : 1) * 1024 * sizeof(float);
+    return plans && !pair ? std::max(bytes, tile_i8_workspace_bytes(cols, tiles, n_tokens)) : bytes;
 }
 
 // The INT8 product of n_tokens per-32 quantized activation rows with
@@ -1001,12 +1004,12 @@ size_t al256(size_t b) { return (b + 255) / 256 * 256; }
 // hidden / 32 scales per token, each array 256-byte aligned), then the
 // split sums of the two products (the larger); below kMatrixCoreTokens the
 // fp32 gate and up outputs of the GEMV form instead.
-size_t ffn_i8_bytes(int dim, int hidden, int n_tokens) {
+size_t ffn_i8_bytes(int dim, int hidden, int n_tokens, bool plans) {
     const size_t t = static_cast<size_t>(n_tokens);
     const size_t h = al256(t * hidden) + al256(t * (hidden / 32) * sizeof(float));
     if (n_tokens < kMatrixCoreTokens) return h + 2 * al256(t * hidden * sizeof(float));
-    return h + std::max(qk::skinny_i8_workspace_bytes(dim, hidden / 32, n_tokens, true),
-                        qk::skinny_i8_workspace_bytes(hidden, (dim + 31) / 32, n_tokens, false));
+    return h + std::max(qk::skinny_i8_workspace_bytes(dim, hidden / 32, n_tokens, true, plans),
+                        qk::skinny_i8_workspace_bytes(hidden, (dim + 31) / 32, n_tokens, false, plans));
 }
 
 }  // namespace
@@ -1064,8 +1067,8 @@ size_t qk_ffn_batched_i8_workspace_bytes(int dim, int hidden, int n_tokens) {
     if (dim <= 0 || dim % 256 || hidden <= 0 || hidden % 256 || n_tokens <= 0) return 0;
     // Enough for any token count up to n_tokens: each form's need grows
     // with the count, so the larger of the two forms' needs covers both.
-    return std::max(ffn_i8_bytes(dim, hidden, n_tokens),
-                    ffn_i8_bytes(dim, hidden, std::min(n_tokens, kMatrixCoreTokens - 1)));
+    return std::max(ffn_i8_bytes(dim, hidden, n_tokens, true),
+                    ffn_i8_bytes(dim, hidden, std::min(n_tokens, kMatrixCoreTokens - 1), true));
 }
 
 int qk_ffn_batched_i8(int gate_type, const void *gate, int up_type, const void *up, int down_type, const void *down,
@@ -1084,7 +1087,7 @@ int qk_ffn_batched_i8(int gate_type, const void *gate, int up_type, const void *
     if (!y || ldy < dim) return qk::fail(QK_ERR_INVALID_ARG, "qk_ffn_batched_i8: null y or ldy smaller than dim");
     if (!qk::aligned(y, 4)) return qk::fail(QK_ERR_ALIGN, "qk_ffn_batched_i8: y must be 4-byte aligned");
     if (n_tokens == 0) return qk::ok();
-    const size_t need = ffn_i8_bytes(dim, hidden, n_tokens);
+    const size_t need = ffn_i8_bytes(dim, hidden, n_tokens, false);
     if (!workspace || workspace_bytes < need)
         return qk::fail(QK_ERR_INVALID_ARG, "qk_ffn_batched_i8: workspace smaller than " + std::to_string(need) +
                                                 " bytes (qk_ffn_batched_i8_workspace_bytes)");

@@ -52,6 +52,7 @@ constexpr int kTok = 32, kRowTile = 32;
 constexpr int kPairRows = 64, kStoreRows = 128;   // weight rows of a workgroup (of each matrix of a pair)
 constexpr int kHalfTile = 8 * 1024;                // one token tile's half block: 4 sub-blocks x 2 operands x 1 KB
 constexpr int kMaxSplits = 8;
+constexpr int kMaxItems = 2048;   // workgroups of a split launch at most: bounds the sums to 64 MB
 
 struct TiMatrix {
     const uint8_t *w;
@@ -534,6 +535,12 @@ void launch(int type, const TiParams &p, hipStream_t stream) {
 
 }  // namespace
 
+// Without a pair, few tokens leave part of a token group empty and the sum
+// traffic outweighs the gain: Q4_K 8192 x 3072 takes 33 / 41 us here and 26 /
+// 37 there on 96 / 130 tokens, 46 and 51 on 256; Q6_K 40 and 36 on 96, 49 and
+// 50 on 130; rows of 14336 gain from 40 tokens on (38 and 56).
+static int least_tokens(bool q4, int nb) { return q4 ? 192 : nb > 32 ? 0 : 128; }
+
 // Splits of least modelled time: a block takes a workgroup kBlockUs[r] with r
 // workgroups on its CU (measured, Q4_K), split sums their traffic and a
 // launch.  A pair is not split: its epilogue needs whole sums.  Launches of
@@ -544,12 +551,10 @@ int tile_i8_splits(const qk_matrix *mats, int n_mats, int cols, int n_tokens, in
     // A 64-token tile's offsets are 32 bits.
     if (ldxq >= 1 << 26 || ldscale >= 1 << 24) return 0;
     const int nb = cols / 256, cus = std::max(1, device_info().cus);
-    // Without a pair, few tokens leave part of a token group empty and the sum
-    // traffic outweighs the gain: Q4_K 8192 x 3072 takes 33 / 41 us here and 26
-    // / 37 there on 96 / 130 tokens, 46 and 51 on 256; Q6_K 40 and 36 on 96, 49
-    // and 50 on 130; rows of 14336 gain from 40 tokens on (38 and 56).
-    if (!pair && n_tokens < (mats[0].type == QK_TYPE_Q4_K ? 192 : nb > 32 ? 0 : 128)) return 0;
-    int groups = 0, part_rows = 0;
+    const bool q4 = mats[0].type == QK_TYPE_Q4_K;
+    if (!pair && n_tokens < least_tokens(q4, nb)) return 0;
+    int groups = 0;
+    size_t part_rows = 0;
     for (int i = 0; i < (pair ? 1 : n_mats); ++i) {
         groups += (mats[i].rows + (pair ? kPairRows : kStoreRows) - 1) / (pair ? kPairRows : kStoreRows);
         part_rows += (mats[i].rows + kRowTile - 1) / kRowTile * kRowTile;
@@ -557,24 +562,40 @@ int tile_i8_splits(const qk_matrix *mats, int n_mats, int cols, int n_tokens, in
     const int64_t items = static_cast<int64_t>(groups) * ((n_tokens + 2 * kTok - 1) / (2 * kTok));
     if (items * kMaxSplits > (1 << 30)) return 0;
     constexpr double kBlockUs[3] = {2.4, 3.8, 5.5}, kReduceUs = 4., kSumUsPerMb = 0.4;
-    const double mb = 1e-6 * n_tokens * part_rows * sizeof(float);
-    int best = 0;
-    double least = 0;
-    for (int s = 1; s <= (pair ? 1 : std::min(nb, kMaxSplits)); ++s) {
-        if (s > 1 && mb * s > 1e-6 * static_cast<double>(workspace_size)) break;
-        if (items * s < cus) continue;
-        const int per = (nb + s - 1) / s;
-        const int resident = per > (mats[0].type == QK_TYPE_Q4_K ? kShortBlocks<QK_TYPE_Q4_K> : kShortBlocks<QK_TYPE_Q6_K>)
-                                 ? 2 : 3;
-        const int64_t wgs = items * s, full = wgs / (resident * cus), rest = wgs % (resident * cus);
-        const double us = per * (full * kBlockUs[resident - 1] + (rest ? kBlockUs[(rest - 1) / cus] : 0.)) +
-                          (s > 1 ? kReduceUs + kSumUsPerMb * mb * s : 0.);
-        if (!best || us < least) {
-            best = s;
-            least = us;
+    const size_t bytes = part_rows * n_tokens * sizeof(float);
+    const double mb = 1e-6 * static_cast<double>(bytes);
+    auto least_of = [&](int max_splits) {
+        int best = 0;
+        double least = 0;
+        for (int s = 1; s <= max_splits; ++s) {
+            if (items * s < cus || (s > 1 && items * s > kMaxItems)) continue;
+            const int per = (nb + s - 1) / s;
+            const int resident = per > (q4 ? kShortBlocks<QK_TYPE_Q4_K> : kShortBlocks<QK_TYPE_Q6_K>) ? 2 : 3;
+            const int64_t wgs = items * s, full = wgs / (resident * cus), rest = wgs % (resident * cus);
+            const double us = per * (full * kBlockUs[resident - 1] + (rest ? kBlockUs[(rest - 1) / cus] : 0.)) +
+                              (s > 1 ? kReduceUs + kSumUsPerMb * mb * s : 0.);
+            if (!best || us < least) {
+                best = s;
+                least = us;
+            }
         }
-    }
-    return best;
+        return best;
+    };
+    const int best = least_of(pair ? 1 : std::min(nb, kMaxSplits));
+    // Less than the queried size: the splits that fit.
+    return best > 1 && best * bytes > workspace_size ? least_of(static_cast<int>(workspace_size / bytes)) : best;
+}
+
+// Bytes that tile_i8_splits' choice takes, for any types and any division of
+// `tiles` 32-row tiles over matrices, at this token count and below: splits *
+// tokens is at most kMaxSplits times them, and kMaxItems workgroups' tokens.
+size_t tile_i8_workspace_bytes(int cols, int tiles, int n_tokens) {
+    const int nb = cols / 256;
+    if (n_tokens < std::min(least_tokens(true, nb), least_tokens(false, nb))) return 0;
+    const int64_t groups = (static_cast<int64_t>(tiles) * kRowTile + kStoreRows - 1) / kStoreRows;
+    const int64_t split_tokens = std::min<int64_t>(static_cast<int64_t>(std::min(nb, kMaxSplits)) * n_tokens,
+                                                   kMaxItems / std::max<int64_t>(1, groups - QK_MAX_FUSED) * 2 * kTok);
+    return static_cast<size_t>(split_tokens) * tiles * kRowTile * sizeof(float);
 }
 
 int launch_tile_i8(int splits, const qk_matrix *mats, int n_mats, const int *ldy, const int8_t *xq, int ldxq,

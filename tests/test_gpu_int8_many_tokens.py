@@ -14,6 +14,7 @@ import pytest
 
 from conftest import rel_l2, to_dev
 from test_gpu_int8_matrix_core import Q4_K, Q6_K, _integer_blocks
+from test_gpu_tile_gemm import sizes_of
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +132,53 @@ def test_ffn(qk, torch_gpu, synth, down, dim, hidden, ntok):
         # group's peak (some three times its RMS): sqrt(127 * 2^-20) * 3 / 127
         # = 2.6e-4 of the whole.
         assert rel_l2(y.cpu().numpy(), ref.numpy()) < 5e-4
+
+
+@pytest.mark.parametrize("qtype,cols,rows,ntok", [(Q4_K, 8192, 3072, 256), (Q6_K, 8192, 2048, 300), (Q6_K, 5632, 2048, 400)])
+def test_bits_do_not_depend_on_a_larger_workspace(qk, torch_gpu, synth, qtype, cols, rows, ntok):
+    """The queried size and a larger one give the same bits; the least size that
+    is accepted holds fewer splits."""
+    t = torch_gpu
+    g = t.Generator().manual_seed(19)
+    w = to_dev(t, synth.quant_matrix(qtype, cols, rows, 15, 1))
+    xq = t.randint(-127, 128, (ntok, cols), generator=g, dtype=t.int8).cuda()
+    xs = (t.rand(ntok, cols // 32, generator=g) * 1e-2).cuda()
+    L = qk.lib()
+    query = L.qk_gemv_batched_i8_workspace_bytes(cols, rows, ntok)
+    ws = t.empty(query + (64 << 20), dtype=t.uint8, device="cuda")
+
+    def call(n):
+        y = t.empty(ntok, rows, device="cuda")
+        qk.check(L.qk_gemv_batched_i8(qtype, w.data_ptr(), xq.data_ptr(), cols, xs.data_ptr(), cols // 32, y.data_ptr(),
+                                      rows, cols, rows, ntok, ws.data_ptr(), n, None), "batched INT8")
+        t.cuda.synchronize()
+        return y.cpu().numpy()
+
+    queried, more, least = (call(n) for n in sizes_of(qk, call, query))
+    assert np.array_equal(queried, more)
+    assert rel_l2(least, queried) < 1e-6
+
+
+def test_ffn_bits_do_not_depend_on_a_larger_workspace(qk, torch_gpu, synth):
+    t = torch_gpu
+    dim, hidden, ntok = 2048, 8192, 256
+    g = t.Generator().manual_seed(23)
+    w = [to_dev(t, synth.quant_matrix(ty, c, r, 16, i)) for i, (ty, c, r) in
+         enumerate([(Q4_K, dim, hidden), (Q4_K, dim, hidden), (Q6_K, hidden, dim)])]
+    xq = t.randint(-127, 128, (ntok, dim), generator=g, dtype=t.int8).cuda()
+    xs = (t.rand(ntok, dim // 32, generator=g) * 2e-4).cuda()
+    L = qk.lib()
+    query = L.qk_ffn_batched_i8_workspace_bytes(dim, hidden, ntok)
+    ws = t.empty(query + (64 << 20), dtype=t.uint8, device="cuda")
+
+    def call(n):
+        y = t.empty(ntok, dim, device="cuda")
+        qk.check(L.qk_ffn_batched_i8(Q4_K, w[0].data_ptr(), Q4_K, w[1].data_ptr(), Q6_K, w[2].data_ptr(), xq.data_ptr(),
+                                     dim, xs.data_ptr(), dim // 32, y.data_ptr(), dim, dim, hidden, ntok, 0,
+                                     ws.data_ptr(), n, None), "INT8 FFN")
+        t.cuda.synchronize()
+        return y.cpu().numpy()
+
+    queried, more, least = (call(n) for n in sizes_of(qk, call, query))
+    assert np.array_equal(queried, more)
+    assert rel_l2(least, queried) < 1e-6

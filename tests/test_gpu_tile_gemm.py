@@ -2,6 +2,8 @@
 the edges of its tiles: token counts around multiples of 32 and 64, row counts
 around multiples of 32 and 128, one block and odd block counts, every storage
 type alone and mixed in one launch, with and without split sums."""
+import re
+
 import numpy as np
 import pytest
 
@@ -111,3 +113,53 @@ def test_error_of_long_rows(qk, torch_gpu, workloads, synth, qtype):
         return float((y.double() - want).norm() / want.norm())
 
     assert error(ntok) < 1.02 * error(32)
+
+
+def sizes_of(qk, call, query):
+    """The queried size, more, and the least size the call takes."""
+    with pytest.raises(qk.QKError) as e:
+        call(256)
+    least = int(re.search(r"smaller than (\d+) bytes", str(e.value))[1])
+    assert least <= query
+    return query, query + (64 << 20), least
+
+
+@pytest.mark.parametrize("ntok,cols,rows", [(40, 4096, 200), (97, 8192, 640), (256, 2048, 512)])
+def test_bits_do_not_depend_on_a_larger_workspace(qk, torch_gpu, workloads, synth, ntok, cols, rows):
+    t = torch_gpu
+    ten, _, _ = matrix(qk, t, workloads, synth, Q4_K, cols, rows, 51)
+    x = to_dev(t, synth.normal_f32(ntok * cols, 34, ntok))
+    query = qk.batch_workspace_bytes(cols, rows, ntok)
+    ws = t.empty(query + (64 << 20), dtype=t.uint8, device="cuda")
+
+    def call(n):
+        y = t.empty((ntok, rows), device="cuda")
+        qk.check(qk.lib().qk_gemv_batched_f32(Q4_K, ten.gpu, x.data_ptr(), cols, y.data_ptr(), rows, cols, rows, ntok,
+                                              ws.data_ptr(), n, None), "batched")
+        t.cuda.synchronize()
+        return y.cpu().numpy()
+
+    queried, more, least = (call(n) for n in sizes_of(qk, call, query))
+    assert np.array_equal(queried, more)
+    assert rel_l2(least, queried) < TOL
+
+
+@pytest.mark.parametrize("ntok,dim,hidden", [(64, 1024, 2816), (130, 3072, 8192)])
+def test_ffn_bits_do_not_depend_on_a_larger_workspace(qk, torch_gpu, workloads, synth, ntok, dim, hidden):
+    t = torch_gpu
+    g, u, d = (matrix(qk, t, workloads, synth, Q4_K, c, r, 52 + i)[0]
+               for i, (c, r) in enumerate([(dim, hidden), (dim, hidden), (hidden, dim)]))
+    x = to_dev(t, synth.normal_f32(ntok * dim, 35, ntok) * np.float32(0.05))
+    query = qk.lib().qk_ffn_batched_workspace_bytes(dim, hidden, ntok)
+    ws = t.empty(query + (64 << 20), dtype=t.uint8, device="cuda")
+
+    def call(n):
+        y = t.empty((ntok, dim), device="cuda")
+        qk.check(qk.lib().qk_ffn_batched_f32(Q4_K, g.gpu, Q4_K, u.gpu, Q4_K, d.gpu, x.data_ptr(), dim, y.data_ptr(), dim,
+                                             dim, hidden, ntok, 0, ws.data_ptr(), n, None), "ffn")
+        t.cuda.synchronize()
+        return y.cpu().numpy()
+
+    queried, more, least = (call(n) for n in sizes_of(qk, call, query))
+    assert np.array_equal(queried, more)
+    assert rel_l2(least, queried) < 4 * TOL
