@@ -546,15 +546,14 @@ __device__ __forceinline__ TokenTile token_tile(const qk_batch_token *desc, int 
 }
 
 // The tile kernel serves a's layout (head_dim 64 or 128, caches already
-// holding every row); takes less time than the per-token form for n_tokens
-// tokens of `rows` rows in all, the longest max_rows; runs.
+// holding every row).  A call that knows its shape only: whether tiles are
+// tried (each one's descriptors decide).
 bool tile_attention_supported(const SplitAttention &a);
-bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int64_t max_rows,
-                         bool two_runs);
+bool tile_attention_call(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim);
 int launch_tile_attention(const SplitAttention &a, hipStream_t stream);
 // SplitAttention::tile_mode of a batch whose descriptors the host holds
-// (valid ones): by the tiles' own test, when it pays.  Sets a.rows_hint to
-// the rows left to the per-token form.
+// (valid ones): by the tiles' own test, when it pays.  Sets a.tile_runs, and
+// a.rows_hint to the rows left to the per-token form.
 int tile_attention_mode(const qk_batch_token *desc, SplitAttention &a);
 
 // RoPE of q and k at each token's position, k and v written to row kv_row +
@@ -767,3 +766,6 @@ int launch_embedding_records(int type, const void *w, const int32_t *token, int 
 int launch_q6k_join(const void *src, void *dst, int cols, int rows, hipStream_t stream);
 
 }  // namespace qk
+
+// Dispatch rules by plain arguments: the tests ask them which form a call takes.
+extern "C" int qk_rule_tile_attention(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim);

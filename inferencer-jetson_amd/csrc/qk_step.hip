@@ -866,19 +866,10 @@ const void *split_merge_instance(int G) {
 
 inline hipStream_t S(qk_stream s) { return static_cast<hipStream_t>(s); }
 
-// tile_mode of a call whose descriptors are on the device: n tokens of
-// sequences of their own hold at most cache_rows rows together, so when
-// n * (max_pos + 1) is far beyond that, tokens share rows (a prefill chunk) and
-// the tile kernel goes first; each tile's descriptors decide.  A decode batch
-// stays below it and launches no tile kernel.  Sixteen tokens a row on average
-// keep a tile to two runs; a cache of more rows than one sequence may hold
-// several, and then the tile of two runs, which walks both, sets the time.
+// tile_mode of a call whose descriptors are on the device.
 int call_tile_mode(const SplitAttention &a) {
-    const int64_t rows = static_cast<int64_t>(a.n_tokens) * (a.max_pos + 1);
-    const int runs = a.cache_rows > a.max_pos + 1 ? 2 : 1;
-    return rows / 16 >= a.cache_rows && tile_attention_supported(a) &&
-           tile_attention_pays(a.n_tokens, a.kv_heads, a.heads, a.head_dim, rows / 4 * 3,
-                               static_cast<int64_t>(runs) * (a.max_pos + 1), runs > 1);
+    return tile_attention_supported(a) &&
+           tile_attention_call(a.n_tokens, a.max_pos, a.cache_rows, a.heads, a.kv_heads, a.head_dim);
 }
 
 }  // namespace

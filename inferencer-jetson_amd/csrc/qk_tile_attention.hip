@@ -361,56 +361,79 @@ bool tile_attention_supported(const SplitAttention &a) {
            (!a.gemm_rec || G * a.head_dim % 256 == 0) && (!a.q8_out || aligned(a.q8_out, 4));
 }
 
-// Whether 16-token tiles take less time than reading every token's rows, both
-// estimated.  Tiles: rounds of one workgroup per CU, each walking ceil(rows /
-// 32 / S) row tiles in 2.4 us per wave of a SIMD at head_dim 128 (half that at
-// 64), and 12 us of launch, ramp and merge.  Per token: 6 ns a (token, KV
-// head) and the rows through L2 at 20 TB/s.  Both within a fifth of what 100
-// to 1024 tokens over 128 to 4096 rows measured on either layout, so the
-// tiles have to be a tenth shorter.  One query head a KV head leaves a SIMD one
-// wave, 3.7 us a step.  Where tiles may hold two runs, the second one's start
-// adds 12 us and the margin is three tenths (8 heads of 128, 4 x 58 tokens over
-// 450 rows: 34.5 us per token, 53 in tiles).
-bool tile_attention_pays(int n_tokens, int kv_heads, int heads, int head_dim, int64_t rows, int64_t max_rows,
-                         bool two_runs) {
+namespace {
+
+// Estimated times of both forms.  Tiles: rounds of one workgroup (16-token tile
+// or run, KV head) per CU, each walking ceil(rows / 32 / S) row tiles in 2.4 us
+// per wave of a SIMD at head_dim 128 (half that at 64; one query head a KV head
+// leaves a SIMD one wave, 3.8 and 2.2 us), and 12 us of launch, ramp, merge and
+// the other form's launch.  Per token: 6 ns a (token, KV head) and the rows
+// through L2 at 20 TB/s.  Both within a fifth of what 128 to 1024 tokens of one
+// sequence over 128 to 4096 rows measured (64 over 8 heads excepted, whose
+// per-token form takes twice that), so the tiles have to be a tenth shorter.
+double tile_us(int64_t workgroups, int heads, int kv_heads, int head_dim, int64_t max_rows, double step_factor) {
     const int G = heads / kv_heads, S = tile_groups(G, head_dim);
-    const int64_t wgs = static_cast<int64_t>((n_tokens + kAttnTile - 1) / kAttnTile) * kv_heads;
-    const int64_t rounds = (wgs + device_info().cus - 1) / device_info().cus;
+    const int64_t rounds = (workgroups + device_info().cus - 1) / device_info().cus;
     const int64_t steps = ((max_rows + kKeys - 1) / kKeys + S - 1) / S;
-    const double step_us = std::max(3.7, 2.4 * ((G * S + 3) / 4)) * head_dim / 128.;
-    const double tile_us = (two_runs ? 24. : 12.) + static_cast<double>(rounds * steps) * step_us;
-    const double split_us = 6e-3 * n_tokens * kv_heads + static_cast<double>(rows) * kv_heads * head_dim * 8. / 20e6;
-    return (two_runs ? 1.3 : 1.1) * tile_us < split_us;
+    const double step = std::max(head_dim == 64 ? 4.4 : 3.8, 2.4 * ((G * S + 3) / 4)) * head_dim / 128.;
+    return 12. + static_cast<double>(rounds * steps) * step * step_factor;
+}
+double per_token_us(int64_t n_tokens, int kv_heads, int head_dim, int64_t rows) {
+    return 6e-3 * static_cast<double>(n_tokens * kv_heads) + static_cast<double>(rows) * kv_heads * head_dim * 8. / 20e6;
+}
+constexpr double kMargin = 1.1;
+
+}  // namespace
+
+// A call whose descriptors are on the device, row-major caches.  Tokens of
+// sequences of their own hold at most cache_rows rows together, so with n *
+// (max_pos + 1) far beyond that they share rows, about that many to a row; each
+// tile's descriptors decide.  A decode batch stays below, unless one sequence is
+// many times as long as the rest.
+//   * Sixteen tokens a row keep tiles to two runs, and a launch in vain costs 4
+//     us; where reading the rows per token takes 100 us and more, four tokens a
+//     row are enough (a cache with room to spare shows no more).
+//   * A cache of more rows than one sequence may hold several: then a step takes
+//     twice the time (rows 2 KB apart share few sets of an XCD's L2: 2 x 256
+//     tokens over 800 rows 77 us, over the same rows 45; 4 x 128 over 600, 63).
+// Measured with this rule, 24 over 8 heads of 128: 512 tokens over 1112 rows 166
+// -> 82 us at 1112 to 65536 cache rows; 4 x 128 over 600 116 -> 91; 4 x 58 over
+// 450 and 300 decoding sequences stay per token (53 against 54, 120 against 123).
+bool tile_attention_call(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim) {
+    const int64_t rows = static_cast<int64_t>(n_tokens) * (max_pos + 1);
+    const double per_token = per_token_us(n_tokens, kv_heads, head_dim, rows / 4 * 3);
+    if (rows / (per_token < 100. ? 16 : 4) < cache_rows) return false;
+    const int64_t wgs = static_cast<int64_t>((n_tokens + kAttnTile - 1) / kAttnTile) * kv_heads;
+    return kMargin * tile_us(wgs, heads, kv_heads, head_dim, max_pos + 1, cache_rows > max_pos + 1 ? 2. : 1.) < per_token;
 }
 
 int tile_attention_mode(const qk_batch_token *desc, SplitAttention &a) {
     if (!tile_attention_supported(a)) return 0;
-    int64_t tiled_rows = 0, rows = 0, max_rows = 0;
+    int64_t tiled_rows = 0, rows = 0, max_rows = 0, workgroups = 0;
     int tiled = 0;
-    bool two_runs = false;
+    a.tile_runs = 1;
     for (int t0 = 0; t0 < a.n_tokens; t0 += kAttnTile) {
         const int t1 = std::min(t0 + kAttnTile, a.n_tokens);
         int runs = 0;
-        int64_t walked = 0;   // rows the tile's workgroup walks: each run's last position
-        int64_t tile_rows = 0;
+        int64_t tile_rows = 0, longest = 0;
         for (int t = t0; t < t1; ++t) {
             runs += t == t0 || desc[t].kv_row != desc[t - 1].kv_row || desc[t].pos != desc[t - 1].pos + 1;
             tile_rows += desc[t].pos + 1;
-            if (t + 1 == t1 || desc[t + 1].kv_row != desc[t].kv_row || desc[t + 1].pos != desc[t].pos + 1)
-                walked += desc[t].pos + 1;
+            longest = std::max<int64_t>(longest, desc[t].pos + 1);
         }
         if (runs <= kMaxRuns) {
             tiled += t1 - t0;
             tiled_rows += tile_rows;
-            max_rows = std::max(max_rows, walked);
-            two_runs |= runs > 1;
+            max_rows = std::max(max_rows, longest);
+            workgroups += static_cast<int64_t>(runs) * a.kv_heads;
+            if (runs > 1) a.tile_runs = kMaxRuns;
         } else {
             rows += tile_rows;
         }
     }
-    if (!tiled || !tile_attention_pays(tiled, a.kv_heads, a.heads, a.head_dim, tiled_rows, max_rows, two_runs))
+    if (!tiled || kMargin * tile_us(workgroups, a.heads, a.kv_heads, a.head_dim, max_rows, 1.) >=
+                      per_token_us(tiled, a.kv_heads, a.head_dim, tiled_rows))
         return 0;
-    a.tile_runs = two_runs ? kMaxRuns : 1;
     if (tiled == a.n_tokens) return 2;
     a.rows_hint = rows;
     return 1;
@@ -433,3 +456,7 @@ int launch_tile_attention(const SplitAttention &a, hipStream_t stream) {
 }
 
 }  // namespace qk
+
+extern "C" int qk_rule_tile_attention(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim) {
+    return qk::tile_attention_call(n_tokens, max_pos, cache_rows, heads, kv_heads, head_dim);
+}

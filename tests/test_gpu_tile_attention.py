@@ -3,6 +3,8 @@ against float64: head layouts of every wave count, chunk lengths around the
 16-token tile and context lengths around the 32-row tile, chunks that begin or
 end inside a tile, tokens left to the per-token kernel, and values that are
 not finite in rows an earlier token must not see."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -27,6 +29,13 @@ def reference(q, key, value, tokens, heads, kvh, hd):
             p = np.exp(s - s.max())
             out[t, h * hd:(h + 1) * hd] = p @ v64[row:row + pos + 1, c] / p.sum()
     return out
+
+
+def tiles(qk, tokens, cache_rows, heads, kvh, hd):
+    """Whether the call tries tiles (its descriptors are on the device)."""
+    rule = qk.lib().qk_rule_tile_attention
+    rule.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3
+    return bool(rule(len(tokens), max(p for p, _ in tokens), cache_rows, heads, kvh, hd))
 
 
 def run(qk, t, q, key, value, tokens, heads, kvh, hd, split_rows=0):
@@ -167,3 +176,27 @@ def test_error_against_float64(qk, torch_gpu, heads, kvh, hd, ctx, chunk):
     tile = rel_l2(run(qk, t, q, key, value, tokens, heads, kvh, hd), want)
     per_token = rel_l2(run(qk, t, q, key, value, tokens, heads, kvh, hd, split_rows=ctx), want)
     assert tile < 1.02 * per_token
+
+
+def test_cache_with_room(qk, torch_gpu):
+    """A chunk takes the tile form whatever room its cache has beside it."""
+    heads, kvh, hd = 24, 8, 128
+    rng = np.random.default_rng(12)
+    q, key, value, tokens = batch(rng, [(1112, 512)], heads, kvh, hd)
+    want = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
+    assert tiles(qk, tokens, 1112, heads, kvh, hd)
+    for room in (1113, 4096, 65536):
+        assert tiles(qk, tokens, room, heads, kvh, hd)
+        pad = np.zeros((room, kvh * hd), np.float32)
+        pad[:1112] = key
+        vpad = np.full((room, kvh * hd), np.nan, np.float32)
+        vpad[:1112] = value
+        assert np.array_equal(run(qk, torch_gpu, q, pad, vpad, tokens, heads, kvh, hd), want)
+
+
+@pytest.mark.parametrize("heads,kvh,hd", [(32, 8, 64), (24, 8, 128), (16, 8, 64), (8, 8, 128)])
+def test_decode_batches_stay_per_token(qk, torch_gpu, heads, kvh, hd):
+    for lengths in ([700] * 32, list(range(64, 2048, 31)), [300] * 300, [4096] * 8):
+        tokens = [(n - 1, sum(lengths[:i])) for i, n in enumerate(lengths)]
+        for cache in (sum(lengths), 4 * sum(lengths)):
+            assert not tiles(qk, tokens, cache, heads, kvh, hd)
