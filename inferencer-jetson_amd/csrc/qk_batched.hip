@@ -218,10 +218,7 @@ __device__ __forceinline__ RawBlock load_block(const uint8_t *row, int b, int nb
     return r;
 }
 
-__device__ __forceinline__ uint32_t word(const uint4 *v, int i) {
-    const uint4 &u = v[i >> 2];
-    return (i & 3) == 0 ? u.x : (i & 3) == 1 ? u.y : (i & 3) == 2 ? u.z : u.w;
-}
+__device__ __forceinline__ uint32_t word(const uint4 *v, int i) { return quad_word(v[i >> 2], i & 3); }
 
 // Bytes 0 and 2 (sel 0x04020400) or 1 and 3 (sel 0x04030401) of v as the
 // fp16 halves 0x64nn = 1024 + n, then fma(1024 + n, s, bias) with bias =
@@ -321,119 +318,76 @@ __device__ __forceinline__ void step_scales(const RawBlock &r, int type, uint32_
     bb2 = half2v{static_cast<_Float16>(off * sb), static_cast<_Float16>(off * sb)};
 }
 
-// acc[r][t] += this block's contribution: RT row tiles (32 weight rows each,
-// lane l -> row l%32, block half l/32) x TT token tiles (32 tokens each).
-// Each decoded weight operand feeds TT token tiles; each activation operand
-// read from LDS feeds RT row tiles.
-template <int TYPE, int RT, int TT, bool WIDE = false>
-__device__ __forceinline__ void block_mma(const RawBlock (&r)[RT], int type, const uint8_t *buf_lds, int kh, int col,
-                                          float16v (&acc)[RT][TT]) {
-    float d[RT], dmin[RT];
-    uint32_t sc4[RT], mn4[RT];
-    #pragma unroll
-    for (int i = 0; i < RT; ++i) {
-        dmin[i] = 0.f;
-        sc4[i] = mn4[i] = 0;
-        if (is_q4<TYPE>(type)) {
-            d[i] = f16_bits_to_f32(r[i].hdr.x & 0xFFFFu);
-            dmin[i] = f16_bits_to_f32(r[i].hdr.x >> 16);
-            q4k_scale_min4(r[i].hdr, kh, sc4[i], mn4[i]);
-        } else {
-            d[i] = f16_bits_to_f32(r[i].hdr.z);
-        }
+// acc += this block's contribution: 32 weight rows (lane l -> row l%32, block
+// half l/32) x 32 tokens.
+template <int TYPE, bool WIDE = false>
+__device__ __forceinline__ void block_mma(const RawBlock &r, int type, const uint8_t *tile, int kh, int col,
+                                          float16v &acc) {
+    float d, dmin = 0.f;
+    uint32_t sc4 = 0, mn4 = 0;
+    if (is_q4<TYPE>(type)) {
+        d = f16_bits_to_f32(r.hdr.x & 0xFFFFu);
+        dmin = f16_bits_to_f32(r.hdr.x >> 16);
+        q4k_scale_min4(r.hdr, kh, sc4, mn4);
+    } else {
+        d = f16_bits_to_f32(r.hdr.z);
     }
-    float16v t[RT][TT];
+    float16v t;
     #pragma unroll
-    for (int i = 0; i < RT; ++i)
-        #pragma unroll
-        for (int u = 0; u < TT; ++u)
-            #pragma unroll
-            for (int k = 0; k < 16; ++k) t[i][u][k] = 0.f;
+    for (int k = 0; k < 16; ++k) t[k] = 0.f;
     // Activation operands are read from LDS one step ahead of their use.
-    half8 ah[TT], al[TT];
-    #pragma unroll
-    for (int u = 0; u < TT; ++u) {
-        const uint8_t *tile = buf_lds + u * kTileBytes;
-        ah[u] = reinterpret_cast<const half8 *>(tile)[kh * 32 + col];
-        al[u] = reinterpret_cast<const half8 *>(tile + kTileA)[kh * 32 + col];
-    }
+    half8 ah = reinterpret_cast<const half8 *>(tile)[kh * 32 + col];
+    half8 al = reinterpret_cast<const half8 *>(tile + kTileA)[kh * 32 + col];
     #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
         #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int st = hf * 8 + j;
-            half8 ahn[TT], aln[TT];
-            #pragma unroll
-            for (int u = 0; u < TT; ++u) {
-                const uint8_t *tile = buf_lds + u * kTileBytes;
-                const int sn = st < 15 ? st + 1 : st;
-                ahn[u] = reinterpret_cast<const half8 *>(tile)[sn * 64 + kh * 32 + col];
-                aln[u] = reinterpret_cast<const half8 *>(tile + kTileA)[sn * 64 + kh * 32 + col];
+            const int st = hf * 8 + j, sn = st < 15 ? st + 1 : st;
+            const half8 ahn = reinterpret_cast<const half8 *>(tile)[sn * 64 + kh * 32 + col];
+            const half8 aln = reinterpret_cast<const half8 *>(tile + kTileA)[sn * 64 + kh * 32 + col];
+            half2v sa2, ba2, sb2, bb2;
+            step_scales<TYPE>(r, type, sc4, hf, j, sa2, ba2, sb2, bb2);
+            if constexpr (WIDE) {
+                // Q6_K with wide scales: W = W_a + W_b exactly.
+                half8 wa, wb;
+                decode_b_wide(r, hf, j, sa2, sb2, wa, wb);
+                t = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, wa, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, wa, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, wb, t, 0, 0, 0);
+            } else {
+                const half8 bw = decode_b<TYPE>(r, type, hf, j, sa2, ba2, sb2, bb2);
+                t = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bw, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bw, t, 0, 0, 0);
             }
-            #pragma unroll
-            for (int i = 0; i < RT; ++i) {
-                half2v sa2, ba2, sb2, bb2;
-                step_scales<TYPE>(r[i], type, sc4[i], hf, j, sa2, ba2, sb2, bb2);
-                if constexpr (WIDE) {
-                    // Q6_K with wide scales: W = W_a + W_b exactly.
-                    half8 wa, wb;
-                    decode_b_wide(r[i], hf, j, sa2, sb2, wa, wb);
-                    #pragma unroll
-                    for (int u = 0; u < TT; ++u) {
-                        t[i][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[u], wa, t[i][u], 0, 0, 0);
-                        t[i][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[u], wa, t[i][u], 0, 0, 0);
-                        t[i][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[u], wb, t[i][u], 0, 0, 0);
-                    }
-                } else {
-                    const half8 bw = decode_b<TYPE>(r[i], type, hf, j, sa2, ba2, sb2, bb2);
-                    #pragma unroll
-                    for (int u = 0; u < TT; ++u) {
-                        t[i][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[u], bw, t[i][u], 0, 0, 0);
-                        t[i][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[u], bw, t[i][u], 0, 0, 0);
-                    }
-                }
-            }
-            #pragma unroll
-            for (int u = 0; u < TT; ++u) {
-                ah[u] = ahn[u];
-                al[u] = aln[u];
-            }
+            ah = ahn;
+            al = aln;
         }
     }
+    const float4 *fr = reinterpret_cast<const float4 *>(tile + 2 * kTileA + 2 * kTileM) + kh * 4;
+    float f[16];
     #pragma unroll
-    for (int u = 0; u < TT; ++u) {
-        const uint8_t *tile = buf_lds + u * kTileBytes;
-        const float4 *fr = reinterpret_cast<const float4 *>(tile + 2 * kTileA + 2 * kTileM) + kh * 4;
-        float f[16];
+    for (int q = 0; q < 4; ++q) {
+        const float4 v = fr[q];
+        f[4 * q] = v.x;
+        f[4 * q + 1] = v.y;
+        f[4 * q + 2] = v.z;
+        f[4 * q + 3] = v.w;
+    }
+    #pragma unroll
+    for (int k = 0; k < 16; ++k) acc[k] = fmaf(d * f[k], t[k], acc[k]);
+    if (is_q4<TYPE>(type)) {
+        const half4 mh = reinterpret_cast<const half4 *>(tile + 2 * kTileA)[kh * 32 + col];
+        const half4 ml = reinterpret_cast<const half4 *>(tile + 2 * kTileA + kTileM)[kh * 32 + col];
+        half4 bm;
         #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 v = fr[q];
-            f[4 * q] = v.x;
-            f[4 * q + 1] = v.y;
-            f[4 * q + 2] = v.z;
-            f[4 * q + 3] = v.w;
-        }
+        for (int e = 0; e < 4; ++e) bm[e] = u8_to_h(mn4 >> (8 * e));
+        float16v tm;
         #pragma unroll
-        for (int i = 0; i < RT; ++i)
-            #pragma unroll
-            for (int k = 0; k < 16; ++k) acc[i][u][k] = fmaf(d[i] * f[k], t[i][u][k], acc[i][u][k]);
-        if (is_q4<TYPE>(type)) {
-            const half4 mh = reinterpret_cast<const half4 *>(tile + 2 * kTileA)[kh * 32 + col];
-            const half4 ml = reinterpret_cast<const half4 *>(tile + 2 * kTileA + kTileM)[kh * 32 + col];
-            #pragma unroll
-            for (int i = 0; i < RT; ++i) {
-                half4 bm;
-                #pragma unroll
-                for (int e = 0; e < 4; ++e) bm[e] = u8_to_h(mn4[i] >> (8 * e));
-                float16v tm;
-                #pragma unroll
-                for (int k = 0; k < 16; ++k) tm[k] = 0.f;
-                tm = __builtin_amdgcn_mfma_f32_32x32x8f16(mh, bm, tm, 0, 0, 0);
-                tm = __builtin_amdgcn_mfma_f32_32x32x8f16(ml, bm, tm, 0, 0, 0);
-                #pragma unroll
-                for (int k = 0; k < 16; ++k) acc[i][u][k] = fmaf(-64.f * dmin[i] * f[k], tm[k], acc[i][u][k]);
-            }
-        }
+        for (int k = 0; k < 16; ++k) tm[k] = 0.f;
+        tm = __builtin_amdgcn_mfma_f32_32x32x8f16(mh, bm, tm, 0, 0, 0);
+        tm = __builtin_amdgcn_mfma_f32_32x32x8f16(ml, bm, tm, 0, 0, 0);
+        #pragma unroll
+        for (int k = 0; k < 16; ++k) acc[k] = fmaf(-64.f * dmin * f[k], tm[k], acc[k]);
     }
 }
 
@@ -443,7 +397,13 @@ __device__ __forceinline__ void store_out(const BatchParams &p, float *y, float 
     *y = v;
 }
 
-#include "qk_tile_gemm.h"
+}  // namespace
+}  // namespace qk
+
+#include "qk_tile_gemm.h"   // on the launch parameters and the store above
+
+namespace qk {
+namespace {
 
 // ------------------------------------------------ GEMM of one token tile --
 //
@@ -477,12 +437,10 @@ __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)"
 template <int TYPE>
 __global__ __launch_bounds__(256) void batch_gemm(BatchParams p) {
     extern __shared__ __align__(16) unsigned char lds[];
-    constexpr int RT = 1, TT = 1;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = lane >> 5, col = lane & 31;
     const int split = blockIdx.x % p.splits, group = blockIdx.x / p.splits;
-    const int tile0 = 0;
 
     int m = 0;
     #pragma unroll
@@ -490,101 +448,56 @@ __global__ __launch_bounds__(256) void batch_gemm(BatchParams p) {
     m = __builtin_amdgcn_readfirstlane(m);
     const BatchMatrix &M = p.mat[m];
     const int type = TYPE ? TYPE : M.type;
-    const uint8_t *wrow[RT];
-    int row[RT];
-    #pragma unroll
-    for (int i = 0; i < RT; ++i) {
-        row[i] = (group - M.group_begin) * kGroupRows + (i * 4 + wave) * 32 + col;
-        wrow[i] = M.w + static_cast<size_t>(min(row[i], M.rows - 1)) * M.row_bytes;
-    }
-    // Token tiles past the end read the last tile's records (in bounds) and store nothing.
-    const uint8_t *recs[TT];
-    #pragma unroll
-    for (int u = 0; u < TT; ++u)
-        recs[u] = p.records + static_cast<size_t>(min(tile0 + u, p.tiles - 1)) * p.nb * kTileBytes;
+    const int row = (group - M.group_begin) * kGroupRows + wave * 32 + col;
+    const uint8_t *const wrow = M.w + static_cast<size_t>(min(row, M.rows - 1)) * M.row_bytes;
 
     const int b0 = split * p.blocks_per_split;
     const int b1 = min(p.nb, b0 + p.blocks_per_split);
-    #pragma unroll
-    for (int u = 0; u < TT; ++u) record_dma(recs[u] + static_cast<size_t>(b0) * kTileBytes, lds + u * kTileBytes, wave, lane);
-    RawBlock cur[RT];
-    #pragma unroll
-    for (int i = 0; i < RT; ++i) cur[i] = load_block<TYPE>(wrow[i], b0, p.nb, type, kh);
+    record_dma(p.records + static_cast<size_t>(b0) * kTileBytes, lds, wave, lane);
+    RawBlock cur = load_block<TYPE>(wrow, b0, p.nb, type, kh);
     wait_loads();
     __syncthreads();
 
-    float16v acc[RT][TT];
+    float16v acc;
     #pragma unroll
-    for (int i = 0; i < RT; ++i)
-        #pragma unroll
-        for (int u = 0; u < TT; ++u)
-            #pragma unroll
-            for (int k = 0; k < 16; ++k) acc[i][u][k] = 0.f;
+    for (int k = 0; k < 16; ++k) acc[k] = 0.f;
     for (int b = b0; b < b1; ++b) {
         const int buf = (b - b0) & 1;
         // The last iteration reloads its own weight bytes (unconditional, in bounds).
         const int bn = min(b + 1, b1 - 1);
-        if (b + 1 < b1) {
-            #pragma unroll
-            for (int u = 0; u < TT; ++u)
-                record_dma(recs[u] + static_cast<size_t>(bn) * kTileBytes, lds + ((buf ^ 1) * TT + u) * kTileBytes, wave,
-                           lane);
-        }
-        RawBlock nxt[RT];
-        #pragma unroll
-        for (int i = 0; i < RT; ++i) nxt[i] = load_block<TYPE>(wrow[i], bn, p.nb, type, kh);
+        if (b + 1 < b1) record_dma(p.records + static_cast<size_t>(bn) * kTileBytes, lds + (buf ^ 1) * kTileBytes, wave, lane);
+        const RawBlock nxt = load_block<TYPE>(wrow, bn, p.nb, type, kh);
         // A Q6_K block whose scales leave [-62, 62] in any of the wave's rows
         // takes the exact three-chain decode (wave-uniform branch).
         bool wide = false;
-        if constexpr (TYPE != QK_TYPE_Q4_K) {
-            if (!is_q4<TYPE>(type)) {
-                bool lane_wide = false;
-                #pragma unroll
-                for (int i = 0; i < RT; ++i) lane_wide |= q6_scales_wide(cur[i]);
-                wide = __builtin_amdgcn_ballot_w64(lane_wide) != 0;
-            }
-        }
+        if constexpr (TYPE != QK_TYPE_Q4_K)
+            if (!is_q4<TYPE>(type)) wide = __builtin_amdgcn_ballot_w64(q6_scales_wide(cur)) != 0;
         if (wide)
-            block_mma<TYPE, RT, TT, true>(cur, type, lds + buf * TT * kTileBytes, kh, col, acc);
+            block_mma<TYPE, true>(cur, type, lds + buf * kTileBytes, kh, col, acc);
         else
-            block_mma<TYPE, RT, TT>(cur, type, lds + buf * TT * kTileBytes, kh, col, acc);
-        #pragma unroll
-        for (int i = 0; i < RT; ++i) cur[i] = nxt[i];
+            block_mma<TYPE>(cur, type, lds + buf * kTileBytes, kh, col, acc);
+        cur = nxt;
         wait_loads();
         __syncthreads();
     }
 
-    // Accumulator register k holds token 8*(k/4) + 4*kh + k%4 of its tile.
+    // Accumulator register k holds token 8*(k/4) + 4*kh + k%4 of the tile.
     if (!p.partials) {
+        if (row >= M.rows) return;
         #pragma unroll
-        for (int u = 0; u < TT; ++u) {
-            const int tbase = (tile0 + u) * kTokTile + 4 * kh;
-            #pragma unroll
-            for (int i = 0; i < RT; ++i) {
-                if (row[i] >= M.rows) continue;
-                #pragma unroll
-                for (int k = 0; k < 16; ++k) {
-                    const int t = tbase + 8 * (k >> 2) + (k & 3);
-                    if (t < p.n_tokens) store_out(p, M.y + static_cast<int64_t>(t) * M.ldy + row[i], acc[i][u][k]);
-                }
-            }
+        for (int k = 0; k < 16; ++k) {
+            const int t = 4 * kh + 8 * (k >> 2) + (k & 3);
+            if (t < p.n_tokens) store_out(p, M.y + static_cast<int64_t>(t) * M.ldy + row, acc[k]);
         }
         return;
     }
     // Split blocks: partial sums to the workspace in accumulator order,
-    // [group][token tile][split][wave][row tile][k][lane]; reduce_splits adds
-    // them.  (A last-workgroup reduction inside this kernel would need a
-    // device-scope fence per workgroup, measured slower than the extra launch.)
+    // [group][split][wave][k][lane]; reduce_splits adds them.  (A last-workgroup
+    // reduction inside this kernel would need a device-scope fence per
+    // workgroup, measured slower than the extra launch.)
+    float *mine = p.partials + (static_cast<size_t>(group) * p.splits + split) * kPartialFloats + wave * 1024 + lane;
     #pragma unroll
-    for (int u = 0; u < TT; ++u) {
-        if (tile0 + u >= p.tiles) break;
-        const size_t slot = static_cast<size_t>(group) * p.tiles + tile0 + u;
-        float *mine = p.partials + (slot * p.splits + split) * kPartialFloats + wave * (RT * 1024) + lane;
-        #pragma unroll
-        for (int i = 0; i < RT; ++i)
-            #pragma unroll
-            for (int k = 0; k < 16; ++k) mine[i * 1024 + k * 64] = acc[i][u][k];
-    }
+    for (int k = 0; k < 16; ++k) mine[k * 64] = acc[k];
 }
 
 // y = the sum of a row group's split partials, in split order (deterministic),

@@ -36,7 +36,7 @@ namespace {
 
 typedef float float4v __attribute__((ext_vector_type(4)));
 
-constexpr int kSlots = 8;            // tokens of a launch at most
+constexpr int kSlots = 8;            // token slots of an operand; a launch takes up to kSlots - 1 tokens
 constexpr int kTileRows = 16;
 constexpr int kMaxWaves = 16;
 
@@ -87,13 +87,6 @@ __device__ __forceinline__ Raw<TYPE == QK_TYPE_Q4_K> load_raw(const uint8_t *row
         r.h = make_uint4(sc.x, sc.y, load2(f.d), 0);
     }
     return r;
-}
-
-// First column (of four) of operand step s in a block, for a lane's quarter;
-// the second four are 32 columns on.
-template <bool Q4>
-__device__ __forceinline__ int step_column(int kq, int s) {
-    return Q4 ? kq * 64 + 4 * s : (kq >> 1) * 128 + (s >> 2) * 64 + (kq & 1) * 16 + (s & 3) * 4;
 }
 
 // A block's activations of eight tokens: lane (n, kq) holds operand row n

@@ -26,6 +26,11 @@ constexpr int kTileF = 128;
 constexpr int kTileBytes = 2 * kTileA + 2 * kTileM + kTileF;
 static_assert(kTileBytes % 16 == 0, "tiles keep 16-byte alignment");
 
+// The LDS address of a pointer into it, as direct copies take it (m0).
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void *)p));
+}
+
 // One token's 256-value block into its record, by a whole wave: lane (q, j)
 // = (lane / 8, lane % 8) holds values q*32 + 4j .. +3 (v).  x' = x * 2^shift
 // with the block maximum in [2^14, 2^15) (shift capped at 140 so 2^-shift

@@ -56,10 +56,6 @@ struct TileAttnArgs {
     int groups;    // S: waves sharing a head's rows
 };
 
-__device__ __forceinline__ uint32_t lds_address(const void *p) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void *)p));
-}
-
 // 16 bytes a lane to LDS at dst + 16 * lane (dst wave-uniform), untracked by
 // the compiler's wait insertion.
 #pragma clang diagnostic push

@@ -1,5 +1,6 @@
-// qk_tile_gemm.h - the matrix-core GEMM of two 32-token tiles and more,
-// included by csrc/qk_batched.hip.
+// qk_tile_gemm.h - the matrix-core GEMM of two 32-token tiles and more: the part
+// of csrc/qk_batched.hip (whose launch parameters and output store it uses)
+// that takes them.
 //
 // A workgroup of four waves takes 128 weight rows x 64 tokens x a run of
 // 256-column blocks; wave w owns rows 32w .. 32w + 31 and multiplies them with
@@ -34,6 +35,9 @@
 
 #include <type_traits>
 
+namespace qk {
+namespace {
+
 constexpr int kHalfBytes = 2 * 8 * 1024;                 // one token tile's half block: hi, lo x 8 steps x 1 KB
 constexpr int kTokenBytes = 2 * kTileM + kTileF;         // a tile's sub-block sums and scales
 
@@ -41,10 +45,6 @@ constexpr int kRun = 8;                                  // blocks of one runnin
 
 // LDS: two half-block buffers of two token tiles, then two blocks' token data.
 constexpr int kTileLds = 2 * 2 * (kHalfBytes + kTokenBytes);
-
-__device__ __forceinline__ uint32_t lds_address(const void *p) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void *)p));
-}
 
 // 1 KB from global memory (src, wave-uniform) to LDS (dst): 16 bytes a lane at
 // lane16 = 16 * lane.  Inline assembly: the compiler would wait for every
@@ -399,3 +399,6 @@ __global__ __launch_bounds__(256, 2) void tile_gemm(BatchParams p, int groups, i
         run(std::integral_constant<int, QK_TYPE_Q6_K_SPLIT>{});
     }
 }
+
+}  // namespace
+}  // namespace qk
