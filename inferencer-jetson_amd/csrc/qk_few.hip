@@ -505,3 +505,7 @@ int launch_few(const qk_matrix *mats, int n_mats, const float *x, int ldx, int c
 }
 
 }  // namespace qk
+
+extern "C" int qk_rule_few_tokens(const qk_matrix *mats, int n_mats, int cols, int n_tokens, int pair) {
+    return qk::few_pays(mats, n_mats, cols, n_tokens, pair != 0);
+}

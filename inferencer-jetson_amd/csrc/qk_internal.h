@@ -768,4 +768,11 @@ int launch_q6k_join(const void *src, void *dst, int cols, int rows, hipStream_t 
 }  // namespace qk
 
 // Dispatch rules by plain arguments: the tests ask them which form a call takes.
-extern "C" int qk_rule_tile_attention(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim);
+extern "C" {
+int qk_rule_tile_attention(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim);
+// SplitAttention::tile_mode of a decode driver's step.
+int qk_rule_tile_attention_step(const qk_batch_token *desc, int n_tokens, int heads, int kv_heads, int head_dim);
+int qk_rule_few_tokens(const qk_matrix *mats, int n_mats, int cols, int n_tokens, int pair);
+// The splits of launch_tile_i8 with the queried workspace, or 0.
+int qk_rule_tile_i8(const qk_matrix *mats, int n_mats, int cols, int n_tokens, int pair);
+}

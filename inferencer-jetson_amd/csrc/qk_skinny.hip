@@ -1016,6 +1016,20 @@ size_t ffn_i8_bytes(int dim, int hidden, int n_tokens, bool plans) {
 
 extern "C" {
 
+int qk_rule_tile_i8(const qk_matrix *mats, int n_mats, int cols, int n_tokens, int pair) {
+    if (n_tokens < kMatrixCoreTokens) return 0;
+    const int tiles = qk::row_tiles(mats, n_mats, pair != 0), token_tiles = (n_tokens + qk::kToks - 1) / qk::kToks;
+    int type = mats[0].type;
+    for (int i = 1; i < n_mats; ++i)
+        if (mats[i].type != type) type = 0;
+    const qk::SkPlan plan = qk::split_plan(cols / 256, static_cast<int64_t>(tiles) * token_tiles, token_tiles, type,
+                                           pair ? 2 : 1, false, false);
+    return plan.loop_groups && !plan.rows
+               ? qk::tile_i8_splits(mats, n_mats, cols, n_tokens, cols, cols / 32, pair != 0,
+                                    qk::skinny_i8_workspace_bytes(cols, tiles, n_tokens, pair != 0))
+               : 0;
+}
+
 size_t qk_gemv_batched_i8_workspace_bytes(int cols, int rows, int n_tokens) {
     if (cols <= 0 || cols % 256 || rows <= 0 || n_tokens < kMatrixCoreTokens) return 0;
     // Any split of rows over up to QK_MAX_FUSED matrices has at most

@@ -453,6 +453,20 @@ int launch_tile_attention(const SplitAttention &a, hipStream_t stream) {
 
 }  // namespace qk
 
-extern "C" int qk_rule_tile_attention(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim) {
+extern "C" {
+
+int qk_rule_tile_attention(int n_tokens, int max_pos, int64_t cache_rows, int heads, int kv_heads, int head_dim) {
     return qk::tile_attention_call(n_tokens, max_pos, cache_rows, heads, kv_heads, head_dim);
 }
+
+int qk_rule_tile_attention_step(const qk_batch_token *desc, int n_tokens, int heads, int kv_heads, int head_dim) {
+    qk::SplitAttention a{};
+    a.desc = desc;
+    a.n_tokens = n_tokens;
+    a.heads = heads;
+    a.kv_heads = kv_heads;
+    a.head_dim = head_dim;
+    return qk::tile_attention_mode(desc, a);
+}
+
+}  // extern "C"

@@ -1,9 +1,12 @@
 """Products of 2 to 7 tokens (csrc/qk_few.hip): row counts around the 16-row
-tile and the two-tile step, one to thirty-two blocks a row (one or two a wave),
-every storage type alone and mixed, scales over the whole int8 range, the
-feed-forward block's pair and residual, values that are not finite.  The sizes
-are those that few_pays takes (enough weight bytes for the token count); the
-small ones beside them go to the GEMV kernels."""
+tile and the two-tile step, one to thirty-two blocks a row (one or two a wave,
+with and without a second block in the last wave), every storage type alone and
+mixed, scales over the whole int8 range, the feed-forward block's pair, its down
+product and residual, SiLU(x) * up and the RMSNorm staged by the decode driver,
+values that are not finite.  few_pays decides which calls come here (enough
+weight bytes for the token count); every test asks it."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -13,27 +16,41 @@ from test_gpu_tile_gemm import Q4_K, Q6_K, Q6_K_SPLIT, TOL, check, matrix
 pytestmark = pytest.mark.gpu
 
 
+def few(qk, mats, cols, ntok, pair=False):
+    """Whether a call over mats ((type, rows) each) comes here."""
+    arr = (qk.qk_matrix * len(mats))(*(qk.qk_matrix(ty, rows, None, None) for ty, rows in mats))
+    return bool(qk.lib().qk_rule_few_tokens(arr, len(mats), cols, ntok, int(pair)))
+
+
 @pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q6_K_SPLIT])
 @pytest.mark.parametrize("ntok,cols,rows", [(7, 256, 66001), (7, 768, 32015), (4, 2048, 65541), (6, 3072, 16400),
-                                            (5, 4096, 12001), (7, 4352, 3903), (7, 8192, 3899), (7, 8192, 3700),
-                                            (3, 1024, 20)])
+                                            (5, 4096, 12001), (7, 7424, 4093), (7, 7936, 3900), (7, 8192, 3899),
+                                            (7, 8192, 3700), (3, 2048, 128256)])
 def test_edges(qk, torch_gpu, oracle, workloads, synth, qtype, ntok, cols, rows):
     x = synth.normal_f32(ntok * cols, 61, ntok).reshape(ntok, cols)
+    assert few(qk, [(qtype, rows)], cols, ntok)
     check(qk, torch_gpu, oracle, [matrix(qk, torch_gpu, workloads, synth, qtype, cols, rows, 60 + ntok)], x, cols)
 
 
-@pytest.mark.parametrize("ntok,cols", [(7, 2048), (5, 2560), (3, 512)])
+@pytest.mark.parametrize("ntok,cols", [(7, 2048), (5, 2560), (3, 4096)])
 def test_mixed_types(qk, torch_gpu, oracle, workloads, synth, ntok, cols):
     x = synth.normal_f32(ntok * cols, 62, ntok).reshape(ntok, cols)
-    tensors = [matrix(qk, torch_gpu, workloads, synth, ty, cols, rows, 70 + i)
-               for i, (ty, rows) in enumerate([(Q4_K, 16500), (Q6_K, 96), (Q6_K_SPLIT, 257), (Q4_K, 20)])]
+    mats = [(Q4_K, 16500), (Q6_K, 96), (Q6_K_SPLIT, 257), (Q4_K, 20)]
+    assert few(qk, mats, cols, ntok)
+    tensors = [matrix(qk, torch_gpu, workloads, synth, ty, cols, rows, 70 + i) for i, (ty, rows) in enumerate(mats)]
     check(qk, torch_gpu, oracle, tensors, x, cols)
 
 
 @pytest.mark.parametrize("types", [(Q4_K, Q4_K, Q6_K), (Q4_K, Q6_K, Q4_K), (Q6_K_SPLIT, Q6_K_SPLIT, Q6_K_SPLIT)])
-@pytest.mark.parametrize("ntok,dim,hidden", [(7, 2048, 4096), (5, 3072, 4096), (7, 1024, 8192), (2, 512, 768)])
+@pytest.mark.parametrize("ntok,dim,hidden", [(7, 2048, 4096), (5, 3072, 4096), (7, 1024, 8192), (7, 4096, 4096),
+                                             (6, 4096, 4096)])
 def test_ffn(qk, torch_gpu, oracle, workloads, synth, types, ntok, dim, hidden):
+    """Gate and up of one type in one launch with SiLU * up; down here too from
+    4096 x 4096 on, else by the GEMV kernels."""
     t = torch_gpu
+    if types[0] == types[1]:
+        assert few(qk, [(types[0], hidden), (types[1], hidden)], dim, ntok, True)
+    assert few(qk, [(types[2], dim)], hidden, ntok) == (dim >= 4096)
     x = synth.normal_f32(ntok * dim, 63, ntok).reshape(ntok, dim) * 0.05
     shapes = [(dim, hidden), (dim, hidden), (hidden, dim)]
     (g, wg, tg), (u, wu, tu), (d, wd, td) = [matrix(qk, t, workloads, synth, ty, c, r, 80 + i)
@@ -52,18 +69,71 @@ def test_ffn(qk, torch_gpu, oracle, workloads, synth, types, ntok, dim, hidden):
     assert rel_l2(y.cpu().numpy(), want) < 4 * TOL
 
 
-def test_not_finite(qk, torch_gpu, workloads, synth):
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q6_K_SPLIT])
+@pytest.mark.parametrize("ntok,cols,rows", [(4, 2048, 65541), (7, 7936, 3900)])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_not_finite(qk, torch_gpu, workloads, synth, qtype, ntok, cols, rows, value):
     """A non-finite activation poisons its own token's outputs only."""
     t = torch_gpu
-    ntok, cols, rows = 4, 1024, 100
     x = synth.normal_f32(ntok * cols, 64, 1).reshape(ntok, cols)
-    x[2, 700] = np.inf
-    ten, _, _ = matrix(qk, t, workloads, synth, Q4_K, cols, rows, 90)
+    x[2, 700] = value
+    assert few(qk, [(qtype, rows)], cols, ntok)
+    ten, _, _ = matrix(qk, t, workloads, synth, qtype, cols, rows, 90)
     y = t.empty((ntok, rows), device="cuda")
     qk.batch_matvec(ten, to_dev(t, x), y, cols, rows, ntok)
     t.cuda.synchronize()
     got = y.cpu().numpy()
-    assert np.isnan(got[2]).all() and np.isfinite(got[[0, 1, 3]]).all()
+    assert np.isnan(got[2]).all() and np.isfinite(np.delete(got, 2, 0)).all()
+
+
+def test_pair_not_finite(qk, torch_gpu, workloads, synth):
+    t = torch_gpu
+    ntok, dim, hidden = 7, 4096, 4096
+    x = synth.normal_f32(ntok * dim, 66, 1).reshape(ntok, dim) * 0.05
+    x[3, 17], x[5, 4095] = np.nan, np.inf
+    (g, _, _), (u, _, _), (d, _, _) = [matrix(qk, t, workloads, synth, Q4_K, c, r, 92 + i)
+                                       for i, (c, r) in enumerate([(dim, hidden), (dim, hidden), (hidden, dim)])]
+    assert few(qk, [(Q4_K, hidden)] * 2, dim, ntok, True) and few(qk, [(Q4_K, dim)], hidden, ntok)
+    nb = qk.lib().qk_ffn_batched_workspace_bytes(dim, hidden, ntok)
+    ws, y = t.empty(nb, dtype=t.uint8, device="cuda"), t.empty((ntok, dim), device="cuda")
+    xd = to_dev(t, x)
+    qk.check(qk.lib().qk_ffn_batched_f32(Q4_K, g.gpu, Q4_K, u.gpu, Q4_K, d.gpu, xd.data_ptr(), dim, y.data_ptr(), dim, dim,
+                                         hidden, ntok, 0, ws.data_ptr(), nb, None), "ffn")
+    t.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.isnan(got[[3, 5]]).all() and np.isfinite(got[[0, 1, 2, 4, 6]]).all()
+
+
+@pytest.mark.parametrize("up_type", [Q4_K, Q6_K])
+def test_driver_step(qk, torch_gpu, oracle, workloads, synth, up_type):
+    """Seven sequences decoding in the batched driver: QKV and gate / up with the
+    RMSNorm staged here, gate and up of one type (the pair) or of two (down then
+    stages SiLU * up), both projections into x accumulated; each sequence against
+    its own oracle model."""
+    cfg = dict(dim=4096, layers=2, heads=32, kv_heads=8, hidden=4096, vocab=300, context=32, eps=1e-5,
+               rope_theta=10000.0)
+    ntok = 7
+    W = workloads.llama_weights(cfg, 27, mix=dict(workloads.MIX_1B, up=up_type))
+    for i, L in enumerate(W["layers"]):
+        L["attn_norm"] = 1.0 + 0.2 * synth.normal_f32(cfg["dim"], 27, 500 + i)
+        L["ffn_norm"] = 1.0 + 0.2 * synth.normal_f32(cfg["dim"], 27, 510 + i)
+        kv = cfg["dim"] // cfg["heads"] * cfg["kv_heads"]
+        assert few(qk, [(L["q_type"], cfg["dim"]), (L["k_type"], kv), (L["v_type"], kv)], cfg["dim"], ntok)
+        assert few(qk, [(L["gate_type"], cfg["hidden"]), (L["up_type"], cfg["hidden"])], cfg["dim"], ntok, True) == \
+            (up_type == Q4_K)
+        assert few(qk, [(L["gate_type"], cfg["hidden"]), (L["up_type"], cfg["hidden"])], cfg["dim"], ntok)
+        assert few(qk, [(L["down_type"], cfg["dim"])], cfg["hidden"], ntok)
+    br = qk.BatchRunner(cfg, W, max_tokens=ntok, cache_rows=ntok * cfg["context"])
+    orcs = [oracle.Llama(cfg, W) for _ in range(ntok)]
+    tokens = [int(v) for v in synth.uniform_i32(ntok, 27, 71, 0, cfg["vocab"] - 1)]
+    for pos in range(2):
+        br.forward(tokens, [pos] * ntok, [s * cfg["context"] for s in range(ntok)], True)
+        lg = br.logits(ntok)
+        want = [orcs[s].forward(tokens[s], pos, True) for s in range(ntok)]
+        for s in range(ntok):
+            assert rel_l2(lg[s], want[s][1]) < 1e-4
+        tokens = [o for o, _ in want]
+    br.close()
 
 
 def test_infinite_scale_in_the_last_block(qk, torch_gpu, oracle, workloads, synth):
@@ -73,6 +143,7 @@ def test_infinite_scale_in_the_last_block(qk, torch_gpu, oracle, workloads, synt
     over zeros would make every one NaN."""
     t = torch_gpu
     ntok, cols, rows = 7, 31 * 256, 4096
+    assert few(qk, [(Q4_K, rows)], cols, ntok)
     x = synth.normal_f32(ntok * cols, 65, ntok).reshape(ntok, cols)
     w, _ = workloads.gemv_case(Q4_K, cols, rows, seed=91)
     w = w.reshape(rows, 31, 144).copy()

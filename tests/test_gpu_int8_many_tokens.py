@@ -1,22 +1,28 @@
 """INT8 products of more (row tile, token tile) units than the chip holds at
-once (csrc/qk_tile_i8.hip): ragged token and row tiles, split rows, the gate /
-up pair, accumulation, strided inputs and outputs, and a workspace too small
-for the planned splits.
+once (csrc/qk_tile_i8.hip): ragged token and row tiles, rows in one piece and
+split, short and long sums, the gate / up pair, several matrices of one type,
+accumulation, strided inputs and outputs, every storage type, workspaces at and
+beyond the queried size and below it.  Every test of the kernel asks the dispatch
+rule whether its call comes here.
 
 Integer blocks (d = dmin = 1) with unit scales make every partial sum an exact
-integer below 2^24, so the outputs equal an int64 product bit for bit; random
-blocks are compared with the fp64 combine.  Its bar: an output adds K / 32
-products of fp32 operands, each rounded a few times, so the relative error of
-the whole is below about sqrt(K / 32) * 2^-24 * a small factor: 1e-5 as for the
-integer matrix cores."""
+integer below 2^24, so the outputs equal an int64 product bit for bit; the
+rounding of random blocks is held to a derived bar (test_rounding)."""
 import numpy as np
 import pytest
 
 from conftest import rel_l2, to_dev
 from test_gpu_int8_matrix_core import Q4_K, Q6_K, _integer_blocks
-from test_gpu_tile_gemm import sizes_of
+from test_gpu_tile_gemm import Q6_K_SPLIT, sizes_of
 
 pytestmark = pytest.mark.gpu
+
+
+def splits(qk, mats, cols, ntok, pair=False):
+    """The row splits of a call over mats ((type, rows) each) that comes here, or
+    0."""
+    arr = (qk.qk_matrix * len(mats))(*(qk.qk_matrix(ty, rows, None, None) for ty, rows in mats))
+    return qk.lib().qk_rule_tile_i8(arr, len(mats), cols, ntok, int(pair))
 
 
 def _dense(t, qk, qtype, w, cols, rows):
@@ -27,31 +33,71 @@ def _dense(t, qk, qtype, w, cols, rows):
     return out.cpu().double()
 
 
-@pytest.mark.parametrize("qtype", [Q4_K, Q6_K])
-@pytest.mark.parametrize("cols,rows,ntok", [(5632, 2050, 300), (8192, 1055, 545), (4096, 4096, 161),
-                                            (20480, 2050, 130)])
-def test_exact_ragged(qk, torch_gpu, synth, qtype, cols, rows, ntok):
+def _tensor(t, qk, qtype, w, cols, rows):
+    """The device matrix of GGUF block bytes, in the split layout for Q6_K_SPLIT."""
+    ten = qk.Tensor((cols, rows), Q4_K if qtype == Q4_K else Q6_K, to_dev(t, w))
+    if qtype == Q6_K_SPLIT:
+        ten = qk.split_q6k(ten)
+        t.cuda.synchronize()
+    return ten
+
+
+def _sparse_codes(t, g, ntok, ldxq):
+    """Small codes: whole sums stay below 2^24 (scale * code <= 4096)."""
+    xq = t.randint(-1, 2, (ntok, ldxq), generator=g, dtype=t.int8)
+    return xq * (t.rand(ntok, ldxq, generator=g) < 0.1).to(t.int8)
+
+
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q6_K_SPLIT])
+@pytest.mark.parametrize("cols,rows,ntok,here", [
+    (5632, 2050, 300, True), (8192, 1055, 545, True), (4096, 4096, 193, True), (8192, 8191, 1000, True),
+    (20480, 2050, 130, None)])   # the last: Q4_K by the looping int32 kernel, in ten splits
+def test_exact_ragged(qk, torch_gpu, synth, qtype, cols, rows, ntok, here):
     t = torch_gpu
-    w = _integer_blocks(qtype, synth.quant_matrix(qtype, cols, rows, 5, 1), cols, rows)
-    dense = _dense(t, qk, qtype, w, cols, rows)
+    base = Q4_K if qtype == Q4_K else Q6_K
+    assert bool(splits(qk, [(qtype, rows)], cols, ntok)) == (qtype != Q4_K if here is None else here)
+    w = _integer_blocks(base, synth.quant_matrix(base, cols, rows, 5, 1), cols, rows)
+    dense = _dense(t, qk, base, w, cols, rows)
     g = t.Generator().manual_seed(3)
     ldxq, ldsc, ldy = cols + 32, cols // 32 + 3, rows + 5
-    # Small codes keep whole sums below 2^24 (scale * code <= 4096).
-    xq = t.randint(-1, 2, (ntok, ldxq), generator=g, dtype=t.int8)
-    xq *= (t.rand(ntok, ldxq, generator=g) < 0.1).to(t.int8)
+    xq = _sparse_codes(t, g, ntok, ldxq)
     want = xq[:, :cols].double() @ dense.T
     assert want.abs().max() < 2 ** 24
     L = qk.lib()
     n = L.qk_gemv_batched_i8_workspace_bytes(cols, rows, ntok)
     ws = t.empty(n, dtype=t.uint8, device="cuda")
-    wd, xd, xs = to_dev(t, w), xq.cuda(), t.ones(ntok, ldsc, device="cuda")
+    ten, xd, xs = _tensor(t, qk, qtype, w, cols, rows), xq.cuda(), t.ones(ntok, ldsc, device="cuda")
     y = t.full((ntok, ldy), 7.0, device="cuda")
-    qk.check(L.qk_gemv_batched_i8(qtype, wd.data_ptr(), xd.data_ptr(), ldxq, xs.data_ptr(), ldsc, y.data_ptr(), ldy,
+    qk.check(L.qk_gemv_batched_i8(ten.type, ten.gpu, xd.data_ptr(), ldxq, xs.data_ptr(), ldsc, y.data_ptr(), ldy,
                                   cols, rows, ntok, ws.data_ptr(), n, None), "batched INT8")
     t.cuda.synchronize()
     got = y.cpu().double()
     assert (got[:, :rows] == want).all()
     assert (got[:, rows:] == 7.0).all()
+
+
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q6_K_SPLIT])
+@pytest.mark.parametrize("cols,ntok", [(4096, 300), (8192, 517)])
+def test_several_matrices(qk, torch_gpu, synth, qtype, cols, ntok):
+    """One launch over matrices of one type with ragged rows: each one's row
+    groups, split sums and outputs are its own."""
+    t = torch_gpu
+    base = Q4_K if qtype == Q4_K else Q6_K
+    rows = [1027, 33, 700]
+    assert splits(qk, [(qtype, r) for r in rows], cols, ntok) > 1
+    ws_ = [_integer_blocks(base, synth.quant_matrix(base, cols, r, 6, i), cols, r) for i, r in enumerate(rows)]
+    xq = _sparse_codes(t, t.Generator().manual_seed(4), ntok, cols)
+    tens = [_tensor(t, qk, qtype, w, cols, r) for w, r in zip(ws_, rows)]
+    ys = [t.empty((ntok, r), device="cuda") for r in rows]
+    xd, xs = xq.cuda(), t.ones(ntok, cols // 32, device="cuda")
+    L = qk.lib()
+    n = L.qk_gemv_batched_i8_workspace_bytes(cols, sum(rows), ntok)
+    ws = t.empty(n, dtype=t.uint8, device="cuda")
+    qk.check(L.qk_gemv_multi_batched_i8(qk._matrices(list(zip(tens, ys))), 3, xd.data_ptr(), cols, xs.data_ptr(),
+                                        cols // 32, cols, ntok, ws.data_ptr(), n, None), "multi INT8")
+    t.cuda.synchronize()
+    for w, r, y in zip(ws_, rows, ys):
+        assert (y.cpu().double() == xq.double() @ _dense(t, qk, base, w, cols, r).T).all()
 
 
 def _centred_blocks(synth, cols, rows, seed):
@@ -79,6 +125,7 @@ def test_rounding(qk, torch_gpu, synth, qtype, cols, rows, ntok):
     5.5 = 30, and two where they meet.  The nb blocks' running sum: nb / 2."""
     t = torch_gpu
     nb = cols // 256
+    assert splits(qk, [(qtype, rows)], cols, ntok)
     w = _centred_blocks(synth, cols, rows, 13) if qtype == Q4_K else synth.quant_matrix(Q6_K, cols, rows, 13, 1)
     dense = _dense(t, qk, qtype, w, cols, rows)
     g = t.Generator().manual_seed(17)
@@ -97,14 +144,20 @@ def test_rounding(qk, torch_gpu, synth, qtype, cols, rows, ntok):
     assert rel_l2(y.cpu().numpy(), want.numpy()) < 0.42 * 2 ** -24 * roundings ** 0.5
 
 
-@pytest.mark.parametrize("down", [Q4_K, Q6_K])
-@pytest.mark.parametrize("dim,hidden,ntok", [(2048, 5632, 97), (3072, 8192, 200), (1024, 2816, 517), (5120, 5632, 200)])
-def test_ffn(qk, torch_gpu, synth, down, dim, hidden, ntok):
+@pytest.mark.parametrize("down", [Q4_K, Q6_K, Q6_K_SPLIT])
+@pytest.mark.parametrize("gate", [Q4_K, Q6_K_SPLIT])
+@pytest.mark.parametrize("dim,hidden,ntok", [(2048, 5632, 200), (3072, 8192, 200), (1024, 2816, 517), (5120, 5632, 200)])
+def test_ffn(qk, torch_gpu, synth, gate, down, dim, hidden, ntok):
+    """The pair, its quantized outputs, and down with and without the residual
+    (1024 x 2816: down by the int32 kernels)."""
     t = torch_gpu
-    ws = [synth.quant_matrix(Q4_K, dim, hidden, 9, i) for i in (1, 2)]
-    ws.append(synth.quant_matrix(down, hidden, dim, 9, 3))
-    g, u = (_dense(t, qk, Q4_K, ws[i], dim, hidden) for i in (0, 1))
-    d = _dense(t, qk, down, ws[2], hidden, dim)
+    assert splits(qk, [(gate, hidden)] * 2, dim, ntok, True)
+    assert bool(splits(qk, [(down, dim)], hidden, ntok)) == (dim > 1024)
+    gb, db = (Q4_K if ty == Q4_K else Q6_K for ty in (gate, down))
+    ws = [synth.quant_matrix(gb, dim, hidden, 9, i) for i in (1, 2)]
+    ws.append(synth.quant_matrix(db, hidden, dim, 9, 3))
+    g, u = (_dense(t, qk, gb, ws[i], dim, hidden) for i in (0, 1))
+    d = _dense(t, qk, db, ws[2], hidden, dim)
     gen = t.Generator().manual_seed(11)
     xq = t.randint(-128, 128, (ntok, dim), generator=gen, dtype=t.int8)
     xs = t.rand(ntok, dim // 32, generator=gen) * 2e-4 + 1e-5
@@ -118,12 +171,12 @@ def test_ffn(qk, torch_gpu, synth, down, dim, hidden, ntok):
     want = hq @ d.T
     L = qk.lib()
     n = L.qk_ffn_batched_i8_workspace_bytes(dim, hidden, ntok)
-    dev = [to_dev(t, w) for w in ws]
+    gd, ud, dd = (_tensor(t, qk, ty, w, c, r) for ty, w, c, r in
+                  [(gate, ws[0], dim, hidden), (gate, ws[1], dim, hidden), (down, ws[2], hidden, dim)])
     xd, sd, work = xq.cuda(), xs.cuda(), t.empty(n, dtype=t.uint8, device="cuda")
     for accumulate in (0, 1):
         y = y0.cuda()
-        qk.check(L.qk_ffn_batched_i8(Q4_K, dev[0].data_ptr(), Q4_K, dev[1].data_ptr(), down, dev[2].data_ptr(),
-                                     xd.data_ptr(), dim, sd.data_ptr(), dim // 32, y.data_ptr(), dim, dim, hidden, ntok,
+        qk.check(L.qk_ffn_batched_i8(gate, gd.gpu, gate, ud.gpu, down, dd.gpu, xd.data_ptr(), dim, sd.data_ptr(), dim // 32, y.data_ptr(), dim, dim, hidden, ntok,
                                      accumulate, work.data_ptr(), n, None), "INT8 FFN")
         t.cuda.synchronize()
         ref = want + y0.double() if accumulate else want

@@ -63,18 +63,44 @@ def batch(rng, seqs, heads, kvh, hd):
     return draw(len(tokens), heads * hd), draw(row, kvh * hd), draw(row, kvh * hd), tokens
 
 
-# Sizes at which the tile form is the shorter one (tile_attention_pays).
-@pytest.mark.parametrize("heads,kvh,hd", [(8, 8, 64), (16, 8, 64), (24, 8, 128), (32, 8, 64), (48, 8, 128), (64, 8, 64)])
-@pytest.mark.parametrize("seqs", [[(512, 512)], [(385, 337)], [(640, 300), (33, 17)], [(200, 200), (451, 243)]])
-def test_chunks(qk, torch_gpu, heads, kvh, hd, seqs):
-    rng = np.random.default_rng(heads * 1000 + len(seqs))
-    q, key, value, tokens = batch(rng, seqs, heads, kvh, hd)
-    got = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
+LAYOUTS = [(8, 8, 64), (16, 8, 64), (24, 8, 128), (32, 8, 64), (48, 8, 128), (64, 8, 64)]
+
+
+def check_chunks(qk, t, rng, q, key, value, tokens, heads, kvh, hd):
+    assert tiles(qk, tokens, len(key), heads, kvh, hd)
+    got = run(qk, t, q, key, value, tokens, heads, kvh, hd)
     pick = sorted(set(rng.integers(0, len(tokens), 24).tolist() + [0, 1, 15, 16, len(tokens) - 1]))
     want = reference(q[pick], key, value, [tokens[i] for i in pick], heads, kvh, hd)
     assert rel_l2(got[pick], want) < TOL
     # Every token, against the per-token form (a split size given asks for it).
-    assert rel_l2(got, run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd, split_rows=256)) < TOL
+    assert rel_l2(got, run(qk, t, q, key, value, tokens, heads, kvh, hd, split_rows=256)) < TOL
+
+
+@pytest.mark.parametrize("heads,kvh,hd", LAYOUTS)
+@pytest.mark.parametrize("seqs", [[(512, 512)], [(540, 507)]])
+def test_one_chunk(qk, torch_gpu, heads, kvh, hd, seqs):
+    rng = np.random.default_rng(heads * 1000)
+    check_chunks(qk, torch_gpu, rng, *batch(rng, seqs, heads, kvh, hd), heads, kvh, hd)
+
+
+@pytest.mark.parametrize("heads,kvh,hd", LAYOUTS[:4])
+@pytest.mark.parametrize("seqs", [[(640, 300), (333, 205)], [(640, 480), (33, 17)], [(200, 150), (300, 181), (260, 170)]])
+def test_chunks_of_several_sequences(qk, torch_gpu, heads, kvh, hd, seqs):
+    """Tiles of two sequences, of a sequence's end and a short one, and of one
+    token of one and fifteen of another."""
+    rng = np.random.default_rng(heads * 1000 + len(seqs))
+    check_chunks(qk, torch_gpu, rng, *batch(rng, seqs, heads, kvh, hd), heads, kvh, hd)
+
+
+@pytest.mark.parametrize("heads,kvh,hd", LAYOUTS)
+def test_tile_of_two_runs(qk, torch_gpu, heads, kvh, hd):
+    """Two runs over the rows of one sequence that meet inside a tile, in every
+    head layout: tokens 0..299 and, in the same call, 251..462."""
+    rng = np.random.default_rng(heads * 1000 + 5)
+    q, key, value, _ = batch(rng, [(463, 512 - 49)], heads, kvh, hd)
+    q = rng.standard_normal((512, heads * hd)).astype(np.float32)
+    tokens = [(i, 0) for i in range(300)] + [(i, 0) for i in range(251, 463)]
+    check_chunks(qk, torch_gpu, rng, q, key, value, tokens, heads, kvh, hd)
 
 
 def test_decodes_beside_a_chunk(qk, torch_gpu):
@@ -82,10 +108,63 @@ def test_decodes_beside_a_chunk(qk, torch_gpu):
     heads, kvh, hd = 32, 8, 64
     rng = np.random.default_rng(7)
     q, key, value, tokens = batch(rng, [(500, 460)] + [(40 + i, 1) for i in range(20)], heads, kvh, hd)
+    assert tiles(qk, tokens, len(key), heads, kvh, hd)
     got = run(qk, torch_gpu, q, key, value, tokens, heads, kvh, hd)
     pick = [0, 200, 459] + list(range(460, 480))
     want = reference(q[pick], key, value, [tokens[i] for i in pick], heads, kvh, hd)
     assert rel_l2(got[pick], want) < TOL
+
+
+def step_mode(qk, tokens, cfg):
+    """The decode driver's choice: 0 none, 1 tiles and the other tokens one by
+    one, 2 every token in a tile."""
+    desc = (qk.qk_batch_token * len(tokens))(*(qk.qk_batch_token(p, 0, r) for p, r in tokens))
+    return qk.lib().qk_rule_tile_attention_step(desc, len(tokens), cfg["heads"], cfg["kv_heads"],
+                                                cfg["dim"] // cfg["heads"])
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("heads,kv_heads,hd,chunk,decodes", [
+    (16, 8, 64, (0, 301), 0), (16, 8, 64, (37, 331), 20), (8, 4, 128, (200, 509), 0), (8, 4, 128, (200, 505), 19),
+    (8, 8, 64, (0, 347), 19)])
+def test_driver_chunk(qk, torch_gpu, workloads, synth, int8, heads, kv_heads, hd, chunk, decodes):
+    """A chunk, alone and beside decodes (of long and short contexts, so that
+    their rows are split and merged), in the batched driver's own cache layout
+    with the o projection's records (FP32) or codes (INT8) from the attention:
+    every token's logits against the same step with its tokens in reverse order.
+    Those tokens form no runs, so they take the per-token form; the products do
+    not depend on the order."""
+    pre, n = chunk
+    cfg = dict(dim=heads * hd, layers=2, heads=heads, kv_heads=kv_heads, hidden=512, vocab=300, context=1024, eps=1e-5,
+               rope_theta=10000.0)
+    W, ctx, kv = workloads.llama_weights(cfg, 31), cfg["context"], kv_heads * hd
+    S = 1 + decodes
+    entries = [(0, pre + i) for i in range(n)] + [(1 + i, 40 + 47 * i) for i in range(decodes)]   # (sequence, position)
+    tokens = [(p, s * ctx) for s, p in entries]
+    assert step_mode(qk, tokens, cfg) == (1 if decodes else 2)
+    assert step_mode(qk, tokens[::-1], cfg) == 0
+    caches = [synth.normal_f32(cfg["layers"] * S * ctx * kv, 32, i).reshape(cfg["layers"], S * ctx, kv) for i in (0, 1)]
+    ids = [int(v) for v in synth.uniform_i32(len(entries), 32, 5, 0, cfg["vocab"] - 1)]
+
+    def step(order):
+        br = qk.BatchRunner(cfg, W, max_tokens=len(entries), cache_rows=S * ctx)
+        br.set_int8(int8, int8)
+        br.load_kv(*caches)
+        pick = [entries[i] for i in order]
+        br.forward([ids[i] for i in order], [p for _, p in pick], [s * ctx for s, _ in pick], seq=[s for s, _ in pick],
+                   logit_rows=list(range(len(order))))
+        lg = br.logits(len(order))
+        br.close()
+        out = np.empty_like(lg)
+        out[order] = lg
+        return out
+
+    got, want = step(list(range(len(entries)))), step(list(range(len(entries)))[::-1])
+    errs = np.array([rel_l2(a, b) for a, b in zip(got, want)])
+    # FP32: the forms' roundings (2e-7 of an output each) through two layers,
+    # magnified where a random score is large.  INT8: a code within them of a
+    # midpoint moves by one of 127, in few tokens.
+    assert np.isfinite(got).all() and np.median(errs) < 1e-6 and errs.max() < (5e-2 if int8 else 2e-3)
 
 
 def test_later_rows_not_finite(qk, torch_gpu):
