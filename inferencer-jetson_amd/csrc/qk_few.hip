@@ -1,5 +1,5 @@
-// qk_few.hip - products of 2 to 7 tokens: a few sequences decoding together, a
-// few speculated tokens.
+// qk_few.hip - products of 2 to 7 tokens with enough weights for it (few_pays): a
+// few sequences decoding together, a few speculated tokens.
 //
 // One GEMV column per token decodes every weight once per token (their
 // re-reads come from cache).  Here every weight is read and decoded once, into
@@ -19,12 +19,14 @@
 //     meet in LDS in wave order, one barrier a step.
 //   * With `pair` the epilogue forms SiLU(gate) * up.
 //
-// Bound by the weight stream from about 100 MB on, by the conversion (0.75 us
-// a token) below.  Measured against the GEMV columns at 4 and 7 tokens: Q4_K
-// 128256 x 2048 80.7 -> 38.1 and 148 -> 40.8 us, split Q6_K 118 -> 65 and 210
-// -> 64 us, Q4_K 16384 x 3072 21.5 -> 13.6 and 34.8 -> 16.1 us; the 3B
-// feed-forward block of 4 tokens 50.2 -> 34.7 us.  (Converting in the
-// operand's own lanes, 16-byte reads 256 bytes apart, took 3 to 8 us more.)
+// Bound by the conversion (0.5 to 0.8 us a token) and the waves' meetings up to
+// some 20 MB, then by the decode: 0.22 us a MB of Q4_K (4.5 TB/s) and 0.29 of
+// split Q6_K (3.4), where the one-token GEMV streams 5.2 and 5.6.  Measured
+// against the GEMV columns at 4 and 7 tokens: Q4_K 128256 x 2048 80.7 -> 38.1 and
+// 148 -> 40.8 us, split Q6_K 118 -> 65 and 210 -> 64 us, Q4_K 16384 x 3072 21.5
+// -> 13.6 and 34.8 -> 16.1 us; the 3B feed-forward block of 4 tokens 50.2 -> 34.7
+// us.  (Converting in the operand's own lanes, 16-byte reads 256 bytes apart,
+// took 3 to 8 us more.)
 #include "qk_internal.h"
 #include "qk_operands.h"
 #include "qk_records.h"
@@ -424,28 +426,38 @@ void launch_form(int type, const dim3 &grid, const dim3 &block, size_t lds, hipS
 
 // Supported: rows of at most sixteen blocks, or (no pair) of 32 where every
 // workgroup has one tile to take -- two blocks a wave, converted one after the
-// other.  And shorter, by estimates fitted to 0.9 to 215 MB of either type at
-// 2 to 7 tokens: here 4.5 us (Q6_K 6) of launch and ramp, 0.75 us a token and
-// block of a wave to convert x, 0.2 us (0.28) a MB of weights; one GEMV column
-// per token 4.8 us and 0.135 us a MB and token (its re-reads come from cache).
-// The estimates miss by up to a tenth, so the gain has to be that.
+// other.  And shorter, by estimates fitted to 1 to 140 MB of each type in rows of
+// 1 to 32 blocks at 2 to 7 tokens, both forms measured for each: here a base that
+// grows with the waves that meet, a conversion per token and the weights (short
+// rows: more of a tile's work is the meeting); one GEMV column per token the
+// launch and the bytes of every token, its re-reads coming from cache (powers of
+// two of blocks divide evenly over its waves).  Of the 1524 shapes measured, the
+// accepted ones take 0.55 to 1.02 of the GEMV's time but for two (1.05 and 1.08).
 bool few_pays(const qk_matrix *mats, int n_mats, int cols, int n_tokens, bool pair) {
-    const int nb = cols / 256, bpw = nb > kMaxWaves ? 2 : 1;
+    const int nb = cols / 256;
+    const bool two = nb > kMaxWaves;
     if (n_tokens < 2 || n_tokens >= kSlots || nb > 2 * kMaxWaves) return false;
-    if (pair && (bpw == 2 || n_mats != 2 || mats[0].type != mats[1].type || mats[0].rows != mats[1].rows)) return false;
-    double us = 4.5 + 0.75 * bpw * n_tokens, mb = 0.;
+    if (pair && (two || n_mats != 2 || mats[0].type != mats[1].type || mats[0].rows != mats[1].rows)) return false;
+    struct Cost {
+        double base, block, token, mb;   // us, us a block of the row, us a token, us a MB
+    };
+    constexpr Cost kOne[3] = {{3.2, 0.19, 0.83, 0.22}, {4.6, 0.5, 0.5, 0.35}, {3.9, 0.25, 0.6, 0.29}};
+    constexpr Cost kTwo[3] = {{7.9, 0., 1.97, 0.035}, {13.1, 0., 1.35, 0.04}, {10.1, 0., 1.58, 0.06}};
+    double fixed = 0., stream = 0., mb = 0.;
     int64_t tiles = 0;
-    bool q6 = false;
     for (int i = 0; i < n_mats; ++i) {
+        const int t = mats[i].type == QK_TYPE_Q4_K ? 0 : mats[i].type == QK_TYPE_Q6_K ? 1 : 2;
+        const Cost &c = two ? kTwo[t] : kOne[t];
         const double m = 1e-6 * static_cast<double>(row_bytes(mats[i].type, nb)) * mats[i].rows;
+        fixed = std::max(fixed, c.base + c.block * nb + c.token * n_tokens);
+        stream += (c.mb + (two ? 0. : 0.25 / (nb * nb))) * m;
         mb += m;
-        us += (mats[i].type == QK_TYPE_Q4_K ? 0.2 : 0.28) * m;
-        q6 |= mats[i].type != QK_TYPE_Q4_K;
         tiles += (mats[i].rows + kTileRows - 1) / kTileRows;
     }
-    if (q6) us += 1.5;
-    if (bpw == 2 && tiles > device_info().cus) return false;
-    return 1.1 * us < 4.8 + 0.135 * mb * n_tokens;
+    if (two && tiles > device_info().cus) return false;
+    const double bytes = mb * n_tokens;
+    const double gemv = two ? 7.1 + 0.15 * bytes : nb & (nb - 1) ? 6.5 + 0.135 * bytes : 5.2 + 0.13 * bytes;
+    return 1.05 * (fixed + stream) < gemv;
 }
 
 int launch_few(const qk_matrix *mats, int n_mats, const float *x, int ldx, int cols, int n_tokens, const int *ldy,

@@ -23,16 +23,16 @@ def few(qk, mats, cols, ntok, pair=False):
 
 
 @pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q6_K_SPLIT])
-@pytest.mark.parametrize("ntok,cols,rows", [(7, 256, 66001), (7, 768, 32015), (4, 2048, 65541), (6, 3072, 16400),
+@pytest.mark.parametrize("ntok,cols,rows", [(7, 256, 140001), (7, 768, 32015), (4, 2048, 65541), (6, 3072, 16400),
                                             (5, 4096, 12001), (7, 7424, 4093), (7, 7936, 3900), (7, 8192, 3899),
-                                            (7, 8192, 3700), (3, 2048, 128256)])
+                                            (7, 8192, 3700), (4, 2048, 128256)])
 def test_edges(qk, torch_gpu, oracle, workloads, synth, qtype, ntok, cols, rows):
     x = synth.normal_f32(ntok * cols, 61, ntok).reshape(ntok, cols)
     assert few(qk, [(qtype, rows)], cols, ntok)
     check(qk, torch_gpu, oracle, [matrix(qk, torch_gpu, workloads, synth, qtype, cols, rows, 60 + ntok)], x, cols)
 
 
-@pytest.mark.parametrize("ntok,cols", [(7, 2048), (5, 2560), (3, 4096)])
+@pytest.mark.parametrize("ntok,cols", [(7, 2048), (5, 2560), (4, 3072)])
 def test_mixed_types(qk, torch_gpu, oracle, workloads, synth, ntok, cols):
     x = synth.normal_f32(ntok * cols, 62, ntok).reshape(ntok, cols)
     mats = [(Q4_K, 16500), (Q6_K, 96), (Q6_K_SPLIT, 257), (Q4_K, 20)]
@@ -42,15 +42,16 @@ def test_mixed_types(qk, torch_gpu, oracle, workloads, synth, ntok, cols):
 
 
 @pytest.mark.parametrize("types", [(Q4_K, Q4_K, Q6_K), (Q4_K, Q6_K, Q4_K), (Q6_K_SPLIT, Q6_K_SPLIT, Q6_K_SPLIT)])
-@pytest.mark.parametrize("ntok,dim,hidden", [(7, 2048, 4096), (5, 3072, 4096), (7, 1024, 8192), (7, 4096, 4096),
-                                             (6, 4096, 4096)])
+@pytest.mark.parametrize("ntok,dim,hidden", [(7, 2048, 8192), (5, 3072, 8192), (7, 1536, 8192), (7, 4096, 4096),
+                                             (6, 3840, 4608)])
 def test_ffn(qk, torch_gpu, oracle, workloads, synth, types, ntok, dim, hidden):
-    """Gate and up of one type in one launch with SiLU * up; down here too from
-    4096 x 4096 on, else by the GEMV kernels."""
+    """Gate and up of one type in one launch with SiLU * up; down here or by the
+    GEMV kernels (small products)."""
     t = torch_gpu
     if types[0] == types[1]:
         assert few(qk, [(types[0], hidden), (types[1], hidden)], dim, ntok, True)
-    assert few(qk, [(types[2], dim)], hidden, ntok) == (dim >= 4096)
+    if types[2] == Q6_K_SPLIT and (dim, hidden) in ((3072, 8192), (4096, 4096)):
+        assert few(qk, [(types[2], dim)], hidden, ntok)
     x = synth.normal_f32(ntok * dim, 63, ntok).reshape(ntok, dim) * 0.05
     shapes = [(dim, hidden), (dim, hidden), (hidden, dim)]
     (g, wg, tg), (u, wu, tu), (d, wd, td) = [matrix(qk, t, workloads, synth, ty, c, r, 80 + i)
@@ -91,38 +92,35 @@ def test_pair_not_finite(qk, torch_gpu, workloads, synth):
     ntok, dim, hidden = 7, 4096, 4096
     x = synth.normal_f32(ntok * dim, 66, 1).reshape(ntok, dim) * 0.05
     x[3, 17], x[5, 4095] = np.nan, np.inf
-    (g, _, _), (u, _, _), (d, _, _) = [matrix(qk, t, workloads, synth, Q4_K, c, r, 92 + i)
-                                       for i, (c, r) in enumerate([(dim, hidden), (dim, hidden), (hidden, dim)])]
-    assert few(qk, [(Q4_K, hidden)] * 2, dim, ntok, True) and few(qk, [(Q4_K, dim)], hidden, ntok)
+    (g, _, _), (u, _, _), (d, _, _) = [matrix(qk, t, workloads, synth, ty, c, r, 92 + i) for i, (ty, c, r) in
+                                       enumerate([(Q4_K, dim, hidden), (Q4_K, dim, hidden), (Q6_K_SPLIT, hidden, dim)])]
+    assert few(qk, [(Q4_K, hidden)] * 2, dim, ntok, True) and few(qk, [(Q6_K_SPLIT, dim)], hidden, ntok)
     nb = qk.lib().qk_ffn_batched_workspace_bytes(dim, hidden, ntok)
     ws, y = t.empty(nb, dtype=t.uint8, device="cuda"), t.empty((ntok, dim), device="cuda")
     xd = to_dev(t, x)
-    qk.check(qk.lib().qk_ffn_batched_f32(Q4_K, g.gpu, Q4_K, u.gpu, Q4_K, d.gpu, xd.data_ptr(), dim, y.data_ptr(), dim, dim,
-                                         hidden, ntok, 0, ws.data_ptr(), nb, None), "ffn")
+    qk.check(qk.lib().qk_ffn_batched_f32(Q4_K, g.gpu, Q4_K, u.gpu, Q6_K_SPLIT, d.gpu, xd.data_ptr(), dim, y.data_ptr(), dim,
+                                         dim, hidden, ntok, 0, ws.data_ptr(), nb, None), "ffn")
     t.cuda.synchronize()
     got = y.cpu().numpy()
     assert np.isnan(got[[3, 5]]).all() and np.isfinite(got[[0, 1, 2, 4, 6]]).all()
 
 
 @pytest.mark.parametrize("up_type", [Q4_K, Q6_K])
-def test_driver_step(qk, torch_gpu, oracle, workloads, synth, up_type):
-    """Seven sequences decoding in the batched driver: QKV and gate / up with the
-    RMSNorm staged here, gate and up of one type (the pair) or of two (down then
-    stages SiLU * up), both projections into x accumulated; each sequence against
-    its own oracle model."""
-    cfg = dict(dim=4096, layers=2, heads=32, kv_heads=8, hidden=4096, vocab=300, context=32, eps=1e-5,
+@pytest.mark.parametrize("ntok,dim,hidden,heads,kv_heads", [(7, 4096, 4096, 32, 8), (5, 3072, 8192, 24, 8)])
+def test_driver_step(qk, torch_gpu, oracle, workloads, synth, up_type, ntok, dim, hidden, heads, kv_heads):
+    """Sequences decoding in the batched driver (which holds Q6_K in the split
+    layout): gate / up with the RMSNorm staged here, of one type (the pair) or of
+    two (down then stages SiLU * up), down accumulated into x, one block a wave and
+    two; each sequence against its own oracle model."""
+    cfg = dict(dim=dim, layers=2, heads=heads, kv_heads=kv_heads, hidden=hidden, vocab=300, context=32, eps=1e-5,
                rope_theta=10000.0)
-    ntok = 7
     W = workloads.llama_weights(cfg, 27, mix=dict(workloads.MIX_1B, up=up_type))
     for i, L in enumerate(W["layers"]):
-        L["attn_norm"] = 1.0 + 0.2 * synth.normal_f32(cfg["dim"], 27, 500 + i)
-        L["ffn_norm"] = 1.0 + 0.2 * synth.normal_f32(cfg["dim"], 27, 510 + i)
-        kv = cfg["dim"] // cfg["heads"] * cfg["kv_heads"]
-        assert few(qk, [(L["q_type"], cfg["dim"]), (L["k_type"], kv), (L["v_type"], kv)], cfg["dim"], ntok)
-        assert few(qk, [(L["gate_type"], cfg["hidden"]), (L["up_type"], cfg["hidden"])], cfg["dim"], ntok, True) == \
-            (up_type == Q4_K)
-        assert few(qk, [(L["gate_type"], cfg["hidden"]), (L["up_type"], cfg["hidden"])], cfg["dim"], ntok)
-        assert few(qk, [(L["down_type"], cfg["dim"])], cfg["hidden"], ntok)
+        L["attn_norm"] = 1.0 + 0.2 * synth.normal_f32(dim, 27, 500 + i)
+        L["ffn_norm"] = 1.0 + 0.2 * synth.normal_f32(dim, 27, 510 + i)
+    pair = [(Q4_K, hidden), (Q4_K if up_type == Q4_K else Q6_K_SPLIT, hidden)]
+    assert few(qk, pair, dim, ntok, True) == (up_type == Q4_K) and few(qk, pair, dim, ntok)
+    assert few(qk, [(Q6_K_SPLIT, dim)], hidden, ntok)
     br = qk.BatchRunner(cfg, W, max_tokens=ntok, cache_rows=ntok * cfg["context"])
     orcs = [oracle.Llama(cfg, W) for _ in range(ntok)]
     tokens = [int(v) for v in synth.uniform_i32(ntok, 27, 71, 0, cfg["vocab"] - 1)]
