@@ -13,6 +13,15 @@
 
 namespace qk {
 
+// The hardware deals consecutive workgroups to the eight XCDs in turn: workgroup w
+// of a grid of ceil(total / 8) * 8 takes item (w % 8) * ceil(total / 8) + w / 8 of a
+// list, so that neighbours in the list run on one XCD and share what they read
+// through its L2.  -1: none.
+__device__ __forceinline__ int xcd_item(int workgroup, int total) {
+    const int per = (total + 7) / 8, place = workgroup >> 3, item = (workgroup & 7) * per + place;
+    return item < total && place < per ? item : -1;
+}
+
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 

@@ -361,17 +361,13 @@ __device__ __forceinline__ void tile_gemm_body(const BatchParams &p, const Batch
     }
 }
 
-// Workgroup order: the hardware deals consecutive workgroups to the eight XCDs
-// in turn, so workgroup w takes item (w % 8) * ceil(n / 8) + w / 8 of a list in
-// which the token groups of one row group are neighbours: they run on one XCD
-// and share its weight bytes through that XCD's L2.
+// In xcd_item's list the token groups of one row group are neighbours: they share
+// its weight bytes.
 template <int TYPE>
 __global__ __launch_bounds__(256, 2) void tile_gemm(BatchParams p, int groups, int tgroups) {
     extern __shared__ __align__(16) unsigned char lds[];
-    const int total = groups * tgroups * p.splits;
-    const int per = (total + 7) / 8, place = static_cast<int>(blockIdx.x) >> 3;
-    const int item = (static_cast<int>(blockIdx.x) & 7) * per + place;
-    if (item >= total || place >= per) return;
+    const int item = xcd_item(static_cast<int>(blockIdx.x), groups * tgroups * p.splits);
+    if (item < 0) return;
     const int tgroup = item % tgroups, rest = item / tgroups;
     const int split = rest % p.splits, group = rest / p.splits;
     int m = 0;

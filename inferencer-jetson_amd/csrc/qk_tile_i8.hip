@@ -457,16 +457,13 @@ __device__ __forceinline__ void tile_body(const TiParams &p, const TiMatrix &M, 
     }
 }
 
-// Consecutive workgroups go to the eight XCDs in turn: item (w % 8) *
-// ceil(n / 8) + w / 8 of a list in which the token groups of one row group are
-// neighbours, so they share its weight bytes in one XCD's L2.
+// In xcd_item's list the token groups of one row group are neighbours: they share
+// its weight bytes.
 template <int TYPE, bool PAIR, bool LONG>
 __global__ __launch_bounds__(256, LONG ? 2 : 3) void tile_i8(TiParams p) {
     extern __shared__ __align__(16) unsigned char lds[];
-    const int total = p.groups * p.tgroups * p.splits;
-    const int per = (total + 7) / 8, place = static_cast<int>(blockIdx.x) >> 3;
-    const int item = (static_cast<int>(blockIdx.x) & 7) * per + place;
-    if (item >= total || place >= per) return;
+    const int item = xcd_item(static_cast<int>(blockIdx.x), p.groups * p.tgroups * p.splits);
+    if (item < 0) return;
     const int tgroup = item % p.tgroups, rest = item / p.tgroups;
     const int split = rest % p.splits, group = rest / p.splits;
     int m = 0;
