@@ -154,7 +154,7 @@ int qk_gemv_multi_batched_f32(const qk_matrix *mats, int n_mats, const float *x,
    up straight into the down projection's input records, so neither gate,
    up nor their product is stored as fp32; below 8 tokens, the fused GEMV pair
    of qk_gemv_multi_f32 and a down GEMV staging SiLU * up, or, where that is
-   estimated to take less time (3 to 7 tokens of large like gate and up), one
+   estimated to take less time (2 to 7 tokens, gate and up of one type), one
    read of their weights on the matrix cores that writes SiLU * up, and a down
    launch over it.  workspace:
    qk_ffn_batched_workspace_bytes(dim, hidden, n_tokens) bytes (256-byte
